@@ -117,6 +117,16 @@ class TrajLaunch(C.Structure):
     ]
 
 
+class GroupInfo(C.Structure):
+    _fields_ = [
+        ("targets", C.c_uint64),
+        ("max_qubits", C.c_uint32),
+        ("low_qubits", C.c_uint32),
+        ("max_gates", C.c_uint32),
+        ("reserved", C.c_uint32),
+    ]
+
+
 _vp, _sz, _u8, _u32, _u64, _i = C.c_void_p, C.c_size_t, C.c_uint8, C.c_uint32, C.c_uint64, C.c_int
 _err = C.c_char_p
 _SIGS = {
@@ -165,6 +175,8 @@ _SIGS = {
     "cast_hip_gate_apply": (_i, [_vp, _vp, _u64, _u32, _err, _sz]),
     "cast_hip_gate_apply_batch": (
         _i, [C.POINTER(_vp), C.POINTER(_u64), C.POINTER(_u32), _sz, _vp, _err, _sz]),
+    "cast_hip_gate_group_info": (_i, [_vp, _u32, C.POINTER(GroupInfo), _err, _sz]),
+    "cast_hip_gate_apply_group": (_i, [C.POINTER(_vp), _sz, _vp, _u64, _u32, _err, _sz]),
     "cast_hip_expect_zz": (
         _i, [_u64, _u32, _u8, C.POINTER(_u32), _sz, C.POINTER(C.c_double), _vp, _err, _sz]),
     "cast_hip_traj_run": (_i, [C.POINTER(TrajLaunch), _vp, _err, _sz]),
@@ -301,6 +313,17 @@ def gate_apply_batch(plans, svs, n_qubits, stream: int | None = None) -> None:
     n = len(plans)
     _call("cast_hip_gate_apply_batch", (_vp * n)(*plans), (_u64 * n)(*svs),
           (_u32 * n)(*n_qubits), n, stream)
+
+
+def gate_group_info(plan: int, n_qubits: int) -> GroupInfo:
+    info = GroupInfo()
+    _call("cast_hip_gate_group_info", plan, n_qubits, C.byref(info))
+    return info
+
+
+def gate_apply_group(plans, dptr: int, n_qubits: int, stream: int | None = None) -> None:
+    n = len(plans)
+    _call("cast_hip_gate_apply_group", (_vp * n)(*plans), n, stream, dptr, n_qubits)
 
 
 def expect_zz(dptr: int, n_qubits: int, precision: int, pairs, stream: int | None = None):

@@ -186,36 +186,47 @@ GatePlan *build_plan(const cast_hip_kernel_gen_spec_t *spec, const cast_complex6
 
   ensure_device();
   check(hipGetDevice(&plan->device), "hipGetDevice");
-  const size_t bytes = 2 * K * K * (fp32 ? 4 : 8);
-  plan->d_mat = cache_alloc(bytes);
-  plan->mat_bytes = bytes;
-  if (fp32) {
-    std::vector<float> f(2 * K * K);
-    for (size_t i = 0; i < f.size(); ++i)
-      f[i] = float(m[i]);
-    check(hipMemcpy(plan->d_mat, f.data(), bytes, hipMemcpyHostToDevice), "hipMemcpy(matrix)");
-  } else {
-    check(hipMemcpy(plan->d_mat, m.data(), bytes, hipMemcpyHostToDevice), "hipMemcpy(matrix)");
-  }
-  if (variant != CAST_HIP_VARIANT_MONOMIAL && n_qubits >= 4) {
-    // Real matrices of the three-product form: Re M, Im M, Re M + Im M.
-    const size_t KK = K * K;
+  // The complex matrix, for dense k >= 4 the real matrices Re M, Im M, Re M +
+  // Im M of the three-product form, and the operands for groups of gates:
+  // one allocation, one copy.
+  const size_t KK = K * K, sb = fp32 ? 4 : 8;
+  const bool real3 = variant != CAST_HIP_VARIANT_MONOMIAL && n_qubits >= 4;
+  const size_t mat3_at = 2 * KK * sb, op_at = mat3_at + (real3 ? 3 * KK * sb : 0);
+  const bool op = real3 && n_qubits <= 5;
+  plan->block_bytes =
+      op_at + (op ? group_operand_bytes(uint32_t(n_qubits), plan->precision) : 0);
+  std::vector<unsigned char> host(plan->block_bytes);
+  auto put = [&](size_t at, const double *v, size_t n) {
+    if (fp32) {
+      float *f = reinterpret_cast<float *>(host.data() + at);
+      for (size_t i = 0; i < n; ++i)
+        f[i] = float(v[i]);
+    } else {
+      std::memcpy(host.data() + at, v, n * sizeof(double));
+    }
+  };
+  put(0, m.data(), 2 * KK);
+  if (real3) {
     std::vector<double> m3(3 * KK);
     for (size_t i = 0; i < KK; ++i) {
       m3[i] = m[2 * i];
       m3[KK + i] = m[2 * i + 1];
       m3[2 * KK + i] = m[2 * i] + m[2 * i + 1];
     }
-    const size_t b3 = 3 * KK * (fp32 ? 4 : 8);
-    plan->d_mat3 = cache_alloc(b3);
-    plan->mat3_bytes = b3;
-    if (fp32) {
-      std::vector<float> f(m3.begin(), m3.end());
-      check(hipMemcpy(plan->d_mat3, f.data(), b3, hipMemcpyHostToDevice), "hipMemcpy(m3)");
-    } else {
-      check(hipMemcpy(plan->d_mat3, m3.data(), b3, hipMemcpyHostToDevice), "hipMemcpy(m3)");
-    }
+    put(mat3_at, m3.data(), m3.size());
   }
+  if (op)
+    group_operands(m.data(), uint32_t(n_qubits), plan->precision, host.data() + op_at);
+  plan->d_block = cache_alloc(plan->block_bytes);
+  unsigned char *d = static_cast<unsigned char *>(plan->d_block);
+  plan->d_mat = d;
+  plan->d_mat3 = real3 ? d + mat3_at : nullptr;
+  plan->d_op = op ? d + op_at : nullptr;
+  const hipError_t copied =
+      hipMemcpy(plan->d_block, host.data(), plan->block_bytes, hipMemcpyHostToDevice);
+  if (copied != hipSuccess)
+    cache_release(plan->d_block, plan->block_bytes);
+  check(copied, "hipMemcpy(matrix)");
   return plan.release();
 }
 
@@ -268,10 +279,8 @@ namespace {
 void free_plan(GatePlan *p) {
   if (!p)
     return;
-  if (p->d_mat)
-    cache_release(p->d_mat, p->mat_bytes);
-  if (p->d_mat3)
-    cache_release(p->d_mat3, p->mat3_bytes);
+  if (p->d_block)
+    cache_release(p->d_block, p->block_bytes);
   delete[] p->h_mat;
   delete p;
 }
@@ -671,6 +680,39 @@ int cast_hip_gate_apply_batch(const void *const *plans, const uint64_t *svs,
     }
     launch_gate_batch(items.data(), n_items, p0->precision, p0->k,
                       static_cast<hipStream_t>(stream));
+  });
+}
+
+int cast_hip_gate_group_info(const void *plan, uint32_t sv_n_qubits, cast_hip_group_info_t *out,
+                             char *err, size_t len) {
+  return guard(err, len, [&] {
+    if (!plan || !out)
+      throw Error("null argument");
+    std::memset(out, 0, sizeof(*out));
+    const GroupLimits l = group_limits(*static_cast<const GatePlan *>(plan), sv_n_qubits);
+    out->targets = l.targets;
+    out->max_qubits = l.max_qubits;
+    out->low_qubits = l.low_qubits;
+    out->max_gates = l.max_gates;
+  });
+}
+
+int cast_hip_gate_apply_group(const void *const *plans, size_t n_plans, void *stream,
+                              uint64_t sv_dptr, uint32_t sv_n_qubits, char *err, size_t len) {
+  return guard(err, len, [&] {
+    if (n_plans == 0)
+      return;
+    if (!plans)
+      throw Error("null plan list");
+    for (size_t i = 0; i < n_plans; ++i)
+      if (!plans[i])
+        throw Error("null plan at index " + std::to_string(i));
+    if (!sv_dptr)
+      throw Error("null statevector pointer");
+    check_aligned(sv_dptr);
+    launch_group(reinterpret_cast<const GatePlan *const *>(plans), n_plans,
+                 static_cast<hipStream_t>(stream), reinterpret_cast<void *>(sv_dptr),
+                 sv_n_qubits);
   });
 }
 

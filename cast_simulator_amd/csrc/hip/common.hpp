@@ -87,9 +87,12 @@ struct GatePlan {
   uint32_t flags = 0;    // CAST_HIP_FLAG_*
   uint32_t q[8] = {};
   int device = 0;
+  void *d_block = nullptr;     // the device matrices below, in one allocation
+  size_t block_bytes = 0;
   void *d_mat = nullptr;       // K*K complex, interleaved, device precision
-  void *d_mat3 = nullptr;      // [Re M | Im M | Re M + Im M], 3*K*K real (k = 4, 5)
-  size_t mat_bytes = 0, mat3_bytes = 0;
+  void *d_mat3 = nullptr;      // [Re M | Im M | Re M + Im M], 3*K*K real (dense k >= 4)
+  void *d_op = nullptr;        // matrix-core operands in the order of the lanes (dense k = 4,
+                               // 5; group_operands)
   double *h_mat = nullptr;     // snapped matrix in f64 (host copy, 2*K*K)
   uint64_t scalar_nnz = 0;
   // Monomial form: rows that differ from identity, each with one source col.
@@ -114,6 +117,23 @@ struct BatchItem {
 };
 void launch_gate_batch(const BatchItem *items, size_t n, uint8_t precision, uint32_t k,
                        hipStream_t stream);
+
+// Gate groups (group_kernels.hip): whether a plan may run in a group on an
+// n-qubit statevector (targets = 0: it may not), and what a group may hold.
+struct GroupLimits {
+  uint64_t targets;    // mask of the plan's target qubits
+  uint32_t max_qubits; // qubits of a tile, the low_qubits lowest always among them
+  uint32_t low_qubits;
+  uint32_t max_gates;
+};
+GroupLimits group_limits(const GatePlan &plan, uint32_t n_qubits);
+// Matrix-core operands of a dense k = 4 or 5 gate for a group (bytes, and the
+// buffer itself from the snapped matrix m of 2 K K doubles).
+size_t group_operand_bytes(uint32_t k, uint8_t precision);
+void group_operands(const double *m, uint32_t k, uint8_t precision, void *out);
+// Enqueues the gates, in order, as one pass over the statevector.
+void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stream, void *sv,
+                  uint32_t n_qubits);
 
 // Statevector utility kernels implemented in sv_kernels.hip.
 void launch_sv_zero(void *sv, size_t n_elements, uint8_t precision, hipStream_t stream);

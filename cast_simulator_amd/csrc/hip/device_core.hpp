@@ -405,7 +405,7 @@ template <int KL> struct SplitOperands {
   // of lane l at index (((m * 3 + s) * RB + rb) * KS + ks) * 64 + l: every
   // read is 64 consecutive 16-byte vectors
   static constexpr int kFragments = 2 * 3 * RB * KS * 64;
-  __device__ static constexpr int at(int m, int s, int rb, int ks) {
+  __host__ __device__ static constexpr int at(int m, int s, int rb, int ks) {
     return (((m * 3 + s) * RB + rb) * KS + ks) * 64;
   }
 };

@@ -1,0 +1,785 @@
+// Gate groups: several consecutive gates in one pass over the statevector.
+//
+// A single-gate kernel reads and writes every amplitude from HBM for each
+// gate, so below the matrix-core ridge a circuit costs one HBM round trip per
+// gate.  A group is a list of gates whose targets together lie in a set S of
+// m qubits (m <= 12 at f64, 13 at f32).  A workgroup owns one tile of 2^m
+// amplitudes (the S bits vary, the others are fixed by the tile index),
+// loads it into LDS (64 KiB), applies every gate of the list there with a
+// barrier between gates, and writes it back: one HBM round trip per group.
+//
+// LDS layout: 16-byte units (one f64 amplitude, two f32 ones) at unit index
+// u ^ (u >> 4 & 15) ^ (u >> 8 & 15).  The map is linear over GF(2), so the
+// address of an amplitude is the XOR of one constant per index bit; the host
+// puts these constants (byte offsets) into the gate's descriptor in the order
+// in which the kernel consumes them.  Consecutive lanes get index bits that
+// fall on different banks.
+//
+// A thread holds 2^R amplitudes at a time (f64 R = 3 or 4, f32 one more):
+//   k <= 3        one combo per lane and register group on the VALU, matrix
+//                 rows by scalar loads, each row used for 2^(R-k) combos;
+//   k = 4, f64 5  three real products on the matrix cores, 16 combos per
+//                 MFMA tile, operands laid out by lane when the plan is built;
+//   f32 k = 5     bf16 split products as in the single-gate kernel;
+//   monomial      diagonal gates (any k) multiply in place, permutations
+//                 (k <= 4) move amplitudes between LDS slots.
+//
+// What bounds it (30 qubits, f64): loading and storing the tiles alone takes
+// 6.0-7.5 ms a pass, depending on where the tile's qubits fall on the memory
+// channels (an in-place stream takes 5.3).  Two workgroups share a CU, so one
+// works while the other loads; a further k = 3, 4, 5 gate adds 0.9, 1.6, 3.0
+// ms (matrix cores alone 1.3 and 2.6 for k = 4, 5), where its own pass would
+// take 5.9-6.5.  Measured and not kept: tiles of 2^11 (379 ms against 350 for
+// 90 gates), workgroups that stay and fetch their next tile during the gates
+// (409 against 372 then), operands in LDS instead of in registers (the same
+// time), one workgroup per CU (474-540), wave priorities and staggered starts
+// (no change).
+
+#include "cast_hip.h"
+#include "common.hpp"
+#include "device_core.hpp"
+
+#include <algorithm>
+#include <cstring>
+#include <string>
+
+namespace cast_hip {
+namespace {
+
+using dev::bf16x8_t;
+using dev::f32x4_t;
+using dev::fma_t;
+using dev::insert_zero;
+using dev::NV;
+using dev::Split3;
+using dev::split3;
+
+constexpr uint32_t kMaxOffsets = 13; // one per tile bit
+constexpr int kMaxGroupGates = 64;
+constexpr uint32_t kMaxGroupQubits = 34; // 2^22 workgroups at most
+
+enum Kind : uint32_t { kDense = 0, kDiagonal = 1, kPermutation = 2 };
+
+struct GroupGate {
+  const void *mat;       // dense k >= 4: matrix-core operands (plan.d_op); else the matrix
+  uint64_t cols;         // monomial k <= 4: source column of row r in nibble r
+  uint32_t off2[7];      // LDS byte offsets of the index bits, two per word, in use order
+  uint32_t k;
+  uint32_t kind;
+};
+
+struct GroupArgs {
+  uint32_t n_gates;
+  uint32_t thread_bits;  // log2(threads per workgroup)
+  uint32_t m;            // tile qubits
+  uint32_t xcd_bits;     // 0, or log2(tiles): tiles in XCD order
+  uint8_t s[16];         // tile qubits, ascending
+  GroupGate g[kMaxGroupGates];
+};
+
+// Whether a 16-byte unit holds two amplitudes.
+template <typename T> struct Shape;
+template <> struct Shape<double> {
+  static constexpr int P = 0;
+};
+template <> struct Shape<float> {
+  static constexpr int P = 1;
+};
+
+typedef float Unit __attribute__((ext_vector_type(4))); // 16 bytes
+
+template <typename T> using Const = const __attribute__((address_space(4))) T *;
+
+__device__ __forceinline__ uint32_t offset_of(const GroupGate &g, int b) {
+  return (g.off2[b >> 1] >> (16 * (b & 1))) & 0xffffu;
+}
+
+template <typename T>
+__device__ __forceinline__ typename NV<T>::type lds_get(const unsigned char *lds, uint32_t a) {
+  return *reinterpret_cast<const typename NV<T>::type *>(lds + a);
+}
+template <typename T>
+__device__ __forceinline__ void lds_put(unsigned char *lds, uint32_t a, typename NV<T>::type v) {
+  *reinterpret_cast<typename NV<T>::type *>(lds + a) = v;
+}
+
+// XOR of the offsets first .. first + N - 1 selected by the bits of v.
+template <int N>
+__device__ __forceinline__ uint32_t select_offsets(const GroupGate &g, int first, uint32_t v) {
+  uint32_t a = 0;
+#pragma unroll
+  for (int b = 0; b < N; ++b)
+    a ^= (0u - ((v >> b) & 1u)) & offset_of(g, first + b);
+  return a;
+}
+
+// Dense gate on k <= 3 targets.  Offsets: k targets, R - k combos of the
+// thread, then the thread index bits.  Row r + 1 of the matrix is requested
+// (scalar loads) before row r is used.
+template <typename T, int R, int KL>
+__device__ __forceinline__ void small_gate(unsigned char *lds, const GroupGate &g, uint32_t tid) {
+  constexpr int K = 1 << KL, U = 1 << (R - KL);
+  using V = typename NV<T>::type;
+  typedef T Row __attribute__((ext_vector_type(2 * K)));
+  const uint32_t base = select_offsets<12 - R + Shape<T>::P>(g, R, tid);
+  Const<Row> rows = (Const<Row>)(reinterpret_cast<uintptr_t>(g.mat));
+  Row next = rows[0];
+  __syncthreads();
+  V x[U][K];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      x[u][c] = lds_get<T>(lds, base ^ select_offsets<R>(g, 0, uint32_t(u << KL | c)));
+#pragma unroll
+  for (int r = 0; r < K; ++r) {
+    const Row row = next;
+    if (r + 1 < K)
+      next = rows[r + 1];
+    T ar0[U], ar1[U], ai0[U], ai1[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      ar0[u] = ar1[u] = ai0[u] = ai1[u] = T(0);
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+      const T mr = row[2 * c], mi = row[2 * c + 1];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        ar0[u] = fma_t(mr, x[u][c].x, ar0[u]);
+        ar1[u] = fma_t(mi, x[u][c].y, ar1[u]);
+        ai0[u] = fma_t(mr, x[u][c].y, ai0[u]);
+        ai1[u] = fma_t(mi, x[u][c].x, ai1[u]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      V o;
+      o.x = ar0[u] - ar1[u];
+      o.y = ai0[u] + ai1[u];
+      lds_put<T>(lds, base ^ select_offsets<R>(g, 0, uint32_t(u << KL | r)), o);
+    }
+  }
+}
+
+// Dense gate on the matrix cores, three real products per complex one.
+// Offsets: k targets, 4 column bits (combo of the MFMA tile), R + 2 - k tiles
+// of the wave, wave index bits.  The contraction index is c = j KS + s (j =
+// lane / 16); rows follow the accumulator layout (f64: j + 4 i, f32: 4 j + i,
+// + 16 rb).  A wave reads all its inputs before it writes any output.
+//
+// f64: with P = Re M (vr + vi), Re = P - (Re M + Im M) vi and Im = P + (Im M -
+// Re M) vr: both continue P's accumulator, so no output needs a vector
+// instruction (an f64 MFMA keeps the vector unit busy too).  f32: t1 = Re M
+// vr, t2 = Im M vi, t3 = (Re M + Im M)(vr + vi), Re = t1 - t2, Im = t3 - t1 -
+// t2, the form of the single-gate kernels.
+template <int R, int KL>
+__device__ __forceinline__ void mfma_gate(unsigned char *lds, const GroupGate &g, uint32_t tid,
+                                          double) {
+  constexpr int K = 1 << KL, RB = K / 16, KS = K / 4, LB = R + 2 - KL, NT = 1 << LB;
+  using AV = dev::Acc4<double>::type;
+  typedef double Pair __attribute__((ext_vector_type(2)));
+  const uint32_t lane = tid & 63u, col = lane & 15u, j = lane >> 4, wave = tid >> 6;
+  const uint32_t base = select_offsets<4>(g, KL, col) ^ select_offsets<6 - R>(g, R + 6, wave);
+  const uint32_t in = base ^ select_offsets<2>(g, KL - 2, j);
+  const uint32_t out = base ^ select_offsets<2>(g, 0, j);
+  const Pair *op = static_cast<const Pair *>(g.mat) + lane;
+  Pair a[3][KS / 2];
+  auto load_rows = [&](int rb) {
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+      for (int s = 0; s < KS / 2; ++s)
+        a[m][s] = op[64 * ((m * RB + rb) * (KS / 2) + s)];
+  };
+  load_rows(0);
+  __syncthreads();
+  dev::d2v x[NT][KS];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      x[t][s] = lds_get<double>(lds, in ^ select_offsets<LB>(g, KL + 4, uint32_t(t)) ^
+                                         select_offsets<KL - 2>(g, 0, uint32_t(s)));
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    if (rb > 0)
+      load_rows(rb);
+#pragma unroll
+    for (int t0 = 0; t0 < NT; t0 += 2) { // two tiles: independent accumulator chains
+      constexpr int W = NT < 2 ? NT : 2;
+      AV p[W];
+#pragma unroll
+      for (int w = 0; w < W; ++w)
+        p[w] = AV{0, 0, 0, 0};
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int w = 0; w < W; ++w)
+          p[w] = dev::mfma16(a[0][s / 2][s & 1], x[t0 + w][s].x + x[t0 + w][s].y, p[w]);
+      AV re[W], im[W];
+#pragma unroll
+      for (int w = 0; w < W; ++w)
+        re[w] = im[w] = p[w];
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+          re[w] = dev::mfma16(a[1][s / 2][s & 1], x[t0 + w][s].y, re[w]);
+          im[w] = dev::mfma16(a[2][s / 2][s & 1], x[t0 + w][s].x, im[w]);
+        }
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        const uint32_t ro = out ^ select_offsets<LB>(g, KL + 4, uint32_t(t0 + w)) ^
+                            select_offsets<KL - 4>(g, 4, uint32_t(rb));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          dev::d2v o;
+          o.x = re[w][i];
+          o.y = im[w][i];
+          lds_put<double>(lds, ro ^ select_offsets<2>(g, 2, uint32_t(i)), o);
+        }
+      }
+    }
+  }
+}
+
+template <int R, int KL>
+__device__ __forceinline__ void mfma_gate(unsigned char *lds, const GroupGate &g, uint32_t tid,
+                                          float) {
+  static_assert(KL == 4, "f32 k = 5 has the split products");
+  constexpr int LB = R + 2 - KL, NT = 1 << LB;
+  using AV = dev::Acc4<float>::type;
+  const uint32_t lane = tid & 63u, col = lane & 15u, j = lane >> 4, wave = tid >> 6;
+  const uint32_t base = select_offsets<4>(g, KL, col) ^ select_offsets<7 - R>(g, R + 6, wave);
+  const uint32_t in = base ^ select_offsets<2>(g, 2, j); // rows and columns alike
+  const Unit *op = static_cast<const Unit *>(g.mat) + lane;
+  const Unit ar = op[0], ai = op[64], as = op[128];
+  __syncthreads();
+  dev::f2v x[NT][4];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      x[t][s] = lds_get<float>(lds, in ^ select_offsets<LB>(g, KL + 4, uint32_t(t)) ^
+                                        select_offsets<2>(g, 0, uint32_t(s)));
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    AV t1 = {0, 0, 0, 0}, t2 = {0, 0, 0, 0}, t3 = {0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      t1 = dev::mfma16(ar[s], x[t][s].x, t1);
+      t2 = dev::mfma16(ai[s], x[t][s].y, t2);
+      t3 = dev::mfma16(as[s], x[t][s].x + x[t][s].y, t3);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      dev::f2v o;
+      o.x = t1[i] - t2[i];
+      o.y = t3[i] - t1[i] - t2[i];
+      lds_put<float>(lds, in ^ select_offsets<LB>(g, KL + 4, uint32_t(t)) ^
+                              select_offsets<2>(g, 0, uint32_t(i)),
+                     o);
+    }
+  }
+}
+
+// f32 k = 5 as bf16 split products (the partial products and their order are
+// those of dev::split_tile); the operands are the splits of Re M and Im M.
+// Offsets as in mfma_gate.
+template <int R>
+__device__ __forceinline__ void split_gate5(unsigned char *lds, const GroupGate &g, uint32_t tid) {
+  constexpr int KL = 5, LB = R + 2 - KL, NT = 1 << LB;
+  const uint32_t lane = tid & 63u, col = lane & 15u, j = lane >> 4, wave = tid >> 6;
+  const bf16x8_t *op = static_cast<const bf16x8_t *>(g.mat) + lane;
+  bf16x8_t a[2][3][2]; // [Re, Im][split][row block]
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        a[m][s][h] = op[dev::SplitOperands<5>::at(m, s, h, 0)];
+  const uint32_t base = select_offsets<4>(g, KL, col) ^ select_offsets<7 - R>(g, R + 6, wave);
+  const uint32_t in = base ^ select_offsets<2>(g, 3, j);
+  const uint32_t out = base ^ select_offsets<2>(g, 2, j);
+  __syncthreads();
+  dev::f2v x[NT][8];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      x[t][e] = lds_get<float>(lds, in ^ select_offsets<LB>(g, KL + 4, uint32_t(t)) ^
+                                        select_offsets<3>(g, 0, uint32_t(e)));
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    bf16x8_t br[3], bi[3];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const Split3 sr = split3(x[t][e].x), si = split3(x[t][e].y);
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {
+        br[s][e] = sr.p[s];
+        bi[s][e] = si.p[s];
+      }
+    }
+    f32x4_t t1[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}}, t2[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}},
+            t3[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+    for (int sa = 2; sa >= 0; --sa)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int sb = 2 - sa; sb >= 0; --sb) {
+          t1[h] = dev::mfma_bf16(a[0][sa][h], br[sb], t1[h]);
+          t3[h] = dev::mfma_bf16(a[0][sa][h], bi[sb], t3[h]);
+          t2[h] = dev::mfma_bf16(a[1][sa][h], bi[sb], t2[h]);
+          t3[h] = dev::mfma_bf16(a[1][sa][h], br[sb], t3[h]);
+        }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        dev::f2v o;
+        o.x = t1[h][i] - t2[h][i];
+        o.y = t3[h][i];
+        lds_put<float>(lds,
+                       out ^ select_offsets<LB>(g, KL + 4, uint32_t(t)) ^
+                           select_offsets<2>(g, 0, uint32_t(i)) ^
+                           select_offsets<1>(g, 4, uint32_t(h)),
+                       o);
+      }
+  }
+}
+
+// v times an entry (re, im).
+template <typename T>
+__device__ __forceinline__ typename NV<T>::type times(typename NV<T>::type v, T re, T im) {
+  typename NV<T>::type o;
+  o.x = re * v.x - im * v.y;
+  o.y = re * v.y + im * v.x;
+  return o;
+}
+
+// Monomial gate on k <= R targets (diagonal or permutation): row r takes
+// entry (r, col(r)) times amplitude col(r).  Rows equal to the identity's
+// touch nothing.  Offsets as in small_gate; the mask of the other rows is in
+// the upper half of off2[6].
+template <typename T, int R, int KL>
+__device__ __forceinline__ void monomial_gate(unsigned char *lds, const GroupGate &g,
+                                              uint32_t tid) {
+  constexpr int K = 1 << KL, U = 1 << (R - KL);
+  using V = typename NV<T>::type;
+  const uint32_t base = select_offsets<12 - R + Shape<T>::P>(g, R, tid), active = g.off2[6] >> 16;
+  Const<T> mat = (Const<T>)(reinterpret_cast<uintptr_t>(g.mat));
+  __syncthreads();
+  V x[U][K];
+#pragma unroll
+  for (int r = 0; r < K; ++r)
+    if (active >> r & 1u) {
+      const uint32_t c = uint32_t(g.cols >> (4 * r)) & 15u;
+      const uint32_t co = select_offsets<KL>(g, 0, c);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        x[u][r] = lds_get<T>(lds, base ^ co ^ select_offsets<R>(g, 0, uint32_t(u << KL)));
+    }
+#pragma unroll
+  for (int r = 0; r < K; ++r)
+    if (active >> r & 1u) {
+      const uint32_t c = uint32_t(g.cols >> (4 * r)) & 15u;
+      const T re = mat[2 * (r * K + c)], im = mat[2 * (r * K + c) + 1];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        lds_put<T>(lds, base ^ select_offsets<R>(g, 0, uint32_t(u << KL | r)),
+                   times<T>(x[u][r], re, im));
+    }
+}
+
+// Monomial gate on more than R targets: the targets from the R-th on are the
+// lowest thread index bits, so a wave holds whole combos and reads them
+// before it writes.
+template <typename T, int R>
+__device__ __forceinline__ void wide_monomial_gate(unsigned char *lds, const GroupGate &g,
+                                                   uint32_t tid, uint32_t k, bool diagonal) {
+  constexpr int N = 1 << R;
+  using V = typename NV<T>::type;
+  const uint32_t base = select_offsets<12 - R + Shape<T>::P>(g, R, tid);
+  const uint32_t hi = tid & ((1u << (k - R)) - 1);
+  const V *mat = static_cast<const V *>(g.mat);
+  __syncthreads();
+  V x[N], e[N];
+#pragma unroll
+  for (int c = 0; c < N; ++c) {
+    const uint32_t r = hi << R | uint32_t(c);
+    const uint32_t col = diagonal ? r : uint32_t(g.cols >> (4 * r)) & 15u;
+    e[c] = mat[r << k | col];
+    x[c] = lds_get<T>(lds, base ^ select_offsets<R>(g, 0, col) ^
+                               select_offsets<6 - R>(g, R, (col >> R) ^ hi));
+  }
+#pragma unroll
+  for (int c = 0; c < N; ++c) {
+    // a diagonal entry of exactly 1 leaves the amplitude as it is
+    const bool keep = diagonal && e[c].x == T(1) && e[c].y == T(0);
+    const V o = times<T>(x[c], e[c].x, e[c].y);
+    lds_put<T>(lds, base ^ select_offsets<R>(g, 0, uint32_t(c)), keep ? x[c] : o);
+  }
+}
+
+// The 16-byte units of a thread: unit i * threads + tid of a tile, i < 2^RU.
+template <typename T, int RU> struct TileUnits {
+  static constexpr int P = Shape<T>::P, N = 1 << RU;
+  Unit *p;          // global address of unit tid
+  uint64_t reg[RU]; // global unit offsets of the bits of i
+  uint32_t lds_t, thread_bits;
+
+  __device__ __forceinline__ TileUnits(T *sv, const GroupArgs &a, uint64_t tile, uint32_t tid) {
+    for (uint32_t b = 0; b < a.m; ++b)
+      tile = insert_zero(tile, a.s[b]);
+#pragma unroll
+    for (int b = 0; b < 12 - RU; ++b)
+      tile |= uint64_t((tid >> b) & 1u) << a.s[b + P];
+    thread_bits = a.thread_bits;
+#pragma unroll
+    for (int b = 0; b < RU; ++b)
+      reg[b] = (uint64_t(1) << a.s[thread_bits + b + P]) >> P;
+    p = reinterpret_cast<Unit *>(sv) + (tile >> P);
+    lds_t = tid ^ ((tid >> 4) & 15u) ^ ((tid >> 8) & 15u);
+  }
+  __device__ __forceinline__ Unit *global(int i) const {
+    uint64_t o = 0;
+#pragma unroll
+    for (int b = 0; b < RU; ++b)
+      o |= (i >> b & 1) ? reg[b] : 0;
+    return p + o;
+  }
+  __device__ __forceinline__ uint32_t local(int i) const { // LDS byte offset
+    const uint32_t u = uint32_t(i) << thread_bits;
+    return 16 * (lds_t ^ u ^ ((u >> 4) & 15u) ^ ((u >> 8) & 15u));
+  }
+};
+
+// R amplitude bits per thread.  The gate functions begin with the barrier that
+// orders them after the previous gate; what they need from global memory is
+// requested before it.
+template <typename T, int R>
+__global__ void __launch_bounds__(1 << (12 + Shape<T>::P - R), R == 3 + Shape<T>::P ? 4 : 2)
+    k_group(T *__restrict__ sv, GroupArgs a) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  using Units = TileUnits<T, R - Shape<T>::P>;
+  const uint32_t tid = threadIdx.x;
+  uint64_t tile = blockIdx.x;
+  if (a.xcd_bits)
+    tile = ((tile & 7u) << (a.xcd_bits - 3)) | (tile >> 3);
+  {
+    const Units t(sv, a, tile, tid);
+    Unit x[Units::N];
+#pragma unroll
+    for (int i = 0; i < Units::N; ++i)
+      x[i] = __builtin_nontemporal_load(t.global(i));
+#pragma unroll
+    for (int i = 0; i < Units::N; ++i)
+      *reinterpret_cast<Unit *>(lds + t.local(i)) = x[i];
+  }
+  for (uint32_t gi = 0; gi < a.n_gates; ++gi) {
+    const GroupGate &g = a.g[gi];
+    if (g.kind != kDense) {
+      switch (g.k) {
+      case 1:
+        monomial_gate<T, R, 1>(lds, g, tid);
+        break;
+      case 2:
+        monomial_gate<T, R, 2>(lds, g, tid);
+        break;
+      case 3:
+        monomial_gate<T, R, 3>(lds, g, tid);
+        break;
+      default:
+        if (g.k == 4 && R >= 4)
+          monomial_gate<T, R, R < 4 ? R : 4>(lds, g, tid);
+        else
+          wide_monomial_gate<T, R>(lds, g, tid, g.k, g.kind == kDiagonal);
+        break;
+      }
+    } else {
+      switch (g.k) {
+      case 1:
+        small_gate<T, R, 1>(lds, g, tid);
+        break;
+      case 2:
+        small_gate<T, R, 2>(lds, g, tid);
+        break;
+      case 3:
+        small_gate<T, R, 3>(lds, g, tid);
+        break;
+      case 4:
+        mfma_gate<R, 4>(lds, g, tid, T(0));
+        break;
+      default:
+        if constexpr (sizeof(T) == 8)
+          mfma_gate<R, 5>(lds, g, tid, T(0));
+        else
+          split_gate5<R>(lds, g, tid);
+        break;
+      }
+    }
+  }
+  __syncthreads();
+  // Addresses again from the thread index: kept over the gates they would
+  // take the registers that the gates need.
+  uint32_t again = tid;
+  asm volatile("" : "+v"(again));
+  const Units t(sv, a, tile, again);
+#pragma unroll
+  for (int i = 0; i < Units::N; ++i)
+    __builtin_nontemporal_store(*reinterpret_cast<const Unit *>(lds + t.local(i)), t.global(i));
+}
+
+// ── Host side ───────────────────────────────────────────────────────────────
+
+bool is_diagonal(const GatePlan &p) {
+  for (uint32_t i = 0; i < p.n_active; ++i)
+    if (p.act_row[i] != p.act_col[i])
+      return false;
+  return true;
+}
+
+uint32_t max_tile(uint8_t precision) { return precision == 0 ? 13 : 12; }
+// Lowest qubits that every tile holds: 64-byte rows.  Fewer leave more qubits
+// to the gates, so fewer passes, and tiles that share 128-byte lines run on
+// one XCD at about the same time (XCD order).  90 gates at 30 qubits, ms at
+// 16, 32, 64, 128 and 256 bytes: f64 380, 346, 350, 361, 379; f32 (32 to 128
+// bytes) 162, 160, 162.
+uint32_t low_qubits(uint8_t precision) { return precision == 0 ? 3 : 2; }
+uint32_t regs_log2(uint8_t precision) { return precision == 0 ? 4 : 3; }
+
+bool can_join(const GatePlan &p, uint32_t n) {
+  if (n < regs_log2(p.precision) + 6 || n > kMaxGroupQubits || n < p.k || p.q[p.k - 1] >= n)
+    return false;
+  if (p.variant == 2)
+    return is_diagonal(p) || p.k <= 4;
+  return p.k <= 5;
+}
+
+// LDS byte offset of local index bit `p` (see the file comment).
+uint32_t bit_offset(uint32_t p, bool f32) {
+  if (f32 && p == 0)
+    return 8;
+  const uint32_t u = f32 ? p - 1 : p;
+  return 16 * ((1u << u) | (u >= 4 ? 1u << (u & 3) : 0u));
+}
+
+template <typename T, int R>
+void launch_k_group(dim3 grid, dim3 block, size_t lds, hipStream_t stream, void *sv,
+                    const GroupArgs &a) {
+  hipLaunchKernelGGL((k_group<T, R>), grid, block, lds, stream, static_cast<T *>(sv), a);
+}
+
+} // namespace
+
+// Operand vector x of lane l is 16-byte unit x * 64 + l, so that a wave reads
+// 1 KiB in order.
+//   f64: x = (matrix * RB + rb) * KS / 2 + s / 2, two entries of row 16 rb + l %
+//        16 from column (l / 16) KS + s on, matrices Re M, -(Re M + Im M), Im M -
+//        Re M;
+//   f32 k = 4: x = matrix, four entries of row l % 16 from column 4 (l / 16)
+//        on, matrices Re M, Im M, Re M + Im M;
+//   f32 k = 5: the bf16 fragments of dev::split_stage.
+size_t group_operand_bytes(uint32_t k, uint8_t precision) {
+  const size_t K = size_t(1) << k;
+  if (precision == 0)
+    return k == 4 ? 3 * K * K * sizeof(float) : dev::SplitOperands<5>::kFragments * 16;
+  return 3 * K * K * sizeof(double);
+}
+
+namespace {
+// Round to nearest even, as the device's conversion does (finite values).
+uint16_t to_bf16(float x) {
+  uint32_t b;
+  std::memcpy(&b, &x, 4);
+  if ((b & 0x7fffffffu) > 0x7f800000u)
+    return uint16_t(b >> 16 | 0x40u); // NaN
+  return uint16_t((b + 0x7fffu + (b >> 16 & 1u)) >> 16);
+}
+float from_bf16(uint16_t h) {
+  const uint32_t b = uint32_t(h) << 16;
+  float x;
+  std::memcpy(&x, &b, 4);
+  return x;
+}
+} // namespace
+
+void group_operands(const double *m, uint32_t k, uint8_t precision, void *out) {
+  const uint32_t K = 1u << k, RB = K / 16, KS = K / 4;
+  auto re = [&](uint32_t r, uint32_t c) { return m[2 * (r * K + c)]; };
+  auto im = [&](uint32_t r, uint32_t c) { return m[2 * (r * K + c) + 1]; };
+  if (precision == 1) {
+    double *d = static_cast<double *>(out);
+    for (uint32_t x = 0; x < 3; ++x)
+      for (uint32_t rb = 0; rb < RB; ++rb)
+        for (uint32_t s = 0; s < KS; ++s)
+          for (uint32_t l = 0; l < 64; ++l) {
+            const uint32_t r = 16 * rb + (l & 15u), c = (l >> 4) * KS + s;
+            const double v = x == 0   ? re(r, c)
+                             : x == 1 ? -(re(r, c) + im(r, c))
+                                      : im(r, c) - re(r, c);
+            d[(((x * RB + rb) * (KS / 2) + s / 2) * 64 + l) * 2 + (s & 1u)] = v;
+          }
+  } else if (k == 4) {
+    float *f = static_cast<float *>(out);
+    for (uint32_t x = 0; x < 3; ++x)
+      for (uint32_t l = 0; l < 64; ++l)
+        for (uint32_t s = 0; s < 4; ++s) {
+          const uint32_t r = l & 15u, c = (l >> 4) * 4 + s;
+          f[(x * 64 + l) * 4 + s] =
+              float(x == 0 ? re(r, c) : x == 1 ? im(r, c) : re(r, c) + im(r, c));
+        }
+  } else {
+    uint16_t *h = static_cast<uint16_t *>(out);
+    for (uint32_t x = 0; x < 2; ++x)
+      for (uint32_t rb = 0; rb < 2; ++rb)
+        for (uint32_t l = 0; l < 64; ++l)
+          for (uint32_t e = 0; e < 8; ++e) {
+            const uint32_t r = 16 * rb + (l & 15u), c = 8 * (l >> 4) + e;
+            float rest = float(x == 0 ? re(r, c) : im(r, c));
+            for (uint32_t s = 0; s < 3; ++s) {
+              const uint16_t b = to_bf16(rest);
+              h[(size_t(dev::SplitOperands<5>::at(int(x), int(s), int(rb), 0)) + l) * 8 + e] = b;
+              rest -= from_bf16(b);
+            }
+          }
+  }
+}
+
+GroupLimits group_limits(const GatePlan &p, uint32_t n) {
+  GroupLimits l{};
+  if (!can_join(p, n))
+    return l;
+  for (uint32_t b = 0; b < p.k; ++b)
+    l.targets |= uint64_t(1) << p.q[b];
+  l.max_qubits = std::min(n, max_tile(p.precision));
+  l.low_qubits = low_qubits(p.precision);
+  l.max_gates = kMaxGroupGates;
+  return l;
+}
+
+void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stream, void *sv,
+                  uint32_t n) {
+  if (n_plans == 0)
+    return;
+  if (n_plans > size_t(kMaxGroupGates))
+    throw Error("a gate group holds at most " + std::to_string(kMaxGroupGates) + " gates");
+  if (n > 40)
+    throw Error("statevector qubit count " + std::to_string(n) + " is out of range");
+  const uint8_t prec = plans[0]->precision;
+  const bool f32 = prec == 0;
+  uint64_t set = 0;
+  for (size_t i = 0; i < n_plans; ++i) {
+    const GatePlan &p = *plans[i];
+    if (p.precision != prec)
+      throw Error("grouped plans must share the precision");
+    if (!can_join(p, n))
+      throw Error("gate " + std::to_string(i) + " cannot join a group on a " + std::to_string(n) +
+                  "-qubit statevector");
+    for (uint32_t b = 0; b < p.k; ++b)
+      set |= uint64_t(1) << p.q[b];
+  }
+  const uint32_t m = std::min(n, max_tile(prec));
+  // Amplitudes per thread: twice as many, with half the threads, from 2^10
+  // tiles on.  There the tiles are enough to fill the chip and a wave that
+  // runs more MFMA tiles per operand load is the faster one (30 qubits f64,
+  // 90 gates in 44 passes: 373 ms against 393); below it the latency of a
+  // gate counts (12 qubits f64, 23 gates: 64 us against 74).
+  const bool large = n - m >= 10;
+  const uint32_t R = regs_log2(prec) + large;
+  const uint32_t low = low_qubits(prec);
+  set |= (uint64_t(1) << low) - 1;
+  if (uint32_t(__builtin_popcountll(set)) > m)
+    throw Error("grouped gates act on more than " + std::to_string(m) + " qubits (the lowest " +
+                std::to_string(low) + " included)");
+  // The rest of the tile: the lowest free qubits, which lengthens its rows.
+  for (uint32_t q = 0; uint32_t(__builtin_popcountll(set)) < m; ++q)
+    set |= uint64_t(1) << q;
+
+  GroupArgs a{};
+  a.m = m;
+  a.thread_bits = m - R;
+  uint8_t local[64] = {};
+  {
+    uint32_t i = 0;
+    for (uint32_t q = 0; q < n; ++q)
+      if (set >> q & 1u) {
+        local[q] = uint8_t(i);
+        a.s[i++] = uint8_t(q);
+      }
+  }
+  for (size_t i = 0; i < n_plans; ++i) {
+    const GatePlan &p = *plans[i];
+    const bool mono = p.variant == 2;
+    if (mono && p.n_active == 0)
+      continue; // identity
+    GroupGate &g = a.g[a.n_gates++];
+    const bool diag = mono && is_diagonal(p);
+    const bool mfma = !mono && p.k >= 4;
+    g.mat = mfma ? p.d_op : p.d_mat;
+    g.k = p.k;
+    g.kind = mono ? (diag ? kDiagonal : kPermutation) : kDense;
+    uint32_t used = 0;
+    for (uint32_t b = 0; b < p.k; ++b)
+      used |= 1u << local[p.q[b]];
+    if (mono && p.k <= 4) {
+      for (uint32_t r = 0; r < (1u << p.k); ++r)
+        g.cols |= uint64_t(r) << (4 * r);
+      for (uint32_t x = 0; x < p.n_active; ++x) {
+        g.cols &= ~(uint64_t(15) << (4 * p.act_row[x]));
+        g.cols |= uint64_t(p.act_col[x]) << (4 * p.act_row[x]);
+        g.off2[6] |= 0x10000u << p.act_row[x];
+      }
+    }
+    // The other positions, those whose banks differ first (they go to
+    // consecutive lanes).
+    uint32_t order[kMaxOffsets] = {}, lanes = 0, rest[kMaxOffsets] = {}, n_rest = 0, banks = 0;
+    for (uint32_t b = 0; b < m; ++b) {
+      if (used >> b & 1u)
+        continue;
+      const uint32_t bank = f32 ? (b == 0 ? 4u : (b - 1) & 3u) : b & 3u;
+      if (!(banks >> bank & 1u)) {
+        banks |= 1u << bank;
+        order[lanes++] = b;
+      } else {
+        rest[n_rest++] = b;
+      }
+    }
+    for (uint32_t b = 0; b < n_rest; ++b)
+      order[lanes + b] = rest[b];
+    const uint32_t free_bits = m - p.k;
+    uint32_t off[kMaxOffsets + 1] = {}, w = 0;
+    for (uint32_t b = 0; b < p.k; ++b)
+      off[w++] = bit_offset(local[p.q[b]], f32);
+    if (mfma) { // columns, tiles of the wave, waves: as ordered
+      for (uint32_t b = 0; b < free_bits; ++b)
+        off[w++] = bit_offset(order[b], f32);
+    } else { // combos of the thread last in the order, threads first
+      const uint32_t u = p.k < R ? R - p.k : 0;
+      for (uint32_t b = 0; b < u; ++b)
+        off[w++] = bit_offset(order[free_bits - u + b], f32);
+      for (uint32_t b = 0; b < free_bits - u; ++b)
+        off[w++] = bit_offset(order[b], f32);
+    }
+    for (uint32_t b = 0; b < kMaxOffsets; ++b)
+      g.off2[b >> 1] |= off[b] << (16 * (b & 1));
+  }
+  if (a.n_gates == 0)
+    return;
+  const uint32_t tile_bits = n - m;
+  a.xcd_bits = tile_bits >= 6 ? tile_bits : 0;
+  const size_t lds = size_t(16) << (m - (f32 ? 1 : 0));
+  const dim3 grid(1u << tile_bits), block(1u << a.thread_bits);
+  if (f32)
+    large ? launch_k_group<float, 5>(grid, block, lds, stream, sv, a)
+          : launch_k_group<float, 4>(grid, block, lds, stream, sv, a);
+  else
+    large ? launch_k_group<double, 4>(grid, block, lds, stream, sv, a)
+          : launch_k_group<double, 3>(grid, block, lds, stream, sv, a);
+  check(hipGetLastError(), "hipLaunchKernelGGL(k_group)");
+}
+
+} // namespace cast_hip

@@ -15,6 +15,7 @@
 #include "fusion.hpp"
 #include "hip_backend.hpp"
 #include "qasm.hpp"
+#include "schedule.hpp"
 #include "serving.hpp"
 #include "trajectory.hpp"
 
@@ -337,6 +338,24 @@ PYBIND11_MODULE(_host, m) {
   py::enum_<cast_precision_t>(m, "Precision")
       .value("F32", CAST_PRECISION_F32)
       .value("F64", CAST_PRECISION_F64);
+
+  // The passes that an untimed sync cuts a gate list into (schedule.hpp).
+  m.def("plan_passes",
+        [](const std::vector<std::vector<uint32_t>> &targets, const std::vector<bool> &may_join,
+           uint32_t n_qubits, uint32_t max_qubits, uint32_t low_qubits, uint32_t max_gates) {
+          std::vector<PlannedGate> gates(targets.size());
+          for (size_t i = 0; i < targets.size(); ++i) {
+            for (uint32_t q : targets[i])
+              gates[i].qubits |= uint64_t(1) << q;
+            gates[i].may_join = may_join.at(i);
+          }
+          PassPlanner planner(std::move(gates), {n_qubits, max_qubits, low_qubits, max_gates});
+          std::vector<std::vector<uint32_t>> out(1);
+          while (planner.next(out.back()))
+            out.emplace_back();
+          out.pop_back();
+          return out;
+        });
 
   py::class_<HipKernelGenSpec>(m, "HipKernelGenSpec")
       .def(py::init<>())

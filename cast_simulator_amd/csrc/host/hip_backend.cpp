@@ -1,6 +1,8 @@
 // Host-side gfx950 backend over the C ABI; see hip_backend.hpp.
 #include "hip_backend.hpp"
 
+#include "schedule.hpp"
+
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -277,7 +279,7 @@ void HipKernelManager::apply(KernelId id, HipStatevector &sv) {
     throw Error("statevector precision does not match kernel precision");
   if (info.qubits[info.n_qubits - 1] >= sv.n_qubits())
     throw Error("gate acts on a qubit outside the statevector");
-  const void *plan = it->second;
+  const void *plan = it->second, *base = it->second;
   int cand = -1;
   // Tuning applies to dense plans of the automatic family on large states.
   if (autotune_ && spec_.variant == CAST_HIP_VARIANT_AUTO && sv.n_qubits() >= tune_min_qubits_ &&
@@ -296,7 +298,7 @@ void HipKernelManager::apply(KernelId id, HipStatevector &sv) {
       plan = st.plans[best];
     }
   }
-  pending_.push_back({id, sv.dptr(), sv.n_qubits(), plan, cand});
+  pending_.push_back({id, sv.dptr(), sv.n_qubits(), plan, base, cand});
 }
 
 uint32_t HipKernelManager::tune(const std::vector<KernelId> &ids, HipStatevector &sv,
@@ -366,11 +368,54 @@ void *HipKernelManager::stream() {
   return stream_;
 }
 
+// Gates on different statevectors are independent, so each statevector's
+// gates are taken together, in their order, and cut into passes.  A forced
+// kernel variant keeps one launch per gate.
+void HipKernelManager::launch_passes_locked(const std::vector<Pending> &work,
+                                            std::vector<size_t> &sampled) {
+  char err[kErr];
+  std::vector<std::vector<size_t>> lists;
+  std::unordered_map<uint64_t, size_t> list_of;
+  for (size_t i = 0; i < work.size(); ++i) {
+    const auto [it, fresh] = list_of.try_emplace(work[i].dptr, lists.size());
+    if (fresh)
+      lists.emplace_back();
+    lists[it->second].push_back(i);
+  }
+  std::vector<const void *> plans;
+  for (const auto &list : lists) {
+    const uint64_t dptr = work[list[0]].dptr;
+    const uint32_t n = work[list[0]].n_qubits;
+    auto single = [&](uint32_t j) {
+      const Pending &w = work[list[j]];
+      if (w.cand >= 0) {
+        ensure_events_locked(2 * sampled.size() + 2);
+        throw_if(cast_hip_event_record(events_[2 * sampled.size()], stream_, err, kErr), err);
+      }
+      throw_if(cast_hip_gate_apply(w.plan, stream_, dptr, n, err, kErr), err);
+      if (w.cand >= 0) {
+        throw_if(cast_hip_event_record(events_[2 * sampled.size() + 1], stream_, err, kErr), err);
+        sampled.push_back(list[j]);
+      }
+    };
+    if (list.size() == 1 || spec_.variant != CAST_HIP_VARIANT_AUTO) {
+      for (size_t j = 0; j < list.size(); ++j)
+        single(uint32_t(j));
+      continue;
+    }
+    plans.clear();
+    for (size_t i : list)
+      plans.push_back(work[i].base);
+    apply_in_passes(plans, stream_, dptr, n, single);
+  }
+}
+
 SyncStats HipKernelManager::sync(bool timed) {
   const auto w0 = std::chrono::steady_clock::now();
   std::vector<Pending> work;
   void *stream = nullptr;
   std::vector<void *> ev;
+  std::vector<size_t> sampled; // tuning samples of an untimed call
   {
     std::lock_guard<std::mutex> lock(mu_);
     SyncStats empty;
@@ -380,40 +425,48 @@ SyncStats HipKernelManager::sync(bool timed) {
     stream = stream_;
     work.swap(pending_);
     char err[kErr];
-    for (const auto &w : work)
-      timed = timed || w.cand >= 0; // tuning samples are always timed
     if (timed) {
       ensure_events_locked(work.size() + 1);
       ev.assign(events_.begin(), events_.begin() + long(work.size() + 1));
       if (!work.empty())
         throw_if(cast_hip_event_record(ev[0], stream, err, kErr), err);
-    }
-    for (size_t i = 0; i < work.size(); ++i) {
-      throw_if(cast_hip_gate_apply(work[i].plan, stream, work[i].dptr, work[i].n_qubits, err,
-                                   kErr),
-               err);
-      if (timed)
+      for (size_t i = 0; i < work.size(); ++i) {
+        throw_if(cast_hip_gate_apply(work[i].plan, stream, work[i].dptr, work[i].n_qubits, err,
+                                     kErr),
+                 err);
         throw_if(cast_hip_event_record(ev[i + 1], stream, err, kErr), err);
+      }
+    } else {
+      launch_passes_locked(work, sampled);
+      ev.assign(events_.begin(), events_.begin() + long(2 * sampled.size()));
     }
   }
   char err[kErr];
   throw_if(cast_hip_stream_sync(stream, err, kErr), err);
   SyncStats st;
+  std::vector<std::pair<size_t, double>> samples; // (queue position, seconds)
+  auto elapsed = [&](size_t a) {
+    float ms = 0.f;
+    throw_if(cast_hip_event_elapsed_ms(ev[a], ev[a + 1], &ms, err, kErr), err);
+    return double(ms) * 1e-3;
+  };
   if (timed) {
     for (size_t i = 0; i < work.size(); ++i) {
-      float ms = 0.f;
-      throw_if(cast_hip_event_elapsed_ms(ev[i], ev[i + 1], &ms, err, kErr), err);
-      st.kernels.push_back({work[i].id, double(ms) * 1e-3});
+      st.kernels.push_back({work[i].id, elapsed(i)});
+      if (work[i].cand >= 0)
+        samples.emplace_back(i, st.kernels.back().gpu_s);
     }
+  }
+  for (size_t s = 0; s < sampled.size(); ++s)
+    samples.emplace_back(sampled[s], elapsed(2 * s));
+  if (!samples.empty()) {
     std::lock_guard<std::mutex> lock(mu_);
-    for (size_t i = 0; i < work.size(); ++i) {
-      if (work[i].cand < 0)
-        continue;
+    for (const auto &[i, seconds] : samples) {
       auto it = tune_.find(std::make_pair(work[i].id, work[i].n_qubits));
       if (it == tune_.end() || it->second.chosen >= 0)
         continue;
       TuneState &ts = it->second;
-      ts.samples[size_t(work[i].cand)].push_back(st.kernels[i].gpu_s);
+      ts.samples[size_t(work[i].cand)].push_back(seconds);
       // best minimum so far; drop candidates beyond the margin
       double best = 1e300;
       size_t arg = 0;

@@ -169,8 +169,9 @@ private:
     KernelId id;
     uint64_t dptr;
     uint32_t n_qubits;
-    const void *plan;
-    int cand; // tuning candidate index, -1 when not a tuning sample
+    const void *plan; // launched where the gate runs by itself
+    const void *base; // the gate's own plan, for a pass with other gates
+    int cand;         // tuning candidate index, -1 when not a tuning sample
   };
   struct TuneState {
     std::vector<uint32_t> fams;
@@ -179,6 +180,9 @@ private:
     std::vector<char> dropped;
     int chosen = -1;
   };
+  // Untimed work in few passes; the queue positions of tuning samples (each
+  // between two events) go to `sampled`.
+  void launch_passes_locked(const std::vector<Pending> &work, std::vector<size_t> &sampled);
   void ensure_stream_locked();
   void ensure_events_locked(size_t n);
   TuneState &tune_state_locked(KernelId id, uint32_t n);

@@ -255,6 +255,30 @@ int cast_hip_gate_apply_batch(const void *const *plans, const uint64_t *svs,
                               const uint32_t *sv_n_qubits, size_t n_items, void *stream,
                               char *err_buf, size_t err_buf_len);
 
+/* Gate groups: consecutive gates whose targets together lie in few qubits run
+ * as ONE pass over the statevector (one read and one write of every amplitude
+ * for the whole group; the gates are applied to tiles held in LDS, each in
+ * the statevector's precision).  cast_hip_gate_group_info says whether a plan
+ * may join a group on sv_n_qubits qubits (targets = 0: it may not) and what a
+ * group holds: at most max_gates gates, whose targets together with the
+ * low_qubits lowest qubits are at most max_qubits qubits.
+ * cast_hip_gate_apply_group enqueues plans[0], plans[1], ... in that order on
+ * `stream`; a plan's forced kernel variant does not apply there.  Plans that
+ * may not join, or too many qubits or gates, are an error.  No reference
+ * counterpart (the reference launches one kernel per gate). */
+typedef struct cast_hip_group_info_t {
+  uint64_t targets; /* bit q set: the gate acts on qubit q; 0: cannot join */
+  uint32_t max_qubits;
+  uint32_t low_qubits;
+  uint32_t max_gates;
+  uint32_t reserved;
+} cast_hip_group_info_t;
+int cast_hip_gate_group_info(const void *plan, uint32_t sv_n_qubits, cast_hip_group_info_t *out,
+                             char *err_buf, size_t err_buf_len);
+int cast_hip_gate_apply_group(const void *const *plans, size_t n_plans, void *stream,
+                              uint64_t sv_dptr, uint32_t sv_n_qubits, char *err_buf,
+                              size_t err_buf_len);
+
 /* ⟨Z_a Z_b⟩ for n_pairs qubit pairs (pairs = [a0,b0,a1,b1,...]), accumulated
  * in f64 over |amp|^2; no normalisation is applied.  Synchronous on `stream`.
  * No reference counterpart (the reference downloads the whole statevector,
