@@ -653,7 +653,7 @@ int cast_hip_gate_apply_batch(const void *const *plans, const uint64_t *svs,
       return;
     if (!plans || !svs || !sv_n_qubits)
       throw Error("null argument");
-    std::vector<BatchItem> items(n_items);
+    std::vector<BatchItem> lists[2]; // direct kernel, matrix cores
     const GatePlan *p0 = static_cast<const GatePlan *>(plans[0]);
     if (!p0)
       throw Error("null plan at index 0");
@@ -670,16 +670,18 @@ int cast_hip_gate_apply_batch(const void *const *plans, const uint64_t *svs,
       if (n < p->k || p->q[p->k - 1] >= n || n > 40)
         throw Error("item " + std::to_string(i) + ": gate does not fit a " +
                     std::to_string(n) + "-qubit statevector");
-      BatchItem &it = items[i];
+      const bool cores = batch_on_matrix_cores(*p, n);
+      BatchItem &it = lists[cores].emplace_back();
       it.sv = reinterpret_cast<void *>(svs[i]);
-      it.mat = p->d_mat;
+      it.mat = cores ? p->d_mat3 : p->d_mat;
       it.combos = uint64_t(1) << (n - p->k);
       it.k = uint8_t(p->k);
       for (uint32_t b = 0; b < 6; ++b)
         it.q[b] = uint8_t(b < p->k ? p->q[b] : 0);
     }
-    launch_gate_batch(items.data(), n_items, p0->precision, p0->k,
-                      static_cast<hipStream_t>(stream));
+    for (int cores = 0; cores < 2; ++cores)
+      launch_gate_batch(lists[cores].data(), lists[cores].size(), p0->precision, p0->k, cores != 0,
+                        static_cast<hipStream_t>(stream));
   });
 }
 

@@ -115,8 +115,11 @@ struct BatchItem {
   uint8_t k;
   uint8_t pad;
 };
+// Whether an item of a batch runs on the matrix cores (its matrix then is
+// plan.d_mat3); the others run the direct kernel on plan.d_mat.
+bool batch_on_matrix_cores(const GatePlan &plan, uint32_t n_qubits);
 void launch_gate_batch(const BatchItem *items, size_t n, uint8_t precision, uint32_t k,
-                       hipStream_t stream);
+                       bool matrix_cores, hipStream_t stream);
 
 // Gate groups (group_kernels.hip): whether a plan may run in a group on an
 // n-qubit statevector (targets = 0: it may not), and what a group may hold.

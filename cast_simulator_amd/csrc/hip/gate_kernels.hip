@@ -18,8 +18,9 @@
 //                touch consecutive amplitudes.
 //   k_monomial   <= 1 nonzero per row: touches only rows that differ from the
 //                identity row, so e.g. CZ / CP move 1/4 of the bytes.
-//   k_dense_batch  k_dense over many (matrix, statevector) items, item =
-//                blockIdx.z (cast_hip_gate_apply_batch).
+//   k_dense_batch, k_mfma_batch  k_dense or the matrix-core tile loops over
+//                many (matrix, statevector) items, item = blockIdx.z
+//                (cast_hip_gate_apply_batch).
 //   k_tile, k_tile3, k_mfma, k_mfma6, k_mfma_split: see their sections.
 //
 // Tile orders (wave tiles and matrix-core tiles): launch order, the low
@@ -200,8 +201,8 @@ using dev::Acc4;
 using dev::mfma16;
 
 template <typename T, int KL>
-__global__ void __launch_bounds__(256) k_mfma(T *__restrict__ sv, const T *__restrict__ m3,
-                                              GateGeom g, uint64_t n_tiles) {
+__device__ __forceinline__ void mfma_tiles(T *__restrict__ sv, const T *__restrict__ m3,
+                                           const GateGeom &g, uint64_t n_tiles) {
   constexpr int K = 1 << KL, RB = K / 16, KS = K / 4;
   static_assert(RB >= 1, "MFMA path needs k >= 4");
   using VT = typename V2<T>::type;
@@ -263,6 +264,12 @@ __global__ void __launch_bounds__(256) k_mfma(T *__restrict__ sv, const T *__res
   }
 }
 
+template <typename T, int KL>
+__global__ void __launch_bounds__(256) k_mfma(T *__restrict__ sv, const T *__restrict__ m3,
+                                              GateGeom g, uint64_t n_tiles) {
+  mfma_tiles<T, KL>(sv, m3, g, n_tiles);
+}
+
 // ── Matrix cores, k = 6: real matrices in LDS ──────────────────────────────
 //
 // Same three-product contraction as k_mfma for K = 64, where the A operands
@@ -276,8 +283,8 @@ __global__ void __launch_bounds__(256) k_mfma(T *__restrict__ sv, const T *__res
 constexpr unsigned kMfma6Block = 512;
 
 template <typename T>
-__global__ void __launch_bounds__(kMfma6Block) k_mfma6(T *__restrict__ sv, const T *__restrict__ m3,
-                                                       GateGeom g, uint64_t n_tiles) {
+__device__ __forceinline__ void mfma6_tiles(T *__restrict__ sv, const T *__restrict__ m3,
+                                            const GateGeom &g, uint64_t n_tiles) {
   constexpr int KL = 6, K = 64, RB = 4, KS = 16;
   using VT = typename V2<T>::type;
   using AV = typename Acc4<T>::type;
@@ -338,6 +345,12 @@ __global__ void __launch_bounds__(kMfma6Block) k_mfma6(T *__restrict__ sv, const
   }
 }
 
+template <typename T>
+__global__ void __launch_bounds__(kMfma6Block) k_mfma6(T *__restrict__ sv, const T *__restrict__ m3,
+                                                       GateGeom g, uint64_t n_tiles) {
+  mfma6_tiles<T>(sv, m3, g, n_tiles);
+}
+
 // ── Matrix cores, f32 k = 5, 6 through bf16 split products ────────────────
 //
 // On the f32 matrix cores (157 TFLOP/s) a dense 6-qubit f32 gate is
@@ -352,9 +365,8 @@ constexpr unsigned kSplitBlock = 256;
 // One tile per wave step (two per step at k = 5 measured -0.6 % at 30
 // qubits and +1.8 % at 34 on the config-3 circuit's gates).
 template <int KL>
-__global__ void __launch_bounds__(kSplitBlock) k_mfma_split(float *__restrict__ sv,
-                                                          const float *__restrict__ m3,
-                                                          GateGeom g, uint64_t n_tiles) {
+__device__ __forceinline__ void split_tiles(float *__restrict__ sv, const float *__restrict__ m3,
+                                            const GateGeom &g, uint64_t n_tiles) {
   __shared__ dev::bf16x8_t a_lds[dev::SplitOperands<KL>::kFragments];
   dev::split_stage<KL>(m3, a_lds);
   __syncthreads();
@@ -364,6 +376,13 @@ __global__ void __launch_bounds__(kSplitBlock) k_mfma_split(float *__restrict__ 
   for (uint64_t t = dev::grid_wave(g.xcd); t < n_tiles;
        t += n_waves)
     dev::split_tile<KL>(amp, amp, a_lds, g.q, sl, dev::swizzled_tile(t, g.swz));
+}
+
+template <int KL>
+__global__ void __launch_bounds__(kSplitBlock) k_mfma_split(float *__restrict__ sv,
+                                                          const float *__restrict__ m3,
+                                                          GateGeom g, uint64_t n_tiles) {
+  split_tiles<KL>(sv, m3, g, n_tiles);
 }
 
 // ── Batched dense: item = blockIdx.z ────────────────────────────────────────
@@ -391,6 +410,39 @@ __global__ void __launch_bounds__(256) k_dense_batch(BatchArgs a) {
   const uint64_t c = (uint64_t(blockIdx.y) * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
   if (c < it.combos)
     dev::dense_combo<T, KL>(amp, amp, mat, combo_base<KL>(c, q), delta);
+}
+
+// Batched matrix-core kernels: the single-gate tile loops on each item.  With
+// one combo per lane a k = 6 item keeps 64 amplitudes in registers and spills,
+// and a small statevector has too few combos to hide that: over a serving run
+// of 12 to 18 qubits a launch of about 20 items took 425 us (f64 k = 6), 169
+// (f32 k = 6), 46 and 42 (k = 5), now 27, 9.6, 11.5 and 5.9.
+__device__ __forceinline__ GateGeom batch_geom(const BatchItem &it) {
+  GateGeom g{};
+  g.combos = it.combos;
+  g.k = it.k;
+#pragma unroll
+  for (int b = 0; b < 6; ++b)
+    g.q[b] = it.q[b];
+  return g;
+}
+
+template <typename T, int KL>
+__global__ void __launch_bounds__(KL == 6 && sizeof(T) == 8 ? kMfma6Block : 256)
+    k_mfma_batch(BatchArgs a) {
+  const BatchItem &it = a.it[blockIdx.z];
+  const uint64_t n_tiles = it.combos / 16;
+  if (uint64_t(blockIdx.x) * (blockDim.x >> 6) >= n_tiles)
+    return; // whole block
+  T *sv = reinterpret_cast<T *>(it.sv);
+  const T *m3 = reinterpret_cast<const T *>(it.mat);
+  const GateGeom g = batch_geom(it);
+  if constexpr (sizeof(T) == 4)
+    split_tiles<KL>(sv, m3, g, n_tiles);
+  else if constexpr (KL == 6)
+    mfma6_tiles<T>(sv, m3, g, n_tiles);
+  else
+    mfma_tiles<T, KL>(sv, m3, g, n_tiles);
 }
 
 // ── Launch helpers ──────────────────────────────────────────────────────────
@@ -844,7 +896,33 @@ void launch_batch_by_k(const BatchArgs &a, unsigned n, uint32_t k, uint64_t max_
   check(hipGetLastError(), "hipLaunchKernelGGL(k_dense_batch)");
 }
 
+// Items whose matrix is [Re | Im | Re + Im], on the matrix cores.
+void launch_mfma_batch(const BatchArgs &a, unsigned n, uint8_t precision, uint32_t k,
+                       uint64_t max_combos, hipStream_t s) {
+  const unsigned block = k == 6 && precision == 1 ? kMfma6Block : 256;
+  const uint64_t tiles = max_combos / 16, waves = block / 64;
+  const uint64_t cap = uint64_t(std::max(1, device_props().n_cu)) * 32;
+  const dim3 grid(unsigned(std::min<uint64_t>(cap, (tiles + waves - 1) / waves)), 1, n);
+  if (precision == 0 && k == 5)
+    hipLaunchKernelGGL((k_mfma_batch<float, 5>), grid, dim3(block), 0, s, a);
+  else if (precision == 0)
+    hipLaunchKernelGGL((k_mfma_batch<float, 6>), grid, dim3(block), 0, s, a);
+  else if (k == 4)
+    hipLaunchKernelGGL((k_mfma_batch<double, 4>), grid, dim3(block), 0, s, a);
+  else if (k == 5)
+    hipLaunchKernelGGL((k_mfma_batch<double, 5>), grid, dim3(block), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_mfma_batch<double, 6>), grid, dim3(block), 0, s, a);
+  check(hipGetLastError(), "hipLaunchKernelGGL(k_mfma_batch)");
+}
+
 } // namespace
+
+// f32 k = 4 stays with the direct kernel: its product form is the more exact
+// one, and it holds its 16 amplitudes in registers.
+bool batch_on_matrix_cores(const GatePlan &p, uint32_t n) {
+  return p.d_mat3 && n >= p.k + 4 && (p.precision == 1 || p.k >= 5);
+}
 
 uint32_t plan_family(const GatePlan &plan, uint32_t n_qubits) {
   if (plan.variant == 2)
@@ -874,7 +952,7 @@ void launch_gate(const GatePlan &plan, hipStream_t stream, void *sv, uint32_t n_
 }
 
 void launch_gate_batch(const BatchItem *items, size_t n, uint8_t precision, uint32_t k,
-                       hipStream_t stream) {
+                       bool matrix_cores, hipStream_t stream) {
   for (size_t off = 0; off < n; off += kMaxBatch) {
     const unsigned m = unsigned(std::min<size_t>(kMaxBatch, n - off));
     BatchArgs a{};
@@ -883,7 +961,9 @@ void launch_gate_batch(const BatchItem *items, size_t n, uint8_t precision, uint
       a.it[i] = items[off + i];
       max_combos = std::max(max_combos, items[off + i].combos);
     }
-    if (precision == 0)
+    if (matrix_cores)
+      launch_mfma_batch(a, m, precision, k, max_combos, stream);
+    else if (precision == 0)
       launch_batch_by_k<float>(a, m, k, max_combos, stream);
     else
       launch_batch_by_k<double>(a, m, k, max_combos, stream);

@@ -1,6 +1,5 @@
 // Host-side gfx950 backend over the C ABI; see hip_backend.hpp.
 #include "hip_backend.hpp"
-
 #include "schedule.hpp"
 
 #include <chrono>

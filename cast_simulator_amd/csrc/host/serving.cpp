@@ -2,6 +2,7 @@
 #include "serving.hpp"
 
 #include "fusion.hpp"
+#include "schedule.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -443,10 +444,13 @@ std::vector<ServeResult> Server::run(const std::vector<ServeRequest> &reqs, Serv
     if (!batched) {
       for (Member &m : s.members) {
         const uint32_t n = reqs[m.req].n_qubits;
-        for (void *p : m.plans)
-          throw_if(cast_hip_gate_apply(p, s.stream, m.sv, n, err, kErr), err);
-        for (void *p : m.shadow_plans)
-          throw_if(cast_hip_gate_apply(p, s.stream, m.shadow, n, err, kErr), err);
+        auto queue = [&](const std::vector<void *> &plans, uint64_t sv) {
+          apply_in_passes({plans.begin(), plans.end()}, s.stream, sv, n, [&](uint32_t i) {
+            throw_if(cast_hip_gate_apply(plans[i], s.stream, sv, n, err, kErr), err);
+          });
+        };
+        queue(m.plans, m.sv);
+        queue(m.shadow_plans, m.shadow);
       }
     } else {
       ++n_batches;
