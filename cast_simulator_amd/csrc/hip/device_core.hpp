@@ -120,8 +120,9 @@ __device__ __forceinline__ uint64_t local_delta(uint32_t i, const uint32_t *q) {
 // Dense update of one combo: K amplitudes read from `src`, K written to
 // `dst` (src == dst for in-place), new[r] = sum_c M[r][c] old[c].  NTS:
 // nontemporal stores at f64, which pay only when a wave's stores cover whole
-// 128-byte lines (no target below bit 3); otherwise plain stores.
-template <typename T, int KL, bool NTS = false>
+// 128-byte lines (no target below bit 3); otherwise plain stores.  NTL:
+// nontemporal loads at f64.
+template <typename T, int KL, bool NTS = false, bool NTL = true>
 __device__ __forceinline__ void dense_combo(const typename V2<T>::type *src,
                                             typename V2<T>::type *dst, const T *__restrict__ mat,
                                             uint64_t base, const uint64_t *delta) {
@@ -130,7 +131,7 @@ __device__ __forceinline__ void dense_combo(const typename V2<T>::type *src,
   T vr[K], vi[K];
 #pragma unroll
   for (int i = 0; i < K; ++i) {
-    const VT x = ld_amp(src + base + delta[i]);
+    const VT x = NTL ? ld_amp(src + base + delta[i]) : src[base + delta[i]];
     vr[i] = x.x;
     vi[i] = x.y;
   }

@@ -18,6 +18,7 @@
 //                touch consecutive amplitudes.
 //   k_monomial   <= 1 nonzero per row: touches only rows that differ from the
 //                identity row, so e.g. CZ / CP move 1/4 of the bytes.
+//   k_diagonal   diagonal gates with few entries equal to 1, as a stream.
 //   k_dense_batch, k_mfma_batch  k_dense or the matrix-core tile loops over
 //                many (matrix, statevector) items, item = blockIdx.z
 //                (cast_hip_gate_apply_batch).
@@ -38,6 +39,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <string>
+#include <type_traits>
 
 namespace cast_hip {
 namespace {
@@ -54,7 +56,7 @@ using dev::V2;
 
 // ── Dense: one combo per lane ───────────────────────────────────────────────
 
-template <typename T, int KL, bool NTS>
+template <typename T, int KL, bool NTS, bool NTL>
 __global__ void __launch_bounds__(256) k_dense(T *__restrict__ sv, const T *__restrict__ mat,
                                                GateGeom g) {
   constexpr int K = 1 << KL;
@@ -68,7 +70,7 @@ __global__ void __launch_bounds__(256) k_dense(T *__restrict__ sv, const T *__re
   // per wave through scalar loads instead of being hoisted into VGPRs.
   const uint64_t c = (uint64_t(blockIdx.y) * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
   if (c < g.combos)
-    dev::dense_combo<T, KL, NTS>(amp, amp, mat, combo_base<KL>(c, g.q), delta);
+    dev::dense_combo<T, KL, NTS, NTL>(amp, amp, mat, combo_base<KL>(c, g.q), delta);
 }
 
 // ── Wave tiles with cross-lane exchange of low-order targets ───────────────
@@ -182,6 +184,65 @@ __global__ void __launch_bounds__(256) k_monomial(T *__restrict__ sv, MonoArgs<T
   }
 }
 
+// ── Diagonal gates that change most amplitudes ─────────────────────────────
+//
+// A stream of 16-byte units (one f64 amplitude, two f32 ones), four per thread
+// a block apart, each amplitude multiplied by the diagonal entry (in LDS) that
+// its target bits select.  Blocks in XCD order.  k_monomial reads such a gate
+// as a gather of K rows and holds them all: 26 qubits f64, random phases, k =
+// 1..6: 399, 380, 385, 397, 490, 601 us -> 357 on average (6.0 TB/s); k = 6 at
+// 12 and 24 qubits 32 -> 4.7 and 145 -> 71.
+
+constexpr unsigned kDiagUnits = 4; // per thread
+
+template <typename T, bool NT>
+__global__ void __launch_bounds__(256) k_diagonal(T *__restrict__ sv, const T *__restrict__ mat,
+                                                  GateGeom g, uint64_t n_units) {
+  constexpr int P = sizeof(T) == 4 ? 2 : 1; // amplitudes per unit
+  using Unit = T __attribute__((ext_vector_type(16 / sizeof(T))));
+  using VT = typename NV<T>::type;
+  __shared__ VT entry[64];
+  const uint32_t tid = threadIdx.x, K = 1u << g.k;
+  uint64_t block = uint64_t(blockIdx.y) * gridDim.x + blockIdx.x;
+  if (g.xcd) {
+    const uint64_t blocks = uint64_t(gridDim.x) * gridDim.y;
+    block = (block & 7u) * (blocks >> 3) + (block >> 3);
+  }
+  const uint64_t u0 = block * (256 * kDiagUnits) + tid;
+  Unit *p = reinterpret_cast<Unit *>(sv);
+  Unit x[kDiagUnits];
+#pragma unroll
+  for (unsigned i = 0; i < kDiagUnits; ++i)
+    if (u0 + 256 * i < n_units)
+      x[i] = NT ? __builtin_nontemporal_load(p + u0 + 256 * i) : p[u0 + 256 * i];
+  if (tid < K)
+    entry[tid] = reinterpret_cast<const VT *>(mat)[tid * (K + 1)];
+  __syncthreads();
+#pragma unroll
+  for (unsigned i = 0; i < kDiagUnits; ++i) {
+    const uint64_t u = u0 + 256 * i;
+    if (u >= n_units)
+      continue;
+#pragma unroll
+    for (int h = 0; h < P; ++h) {
+      const uint64_t a = u * P + h;
+      uint32_t row = 0;
+      for (uint32_t b = 0; b < g.k; ++b)
+        row |= (uint32_t(a >> g.q[b]) & 1u) << b;
+      const VT e = entry[row];
+      const T re = x[i][2 * h], im = x[i][2 * h + 1];
+      // an entry of exactly 1 leaves the amplitude as it is
+      const bool keep = e.x == T(1) && e.y == T(0);
+      x[i][2 * h] = keep ? re : e.x * re - e.y * im;
+      x[i][2 * h + 1] = keep ? im : e.x * im + e.y * re;
+    }
+    if constexpr (NT)
+      __builtin_nontemporal_store(x[i], p + u);
+    else
+      p[u] = x[i];
+  }
+}
+
 // ── Matrix cores: complex matvec as three real MFMA products ───────────────
 //
 // For a tile of 16 consecutive combos the update is the complex product
@@ -200,7 +261,7 @@ __global__ void __launch_bounds__(256) k_monomial(T *__restrict__ sv, MonoArgs<T
 using dev::Acc4;
 using dev::mfma16;
 
-template <typename T, int KL>
+template <typename T, int KL, bool NT>
 __device__ __forceinline__ void mfma_tiles(T *__restrict__ sv, const T *__restrict__ m3,
                                            const GateGeom &g, uint64_t n_tiles) {
   constexpr int K = 1 << KL, RB = K / 16, KS = K / 4;
@@ -239,7 +300,7 @@ __device__ __forceinline__ void mfma_tiles(T *__restrict__ sv, const T *__restri
     T br[KS], bi[KS], bs[KS];
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      const VT x = ld_amp(amp + base + din[s]);
+      const VT x = NT ? ld_amp(amp + base + din[s]) : amp[base + din[s]];
       br[s] = x.x;
       bi[s] = x.y;
       bs[s] = x.x + x.y;
@@ -258,16 +319,19 @@ __device__ __forceinline__ void mfma_tiles(T *__restrict__ sv, const T *__restri
         VT o;
         o.x = t1[i] - t2[i];
         o.y = t3[i] - t1[i] - t2[i];
-        st_amp(amp + base + dout[rb][i], o);
+        if constexpr (NT)
+          st_amp(amp + base + dout[rb][i], o);
+        else
+          amp[base + dout[rb][i]] = o;
       }
     }
   }
 }
 
-template <typename T, int KL>
+template <typename T, int KL, bool NT>
 __global__ void __launch_bounds__(256) k_mfma(T *__restrict__ sv, const T *__restrict__ m3,
                                               GateGeom g, uint64_t n_tiles) {
-  mfma_tiles<T, KL>(sv, m3, g, n_tiles);
+  mfma_tiles<T, KL, NT>(sv, m3, g, n_tiles);
 }
 
 // ── Matrix cores, k = 6: real matrices in LDS ──────────────────────────────
@@ -442,7 +506,7 @@ __global__ void __launch_bounds__(KL == 6 && sizeof(T) == 8 ? kMfma6Block : 256)
   else if constexpr (KL == 6)
     mfma6_tiles<T>(sv, m3, g, n_tiles);
   else
-    mfma_tiles<T, KL>(sv, m3, g, n_tiles);
+    mfma_tiles<T, KL, true>(sv, m3, g, n_tiles);
 }
 
 // ── Launch helpers ──────────────────────────────────────────────────────────
@@ -451,6 +515,17 @@ constexpr unsigned kBlock = 256;
 
 bool tile_gauss(const GatePlan &p); // defined with the family rule below
 bool auto_choice(const GatePlan &p);
+
+// Whether the statevector fits the 256 MiB memory-side cache.  f64 gathers
+// (direct and matrix-core kernels) then use plain accesses, above it
+// nontemporal ones.  Measured, us plain / nontemporal, averages over targets:
+// direct k = 1..3 at 22, 23, 24 qubits 18-22 / 21-27, 32-40 / 42-51, 62-80 /
+// 85-101, at 25 and 26 qubits 189-205 / 181-243 and 380-410 / 360-467 (less
+// with the wave tiles); matrix cores k = 4 at 24 qubits 82-84 / 98-106, at 25
+// 200-213 / 188-202; k = 5 at 24 qubits 100-109 / 112-124.
+bool cached_state(const GateGeom &g, size_t scalar) {
+  return (g.combos << g.k) * 2 * scalar <= uint64_t(256) << 20;
+}
 
 unsigned grid_for(uint64_t combos) {
   static const unsigned cap = [] {
@@ -484,13 +559,42 @@ void launch_dense_t(const GatePlan &p, hipStream_t s, void *sv, const GateGeom &
   uint32_t qmin = 64;
   for (uint32_t b = 0; b < g.k; ++b)
     qmin = std::min(qmin, g.q[b]);
-  if (sizeof(T) == 8 && qmin >= 3)
-    hipLaunchKernelGGL((k_dense<T, KL, true>), full_grid(g.combos), dim3(kBlock), 0, s,
-                       static_cast<T *>(sv), static_cast<const T *>(p.d_mat), g);
+  auto go = [&](auto stores, auto loads) {
+    hipLaunchKernelGGL((k_dense<T, KL, decltype(stores)::value, decltype(loads)::value>),
+                       full_grid(g.combos), dim3(kBlock), 0, s, static_cast<T *>(sv),
+                       static_cast<const T *>(p.d_mat), g);
+  };
+  if (sizeof(T) == 4 || cached_state(g, sizeof(T)))
+    go(std::false_type{}, std::false_type{});
+  else if (qmin >= 3)
+    go(std::true_type{}, std::true_type{});
   else
-    hipLaunchKernelGGL((k_dense<T, KL, false>), full_grid(g.combos), dim3(kBlock), 0, s,
-                       static_cast<T *>(sv), static_cast<const T *>(p.d_mat), g);
+    go(std::false_type{}, std::true_type{});
   check(hipGetLastError(), "hipLaunchKernelGGL(k_dense)");
+}
+
+// Diagonal gates with three quarters of their entries or more other than 1;
+// with fewer, k_monomial skips what it need not touch.
+bool streamed_diagonal(const GatePlan &p) {
+  for (uint32_t j = 0; j < p.n_active; ++j)
+    if (p.act_row[j] != p.act_col[j])
+      return false;
+  return 4 * p.n_active >= 3u << p.k;
+}
+
+template <typename T> void launch_diagonal(const GatePlan &p, hipStream_t s, void *sv, GateGeom g) {
+  const uint64_t units = (g.combos << g.k) * 2 * sizeof(T) / 16;
+  const uint64_t per_block = 256 * kDiagUnits;
+  const dim3 grid = full_grid((units + per_block - 1) / per_block * kBlock);
+  const uint64_t blocks = uint64_t(grid.x) * grid.y;
+  g.xcd = blocks >= 8 && blocks % 8 == 0;
+  if (cached_state(g, sizeof(T)))
+    hipLaunchKernelGGL((k_diagonal<T, false>), grid, dim3(256), 0, s, static_cast<T *>(sv),
+                       static_cast<const T *>(p.d_mat), g, units);
+  else
+    hipLaunchKernelGGL((k_diagonal<T, true>), grid, dim3(256), 0, s, static_cast<T *>(sv),
+                       static_cast<const T *>(p.d_mat), g, units);
+  check(hipGetLastError(), "hipLaunchKernelGGL(k_diagonal)");
 }
 
 template <typename T, int KL>
@@ -575,8 +679,12 @@ void launch_mfma_t(const GatePlan &p, hipStream_t s, void *sv, const GateGeom &g
   // +0.5-0.7 % on the 30-qubit headline circuit's k = 5 gates.
   const unsigned grid = mfma_order(p, unsigned(std::max<uint64_t>(1, std::min(need, cap))), tiles,
                                    g, sizeof(T) == 8);
-  hipLaunchKernelGGL((k_mfma<T, KL>), dim3(grid), dim3(kBlock), 0, s, static_cast<T *>(sv),
-                     static_cast<const T *>(p.d_mat3), g, tiles);
+  if (sizeof(T) == 4 || cached_state(g, sizeof(T)))
+    hipLaunchKernelGGL((k_mfma<T, KL, false>), dim3(grid), dim3(kBlock), 0, s,
+                       static_cast<T *>(sv), static_cast<const T *>(p.d_mat3), g, tiles);
+  else
+    hipLaunchKernelGGL((k_mfma<T, KL, true>), dim3(grid), dim3(kBlock), 0, s, static_cast<T *>(sv),
+                       static_cast<const T *>(p.d_mat3), g, tiles);
   check(hipGetLastError(), "hipLaunchKernelGGL(k_mfma)");
 }
 
@@ -744,13 +852,16 @@ TileGeom tile_geom(const GatePlan &p, uint32_t n, uint32_t *n_low) {
   if (p.flags & CAST_HIP_FLAG_TILE_SWIZZLE)
     tg.swz = std::min<uint32_t>(10, n - 6 - p.k);
   // blocks = n_tiles / 4 (4 waves per block, one tile each), a power of two.
-  // Automatically chosen tiles (no order flag) use the XCD order too: on the
-  // config-3 circuit's gates forced to wave tiles it streamed 5504 -> 6360
-  // GB/s (k = 3) and 5524 -> 6316 (k = 4) at 33 qubits f64, 5507 -> 6474
-  // (k = 3) at 34 qubits f32, and +1.4 to +5.7 % on the 30-qubit headline
-  // circuit's k = 3, 4 gates; the per-gate autotuner still tries all three.
+  // Automatically chosen tiles (no order flag) use the XCD order too from
+  // states of 4 GiB on: on the config-3 circuit's gates forced to wave tiles
+  // it streamed 5504 -> 6360 GB/s (k = 3) and 5524 -> 6316 (k = 4) at 33
+  // qubits f64, 5507 -> 6474 (k = 3) at 34 qubits f32, and +1.4 to +5.7 % on
+  // the 30-qubit headline circuit's k = 3, 4 gates.  Below it costs: f64 k =
+  // 1..4 launch order / XCD at 24 qubits 82-95 / 86-102 us, at 26 339-397 /
+  // 349-404, at 28 1393-1517 / 1352-1542; the per-gate autotuner tries all.
+  const bool large = (uint64_t(2 * scalar_bytes(p.precision)) << n) >= uint64_t(4) << 30;
   const bool xcd = (p.flags & CAST_HIP_FLAG_TILE_XCD) ||
-                   (auto_choice(p) && !(p.flags & CAST_HIP_FLAG_TILE_SWIZZLE));
+                   (auto_choice(p) && large && !(p.flags & CAST_HIP_FLAG_TILE_SWIZZLE));
   if (xcd && tg.n_tiles >= 32)
     tg.xcd_bits = n - 6 - p.k - 2;
   *n_low = L;
@@ -791,6 +902,40 @@ uint32_t count_low(const GatePlan &p) {
   return n_low;
 }
 
+// Automatic choice for k <= 5 on a statevector of at most 256 MiB (f64 24
+// qubits, f32 25), where the gather kernels read from the caches.  us per
+// gate, averages over random targets, L = targets below bit 6:
+//   k <= 3       the direct kernel: f32 k = 3 at 22, 24, 25 qubits 9-12, 34-42,
+//                70-103 against 10-21, 42-68, 87-131 on wave tiles; f64 k = 3
+//                at 18, 22, 24 qubits 4, 19-26, 66-80 against 4-6.5, 22-25,
+//                88-93;
+//   f64 k = 4    matrix cores up to 16 MiB (4-10 against 7-14 on tiles) and
+//                from 128 MiB on (43, 82 against 45-59, 91-109); between, wave
+//                tiles for L <= 2 (11.3-12.5, 23-27 against 17.6, 28);
+//   f32 k = 4    matrix cores up to 4 MiB (4.7 against 5.6-11); above, tiles for
+//                L = 0 (6.3-45 against 7.4-45 direct), else the direct kernel
+//                (22, 24 qubits 14.5-18, 45-60 against tiles 16-24, 51-75), at
+//                128 MiB and more matrix cores for L >= 3 (53, 98 against 60, 115);
+//   f64 k = 5    wave tiles at 32 and 64 MiB for L <= 1 (26, 31 against 29, 54
+//                on the matrix cores) and at 128 MiB (63 against 66);
+//   else         matrix cores.
+uint32_t automatic_cached(const GatePlan &p, uint32_t n, uint32_t n_low, bool tile_ok,
+                          bool mfma_ok) {
+  const uint64_t mib = (uint64_t(2 * scalar_bytes(p.precision)) << n) >> 20;
+  if (p.k <= 3)
+    return 1;
+  uint32_t v = 4;
+  if (p.precision == 1 && p.k == 4)
+    v = mib > 16 && mib < 128 && n_low <= 2 ? 3 : 4;
+  else if (p.k == 4)
+    v = mib <= 4 ? 4 : n_low == 0 ? 3 : mib >= 128 && n_low >= 3 ? 4 : 1;
+  else if (p.precision == 1)
+    v = mib > 16 && mib <= 128 && n_low <= 1 ? 3 : 4;
+  if (v == 4 && !mfma_ok)
+    v = 3;
+  return v == 3 && !tile_ok ? 1 : v;
+}
+
 uint32_t dense_family(const GatePlan &p, uint32_t n) {
   const bool tile_ok = p.k <= 5 && n >= p.k + 6;
   const bool mfma_ok = p.d_mat3 != nullptr && n >= p.k + 4;
@@ -798,11 +943,15 @@ uint32_t dense_family(const GatePlan &p, uint32_t n) {
   uint32_t v = p.variant;
   if (auto_choice(p)) {
     // Automatic choice, from measurements on MI355X (the per-gate autotuner
-    // refines it where it runs):
-    //  * wave tiles stream full rows and win up to 3 low-order targets for
-    //    k <= 4; beyond that the exchanged register groups cost more than
-    //    the matrix-core kernel's 16-combo tiles;
-    //  * k = 5: the matrix cores (f32: bf16 split products) for any
+    // refines it where it runs); L = targets below bit 6, us per gate:
+    //  * states that the 256 MiB memory-side cache holds: automatic_cached;
+    //  * wave tiles stream full rows and win up to 2 low-order targets for
+    //    k <= 4, and 3 for k = 3; beyond that the exchanged register groups
+    //    cost more than the matrix-core kernel's 16-combo tiles (k = 4, L =
+    //    3, tiles / matrix cores: f64 25 qubits 220 / 188, 28 1588 / 1539;
+    //    f32 26 qubits 286 / 277, 29 2221 / 1951; at f64 30 qubits and more
+    //    tiles up to L = 3);
+    //  * otherwise k = 5: the matrix cores (f32: bf16 split products) for any
     //    targets: on the config-3 circuit's k = 5 gates without autotuning,
     //    wave tiles ran 4979 GB/s at 33 qubits f64 against 6089 on the
     //    matrix cores, and 4849 at 34 qubits f32 against 5214; on the
@@ -810,9 +959,13 @@ uint32_t dense_family(const GatePlan &p, uint32_t n) {
     //    most k = 5 gates (19 of 29 at f64, 21 of 29 at f32);
     //  * k = 6: only the matrix-core kernel keeps its operands out of
     //    scratch memory.
-    if (p.k >= 5 && mfma_ok)
+    const uint32_t tile_low = p.k < 4 || (p.precision == 1 && n >= 30) ? 3 : 2;
+    const uint64_t bytes = uint64_t(2 * scalar_bytes(p.precision)) << n;
+    if (p.k <= 5 && bytes <= uint64_t(256) << 20)
+      v = automatic_cached(p, n, n_low, tile_ok, mfma_ok);
+    else if (p.k >= 5 && mfma_ok)
       v = 4;
-    else if (tile_ok && n_low <= 3)
+    else if (tile_ok && n_low <= tile_low)
       v = 3;
     else if (mfma_ok)
       v = 4;
@@ -839,6 +992,11 @@ bool tile_gauss(const GatePlan &p) {
 template <typename T>
 void launch_by_k(const GatePlan &p, hipStream_t s, void *sv, const GateGeom &g) {
   const bool mono = p.variant == 2;
+  // k = 1 in the caches: two rows a lane are no gather (f64 22 qubits 19 us
+  // against 21, f32 24 qubits 36 against 38).
+  if (mono && g.combos << g.k >= 64 && (p.k > 1 || !cached_state(g, sizeof(T))) &&
+      streamed_diagonal(p))
+    return launch_diagonal<T>(p, s, sv, g);
   if (!mono) {
     const uint32_t n = p.k + uint32_t(63 - __builtin_clzll(g.combos));
     const uint32_t fam = dense_family(p, n);
