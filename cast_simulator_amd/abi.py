@@ -180,6 +180,7 @@ _SIGS = {
     "cast_hip_expect_zz": (
         _i, [_u64, _u32, _u8, C.POINTER(_u32), _sz, C.POINTER(C.c_double), _vp, _err, _sz]),
     "cast_hip_traj_run": (_i, [C.POINTER(TrajLaunch), _vp, _err, _sz]),
+    "cast_hip_traj_run_steps": (_i, [C.POINTER(TrajLaunch), C.POINTER(C.c_uint32), _vp, _err, _sz]),
     "cast_hip_inner_product": (
         _i, [_u64, _u8, _u64, _u8, _u32, C.POINTER(C.c_double), _vp, _err, _sz]),
     "cast_hip_inner_product_scratch_bytes": (_sz, []),
@@ -462,6 +463,14 @@ def dm_populations(sv: int, n_physical: int, precision: int,
 
 def traj_run(args: TrajLaunch, stream: int | None = None) -> None:
     _call("cast_hip_traj_run", C.byref(args), stream)
+
+
+def traj_run_steps(args: TrajLaunch, n_gates, stream: int | None = None) -> None:
+    """`n_gates`: the lengths of the tasks along the order, not increasing."""
+    if len(n_gates) != args.n_tasks:
+        raise ValueError("one length per task")
+    _call("cast_hip_traj_run_steps", C.byref(args), (C.c_uint32 * max(1, len(n_gates)))(*n_gates),
+          stream)
 
 
 def version() -> str:

@@ -742,7 +742,16 @@ int cast_hip_traj_run(const cast_hip_traj_launch_t *args, void *stream, char *er
   return guard(err, len, [&] {
     if (!args)
       throw Error("null trajectory launch descriptor");
-    launch_traj(*args, static_cast<hipStream_t>(stream));
+    launch_traj(*args, nullptr, static_cast<hipStream_t>(stream));
+  });
+}
+
+int cast_hip_traj_run_steps(const cast_hip_traj_launch_t *args, const uint32_t *n_gates,
+                            void *stream, char *err, size_t len) {
+  return guard(err, len, [&] {
+    if (!args || !n_gates)
+      throw Error("null trajectory launch descriptor or task lengths");
+    launch_traj(*args, n_gates, static_cast<hipStream_t>(stream));
   });
 }
 

@@ -183,6 +183,8 @@ void cache_release(void *p, size_t bytes);
 
 // Persistent batched-trajectory launch (traj_kernels.hip); validates the
 // descriptor and enqueues the counter reset and the kernel.
-void launch_traj(const cast_hip_traj_launch_t &args, hipStream_t stream);
+// `n_gates` (host, nonincreasing along the order): the task lengths, for a
+// launch per gate step; null for the persistent launch.
+void launch_traj(const cast_hip_traj_launch_t &args, const uint32_t *n_gates, hipStream_t stream);
 
 } // namespace cast_hip

@@ -1,6 +1,8 @@
-// Persistent batched-trajectory kernel for gfx950.
+// Batched-trajectory kernels for gfx950: a persistent launch (k_traj) for many
+// tasks or small statevectors, a launch per gate step (k_traj_step,
+// k_traj_finish) for few tasks on larger ones.
 //
-// One workgroup owns one statevector slot and takes whole tasks from a
+// k_traj: one workgroup owns one statevector slot and takes whole tasks from a
 // global counter until the list is exhausted; no workgroup ever waits on
 // another, so any grid size drains.  A task is (checkpoint, gate list): the
 // first applied gate reads the checkpoint statevector and writes the slot,
@@ -22,6 +24,7 @@
 #include "common.hpp"
 #include "device_core.hpp"
 
+#include <algorithm>
 #include <string>
 
 namespace cast_hip {
@@ -36,6 +39,10 @@ constexpr int kMaxPairs = 32;
 constexpr int kMaxBlock = 512;
 constexpr int kMaxWaves = kMaxBlock / 64;
 constexpr uint32_t kMaxTrajGateQubits = 6; // 4 at f64
+// Workgroups a step is cut into, eight rounds of the CUs: 188 tasks of 20
+// qubits at f32 (3708 gates) take 20.2 ms in 512, 17.8 in 1024, 17.0 in 2048
+// and in 4096 workgroups of 512 threads (256 threads: 0.5 to 2 ms more).
+constexpr uint32_t kStepGroups = 2048;
 
 // Layouts the host bindings rely on (no padding surprises across compilers).
 static_assert(sizeof(cast_hip_traj_gate_t) == 12, "cast_hip_traj_gate_t layout");
@@ -60,11 +67,17 @@ __global__ void k_fill_u32(uint32_t *__restrict__ p, uint32_t n, uint32_t v) {
 
 using dev::opaque_u32;
 
-// One gate over the whole statevector by the workgroup, wave tiles.  q[] are
+// The calling wave's place among the waves that share a gate: those of the
+// workgroup that owns the statevector, or of all its parts.
+struct Share {
+  uint32_t wave, n_waves;
+};
+
+// One gate over the waves' share of the statevector, wave tiles.  q[] are
 // the ascending targets, of which exactly L are below 6.
 template <typename T, int KL, int L>
 __device__ __forceinline__ void wg_tile_gate(const T *src, T *dst, const T *__restrict__ mat,
-                                             const uint32_t *q, uint32_t n) {
+                                             const uint32_t *q, uint32_t n, Share sh) {
   constexpr int U = KL >= 4 ? 1 : (16 >> KL); // tiles per step
   // Tile layout: register bit j < L -> the j-th non-target position >= 6,
   // register bit j >= L -> target q[j] (targets >= 6); the tile index is
@@ -92,7 +105,7 @@ __device__ __forceinline__ void wg_tile_gate(const T *src, T *dst, const T *__re
     im &= im - 1;
   }
 
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
+  const uint32_t lane = threadIdx.x & 63u, wave = sh.wave, n_waves = sh.n_waves;
   const uint64_t n_tiles = uint64_t(1) << (n - 6 - KL);
   auto tile_ptr = [&](uint64_t tile) {
 #pragma unroll
@@ -128,7 +141,7 @@ __device__ __forceinline__ void wg_tile_gate(const T *src, T *dst, const T *__re
 // Small statevectors (n < k + 6): one combo per thread.
 template <typename T, int KL>
 __device__ __forceinline__ void wg_dense_gate(const T *src, T *dst, const T *__restrict__ mat,
-                                              const uint32_t *q, uint32_t n) {
+                                              const uint32_t *q, uint32_t n, Share sh) {
   constexpr int K = 1 << KL;
   using VT = typename V2<T>::type;
   uint64_t delta[K];
@@ -136,7 +149,7 @@ __device__ __forceinline__ void wg_dense_gate(const T *src, T *dst, const T *__r
   for (int i = 0; i < K; ++i)
     delta[i] = local_delta<KL>(uint32_t(i), q);
   const uint64_t combos = uint64_t(1) << (n - KL);
-  for (uint64_t c = threadIdx.x; c < combos; c += blockDim.x) {
+  for (uint64_t c = sh.wave * 64u + (threadIdx.x & 63u); c < combos; c += sh.n_waves * 64u) {
     const T *m = mat + opaque_u32(0);
     const VT *in = reinterpret_cast<const VT *>(src);
     VT *out = reinterpret_cast<VT *>(dst);
@@ -181,14 +194,14 @@ __device__ __forceinline__ void wg_dense_gate(const T *src, T *dst, const T *__r
 template <int KL>
 __device__ __forceinline__ void wg_mfma_gate(const float *src, float *dst,
                                              const float *__restrict__ m3, const uint32_t *q,
-                                             uint32_t n) {
+                                             uint32_t n, Share sh) {
   constexpr int K = 1 << KL, RB = K / 16, KS = K / 4, U = 2;
   using VT = typename V2<float>::type;
   using AV = dev::Acc4<float>::type;
   const VT *in = reinterpret_cast<const VT *>(src);
   VT *out = reinterpret_cast<VT *>(dst);
   const uint32_t lane = threadIdx.x & 63u, j = lane >> 4, col = lane & 15u;
-  const uint32_t wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
+  const uint32_t wave = sh.wave, n_waves = sh.n_waves;
   float a[3][RB][KS];
 #pragma unroll
   for (int m = 0; m < 3; ++m)
@@ -256,7 +269,7 @@ __device__ __forceinline__ void wg_mfma_gate(const float *src, float *dst,
 // overwriting operands still in use.
 __device__ __forceinline__ void wg_mfma6_gate(const float *src, float *dst,
                                               const float *__restrict__ m3, const uint32_t *q,
-                                              uint32_t n, float *a_lds) {
+                                              uint32_t n, Share sh, float *a_lds) {
   constexpr int KL = 6, K = 64, RB = 4, KS = 16;
   using VT = typename V2<float>::type;
   using AV = dev::Acc4<float>::type;
@@ -268,7 +281,7 @@ __device__ __forceinline__ void wg_mfma6_gate(const float *src, float *dst,
   const VT *in = reinterpret_cast<const VT *>(src);
   VT *out = reinterpret_cast<VT *>(dst);
   const uint32_t lane = threadIdx.x & 63u, j = lane >> 4, col = lane & 15u;
-  const uint32_t wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
+  const uint32_t wave = sh.wave, n_waves = sh.n_waves;
   uint64_t din[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s)
@@ -320,14 +333,15 @@ __device__ __forceinline__ void wg_mfma6_gate(const float *src, float *dst,
 template <int KL>
 __device__ __forceinline__ void wg_split_gate(const float *src, float *dst,
                                               const float *__restrict__ m3, const uint32_t *q,
-                                              uint32_t n, dev::bf16x8_t *a_lds) {
+                                              uint32_t n, Share sh,
+                                              dev::bf16x8_t *a_lds) {
   // k = 5: two tiles per step, so that each lane keeps 16 loads in flight as
   // at k = 6 (one workgroup streams the whole statevector).
   constexpr int U = KL == 5 ? 2 : 1;
   dev::split_stage<KL>(m3, a_lds);
   __syncthreads();
   const dev::SplitLane<KL> sl(q);
-  const uint32_t wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
+  const uint32_t wave = sh.wave, n_waves = sh.n_waves;
   // n >= KL + 5 for k = 5 (checked by the caller), so n_tiles is a multiple of U
   const uint64_t n_tiles = uint64_t(1) << (n - KL - 4);
   for (uint64_t t = uint64_t(wave) * U; t < n_tiles; t += uint64_t(n_waves) * U)
@@ -337,35 +351,35 @@ __device__ __forceinline__ void wg_split_gate(const float *src, float *dst,
 
 template <typename T, int KL>
 __device__ __forceinline__ void wg_gate_k(const T *src, T *dst, const T *__restrict__ mat,
-                                          const uint32_t *q, uint32_t n) {
+                                          const uint32_t *q, uint32_t n, Share sh) {
   if (n < uint32_t(KL) + 6)
-    return wg_dense_gate<T, KL>(src, dst, mat, q, n);
+    return wg_dense_gate<T, KL>(src, dst, mat, q, n, sh);
   uint32_t n_low = 0;
 #pragma unroll
   for (int b = 0; b < KL; ++b)
     n_low += q[b] < 6;
   if constexpr (KL == 5) { // f32 only: matrix cores, any targets
     if constexpr (sizeof(T) == 4)
-      wg_mfma_gate<KL>(src, dst, mat, q, n);
+      wg_mfma_gate<KL>(src, dst, mat, q, n, sh);
   } else {
     switch (n_low) {
     case 0:
-      return wg_tile_gate<T, KL, 0>(src, dst, mat, q, n);
+      return wg_tile_gate<T, KL, 0>(src, dst, mat, q, n, sh);
     case 1:
       if constexpr (KL >= 1)
-        return wg_tile_gate<T, KL, 1>(src, dst, mat, q, n);
+        return wg_tile_gate<T, KL, 1>(src, dst, mat, q, n, sh);
       break;
     case 2:
       if constexpr (KL >= 2)
-        return wg_tile_gate<T, KL, 2>(src, dst, mat, q, n);
+        return wg_tile_gate<T, KL, 2>(src, dst, mat, q, n, sh);
       break;
     case 3:
       if constexpr (KL == 3 || KL == 4)
-        return wg_tile_gate<T, KL, 3>(src, dst, mat, q, n);
+        return wg_tile_gate<T, KL, 3>(src, dst, mat, q, n, sh);
       break;
     case 4:
       if constexpr (KL == 4)
-        return wg_tile_gate<T, KL, 4>(src, dst, mat, q, n);
+        return wg_tile_gate<T, KL, 4>(src, dst, mat, q, n, sh);
       break;
     default:
       break;
@@ -461,6 +475,108 @@ __device__ __forceinline__ void wg_observe(const T *sv, uint32_t n, uint32_t n_p
   __syncthreads();
 }
 
+// One gate of a task by the waves `sh` describes; false for a descriptor that
+// is out of range (nothing is done then).  `gate_lds` holds kGateLdsBytes<T>.
+template <typename T>
+__device__ __forceinline__ bool wg_gate(const cast_hip_traj_gate_t &d, const T *src, T *dst,
+                                        const T *__restrict__ matrices, const TrajScalars &a,
+                                        uint32_t n, Share sh, unsigned char *gate_lds) {
+  const bool f32_products = a.flags & CAST_HIP_TRAJ_FLAG_MFMA_F32;
+  // The descriptor is the same for the whole workgroup; readfirstlane
+  // states that, so geometry and matrix address live in SGPRs.
+  const uint32_t k = __builtin_amdgcn_readfirstlane(d.k);
+  const uint32_t moff = __builtin_amdgcn_readfirstlane(d.matrix_offset);
+  uint32_t q[kMaxTrajGateQubits];
+  bool ok = k >= 1 && k <= (sizeof(T) == 4 ? kMaxTrajGateQubits : 4u);
+  ok = ok && (k < 6 || n >= 12); // the k = 6 path needs 64 tiles of 16 combos
+#pragma unroll
+  for (uint32_t b = 0; b < kMaxTrajGateQubits; ++b) {
+    q[b] = __builtin_amdgcn_readfirstlane(d.q[b]);
+    if (b < k)
+      ok = ok && q[b] < n && (b == 0 || q[b] > q[b - 1]);
+  }
+  // k = 4, 5 entries hold three real K x K matrices: 3 K^2 / 2 complex slots.
+  const uint64_t entries = k >= 4 ? uint64_t(3) << (2 * k - 1) : (uint64_t(1) << (2 * k));
+  ok = ok && uint64_t(moff) + entries <= a.n_matrix_elems;
+  if (!ok)
+    return false;
+  const T *mat = matrices + 2 * uint64_t(moff);
+  switch (k) {
+  case 1:
+    wg_gate_k<T, 1>(src, dst, mat, q, n, sh);
+    break;
+  case 2:
+    wg_gate_k<T, 2>(src, dst, mat, q, n, sh);
+    break;
+  case 3:
+    wg_gate_k<T, 3>(src, dst, mat, q, n, sh);
+    break;
+  case 4:
+    wg_gate_k<T, 4>(src, dst, mat, q, n, sh);
+    break;
+  case 5: // f32 only (checked above)
+    if constexpr (sizeof(T) == 4) {
+      if (f32_products || n < 11)
+        wg_gate_k<T, 5>(src, dst, mat, q, n, sh);
+      else
+        wg_split_gate<5>(src, dst, mat, q, n, sh, reinterpret_cast<dev::bf16x8_t *>(gate_lds));
+    }
+    break;
+  default: // k = 6, f32 only, n >= 12 (checked above)
+    if constexpr (sizeof(T) == 4) {
+      if (f32_products)
+        wg_mfma6_gate(src, dst, mat, q, n, sh, reinterpret_cast<float *>(gate_lds));
+      else
+        wg_split_gate<6>(src, dst, mat, q, n, sh, reinterpret_cast<dev::bf16x8_t *>(gate_lds));
+    }
+    break;
+  }
+  return true;
+}
+
+// The task order[t] of the launch, checked; false (and the error flag set, by
+// every lane: no lane-dependent branch) when it is out of range.
+__device__ __forceinline__ bool fetch_task(const cast_hip_traj_task_t *tasks,
+                                           const uint32_t *order, uint32_t t, uint32_t *work,
+                                           const TrajScalars &a, uint32_t &ti,
+                                           cast_hip_traj_task_t &task) {
+  ti = __builtin_amdgcn_readfirstlane(order[t]);
+  bool ok = ti < a.n_tasks;
+  if (ok) {
+    const cast_hip_traj_task_t tk = tasks[ti];
+    task.first_gate = __builtin_amdgcn_readfirstlane(tk.first_gate);
+    task.n_gates = __builtin_amdgcn_readfirstlane(tk.n_gates);
+    task.checkpoint = __builtin_amdgcn_readfirstlane(tk.checkpoint);
+    ok = task.checkpoint < a.n_checkpoints && task.first_gate <= a.n_gates &&
+         task.n_gates <= a.n_gates - task.first_gate;
+  }
+  if (!ok)
+    atomicOr(&work[1], 1u);
+  return ok;
+}
+
+// The workgroup's copy of a final state.
+template <typename T> __device__ __forceinline__ void wg_dump(const T *cur, T *to, uint64_t len) {
+  using VT = typename V2<T>::type;
+  const VT *src = reinterpret_cast<const VT *>(cur);
+  VT *dst = reinterpret_cast<VT *>(to);
+  for (uint64_t i0 = threadIdx.x; i0 < len; i0 += uint64_t(blockDim.x) * 8) {
+    VT x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const uint64_t i = i0 + uint64_t(u) * blockDim.x;
+      if (i < len)
+        x[u] = src[i];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const uint64_t i = i0 + uint64_t(u) * blockDim.x;
+      if (i < len)
+        dst[i] = x[u];
+    }
+  }
+}
+
 // Built for OCC waves per SIMD (second launch-bound argument): 2 allows 256
 // VGPRs (no spills, one 512-thread workgroup per CU), 4 allows 128 (spills,
 // but two workgroups per CU keep twice the loads in flight).
@@ -474,7 +590,7 @@ __global__ void __launch_bounds__(kMaxBlock, OCC)
   __shared__ uint32_t s_pairs[2 * kMaxPairs];
   __shared__ double red[kMaxWaves * (1 + kMaxPairs)];
   __shared__ __align__(16) unsigned char gate_lds[kGateLdsBytes<T>];
-  const bool f32_products = a.flags & CAST_HIP_TRAJ_FLAG_MFMA_F32;
+  const Share sh{threadIdx.x >> 6, blockDim.x >> 6};
   if (threadIdx.x < 2 * a.n_pairs)
     s_pairs[threadIdx.x] = a.pairs[threadIdx.x];
   for (;;) {
@@ -493,74 +609,15 @@ __global__ void __launch_bounds__(kMaxBlock, OCC)
     const uint32_t n = opaque_u32(a.n_qubits);
     const uint64_t len = uint64_t(1) << n;
     T *slot = slots + 2 * len * blockIdx.x;
-    const uint32_t ti = __builtin_amdgcn_readfirstlane(order[t]);
-    bool task_ok = ti < a.n_tasks;
+    uint32_t ti;
     cast_hip_traj_task_t task{};
-    if (task_ok) {
-      const cast_hip_traj_task_t tk = tasks[ti];
-      task.first_gate = __builtin_amdgcn_readfirstlane(tk.first_gate);
-      task.n_gates = __builtin_amdgcn_readfirstlane(tk.n_gates);
-      task.checkpoint = __builtin_amdgcn_readfirstlane(tk.checkpoint);
-      task_ok = task.checkpoint < a.n_checkpoints && task.first_gate <= a.n_gates &&
-                task.n_gates <= a.n_gates - task.first_gate;
-    }
-    if (!task_ok) {
-      atomicOr(&work[1], 1u); // every lane: no lane-dependent branch here
+    if (!fetch_task(tasks, order, t, work, a, ti, task))
       continue;
-    }
     const T *cur = checkpoints + 2 * len * task.checkpoint; // state the next gate reads
     for (uint32_t g = 0; g < task.n_gates; ++g) {
-      // The descriptor is the same for the whole workgroup; readfirstlane
-      // states that, so geometry and matrix address live in SGPRs.
-      const cast_hip_traj_gate_t d = gates[task.first_gate + g];
-      const uint32_t k = __builtin_amdgcn_readfirstlane(d.k);
-      const uint32_t moff = __builtin_amdgcn_readfirstlane(d.matrix_offset);
-      uint32_t q[kMaxTrajGateQubits];
-      bool ok = k >= 1 && k <= (sizeof(T) == 4 ? kMaxTrajGateQubits : 4u);
-      ok = ok && (k < 6 || n >= 12); // the k = 6 path needs 64 tiles of 16 combos
-#pragma unroll
-      for (uint32_t b = 0; b < kMaxTrajGateQubits; ++b) {
-        q[b] = __builtin_amdgcn_readfirstlane(d.q[b]);
-        if (b < k)
-          ok = ok && q[b] < n && (b == 0 || q[b] > q[b - 1]);
-      }
-      // k = 4, 5 entries hold three real K x K matrices: 3 K^2 / 2 complex slots.
-      const uint64_t slots = k >= 4 ? uint64_t(3) << (2 * k - 1) : (uint64_t(1) << (2 * k));
-      ok = ok && uint64_t(moff) + slots <= a.n_matrix_elems;
-      if (!ok) {
+      if (!wg_gate<T>(gates[task.first_gate + g], cur, slot, matrices, a, n, sh, gate_lds)) {
         atomicOr(&work[1], 1u);
         continue;
-      }
-      const T *mat = matrices + 2 * uint64_t(moff);
-      switch (k) {
-      case 1:
-        wg_gate_k<T, 1>(cur, slot, mat, q, n);
-        break;
-      case 2:
-        wg_gate_k<T, 2>(cur, slot, mat, q, n);
-        break;
-      case 3:
-        wg_gate_k<T, 3>(cur, slot, mat, q, n);
-        break;
-      case 4:
-        wg_gate_k<T, 4>(cur, slot, mat, q, n);
-        break;
-      case 5: // f32 only (checked above)
-        if constexpr (sizeof(T) == 4) {
-          if (f32_products || n < 11)
-            wg_gate_k<T, 5>(cur, slot, mat, q, n);
-          else
-            wg_split_gate<5>(cur, slot, mat, q, n, reinterpret_cast<dev::bf16x8_t *>(gate_lds));
-        }
-        break;
-      default: // k = 6, f32 only, n >= 12 (checked above)
-        if constexpr (sizeof(T) == 4) {
-          if (f32_products)
-            wg_mfma6_gate(cur, slot, mat, q, n, reinterpret_cast<float *>(gate_lds));
-          else
-            wg_split_gate<6>(cur, slot, mat, q, n, reinterpret_cast<dev::bf16x8_t *>(gate_lds));
-        }
-        break;
       }
       cur = slot;
       __syncthreads();
@@ -568,27 +625,69 @@ __global__ void __launch_bounds__(kMaxBlock, OCC)
     wg_observe<T>(cur, n, a.n_pairs, a.log2_block, s_pairs, out + uint64_t(ti) * (1 + a.n_pairs),
                   red);
     if (dump) {
-      using VT = typename V2<T>::type;
-      const VT *src = reinterpret_cast<const VT *>(cur);
-      VT *dst = reinterpret_cast<VT *>(dump + 2 * len * ti);
-      for (uint64_t i0 = threadIdx.x; i0 < len; i0 += uint64_t(blockDim.x) * 8) {
-        VT x[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const uint64_t i = i0 + uint64_t(u) * blockDim.x;
-          if (i < len)
-            x[u] = src[i];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const uint64_t i = i0 + uint64_t(u) * blockDim.x;
-          if (i < len)
-            dst[i] = x[u];
-        }
-      }
+      wg_dump<T>(cur, dump + 2 * len * ti, len);
       __syncthreads();
     }
   }
+}
+
+// Gate g of the tasks order[first ...), every statevector shared by `parts`
+// workgroups; slot t belongs to the task order[first + t].  A workgroup that
+// owns a statevector (k_traj) is held to what one CU can do, and the launch to
+// its longest task: 188 tasks of 20 qubits and up to 40 gates at f32 took
+// 29.4 ms with 0.73 ms per gate on each of 188 CUs.  With a launch per step all
+// CUs share the tasks that are left: 17.0 ms (4.6 us per gate of 16.8 MB moved,
+// 3.7 TB/s, k = 5 and 6 bound by the split products), 32 tasks 23.6 -> 4.4 ms.
+// Each amplitude goes through the same operations as in k_traj.
+template <typename T, int OCC>
+__global__ void __launch_bounds__(kMaxBlock, OCC)
+    k_traj_step(const cast_hip_traj_task_t *__restrict__ tasks, const uint32_t *__restrict__ order,
+                const cast_hip_traj_gate_t *__restrict__ gates, const T *__restrict__ matrices,
+                const T *__restrict__ checkpoints, T *__restrict__ slots,
+                uint32_t *__restrict__ work, TrajScalars a, uint32_t first, uint32_t g,
+                uint32_t parts) {
+  __shared__ __align__(16) unsigned char gate_lds[kGateLdsBytes<T>];
+  const uint32_t slot_i = blockIdx.x / parts, part = blockIdx.x % parts;
+  uint32_t ti;
+  cast_hip_traj_task_t task{};
+  if (!fetch_task(tasks, order, first + slot_i, work, a, ti, task) || g >= task.n_gates)
+    return;
+  const uint32_t n = opaque_u32(a.n_qubits);
+  const uint64_t len = uint64_t(1) << n;
+  T *slot = slots + 2 * len * slot_i;
+  const T *src = g == 0 ? checkpoints + 2 * len * task.checkpoint : slot;
+  const uint32_t waves = blockDim.x >> 6;
+  const Share sh{part * waves + (threadIdx.x >> 6), parts * waves};
+  if (!wg_gate<T>(gates[task.first_gate + g], src, slot, matrices, a, n, sh, gate_lds))
+    atomicOr(&work[1], 1u);
+}
+
+// Sums and dump of the tasks order[first ...), one workgroup each, after
+// their last step.  A task with more gates than `n_steps` is an error.
+template <typename T>
+__global__ void __launch_bounds__(kMaxBlock, 2)
+    k_traj_finish(const cast_hip_traj_task_t *__restrict__ tasks,
+                  const uint32_t *__restrict__ order, const T *__restrict__ checkpoints,
+                  const T *__restrict__ slots, double *__restrict__ out, T *__restrict__ dump,
+                  uint32_t *__restrict__ work, TrajScalars a, uint32_t first, uint32_t n_steps) {
+  __shared__ uint32_t s_pairs[2 * kMaxPairs];
+  __shared__ double red[kMaxWaves * (1 + kMaxPairs)];
+  if (threadIdx.x < 2 * a.n_pairs)
+    s_pairs[threadIdx.x] = a.pairs[threadIdx.x];
+  __syncthreads();
+  uint32_t ti;
+  cast_hip_traj_task_t task{};
+  if (!fetch_task(tasks, order, first + blockIdx.x, work, a, ti, task))
+    return;
+  if (task.n_gates > n_steps)
+    atomicOr(&work[1], 1u);
+  const uint64_t len = uint64_t(1) << a.n_qubits;
+  const T *cur = task.n_gates == 0 ? checkpoints + 2 * len * task.checkpoint
+                                   : slots + 2 * len * blockIdx.x;
+  wg_observe<T>(cur, a.n_qubits, a.n_pairs, a.log2_block, s_pairs,
+                out + uint64_t(ti) * (1 + a.n_pairs), red);
+  if (dump)
+    wg_dump<T>(cur, dump + 2 * len * ti, len);
 }
 
 template <typename T, int OCC>
@@ -604,9 +703,42 @@ void launch_traj_t(const cast_hip_traj_launch_t &L, const TrajScalars &a, hipStr
   check(hipGetLastError(), "hipLaunchKernelGGL(k_traj)");
 }
 
+template <typename T, int OCC>
+void launch_steps_t(const cast_hip_traj_launch_t &L, const TrajScalars &a, const uint32_t *n_gates,
+                    hipStream_t s) {
+  const auto *tasks = reinterpret_cast<const cast_hip_traj_task_t *>(L.tasks);
+  const auto *order = reinterpret_cast<const uint32_t *>(L.order);
+  const auto *gates = reinterpret_cast<const cast_hip_traj_gate_t *>(L.gates);
+  const T *mats = reinterpret_cast<const T *>(L.matrices);
+  const T *ckpt = reinterpret_cast<const T *>(L.checkpoints);
+  T *slots = reinterpret_cast<T *>(L.slots);
+  uint32_t *work = reinterpret_cast<uint32_t *>(L.work);
+  const uint32_t waves = L.block / 64;
+  // At most as many parts as leave every wave a k = 6 tile of 2^10 amplitudes.
+  const uint32_t most =
+      L.n_qubits > 10 ? std::max(1u, (1u << std::min(L.n_qubits - 10, 20u)) / waves) : 1u;
+  for (uint32_t first = 0; first < L.n_tasks; first += L.n_slots) {
+    const uint32_t here = std::min(L.n_slots, L.n_tasks - first);
+    uint32_t active = here;
+    const uint32_t n_steps = n_gates[first];
+    for (uint32_t g = 0; g < n_steps; ++g) {
+      while (n_gates[first + active - 1] <= g)
+        --active;
+      const uint32_t parts = std::min(most, std::max(1u, kStepGroups / active));
+      hipLaunchKernelGGL((k_traj_step<T, OCC>), dim3(active * parts), dim3(L.block), 0, s, tasks,
+                         order, gates, mats, ckpt, slots, work, a, first, g, parts);
+      check(hipGetLastError(), "hipLaunchKernelGGL(k_traj_step)");
+    }
+    hipLaunchKernelGGL((k_traj_finish<T>), dim3(here), dim3(L.block), 0, s, tasks, order, ckpt,
+                       slots, reinterpret_cast<double *>(L.out), reinterpret_cast<T *>(L.dump),
+                       work, a, first, n_steps);
+    check(hipGetLastError(), "hipLaunchKernelGGL(k_traj_finish)");
+  }
+}
+
 } // namespace
 
-void launch_traj(const cast_hip_traj_launch_t &L, hipStream_t stream) {
+void launch_traj(const cast_hip_traj_launch_t &L, const uint32_t *n_gates, hipStream_t stream) {
   if (L.precision > 1)
     throw Error("trajectory launch: precision must be 0 (F32) or 1 (F64)");
   if (L.n_qubits < 1 || L.n_qubits > 34)
@@ -651,6 +783,18 @@ void launch_traj(const cast_hip_traj_launch_t &L, hipStream_t stream) {
   for (uint32_t j = 0; j < 2 * L.n_pairs; ++j)
     a.pairs[j] = L.pairs[j];
   const bool occ4 = L.waves_per_simd == 4;
+  if (n_gates) {
+    for (uint32_t t = 1; t < L.n_tasks; ++t)
+      if (n_gates[t] > n_gates[t - 1])
+        throw Error("trajectory launch: task lengths must not increase along the order");
+    if (L.precision == 0)
+      occ4 ? launch_steps_t<float, 4>(L, a, n_gates, stream)
+           : launch_steps_t<float, 2>(L, a, n_gates, stream);
+    else
+      occ4 ? launch_steps_t<double, 4>(L, a, n_gates, stream)
+           : launch_steps_t<double, 2>(L, a, n_gates, stream);
+    return;
+  }
   if (L.precision == 0)
     occ4 ? launch_traj_t<float, 4>(L, a, stream) : launch_traj_t<float, 2>(L, a, stream);
   else

@@ -4,6 +4,8 @@
 #include "fusion.hpp"
 
 #include <algorithm>
+#include <functional>
+#include <queue>
 #include <atomic>
 #include <chrono>
 #include <cmath>
@@ -580,6 +582,36 @@ TrajectoryPlan TrajectoryEngine::plan(const std::vector<TrajectorySample> &sampl
   return P;
 }
 
+// Whether a launch per gate step (every CU on the tasks that are left) beats
+// the persistent launch (a workgroup per slot, whole tasks).  The latter takes
+// as long as its busiest slot; `load` below is that against gates shared evenly
+// by the CUs.  Steps read and write every state from memory, where a slot of
+// the persistent launch may stay in the caches, and cost a launch each.
+// Measured, persistent -> steps: 20 qubits f32 load 18 23.6 -> 4.4 ms, 2.8
+// 29.7 -> 17.1, 1.2 51.5 -> 53.8; 18 qubits f32 load 3.0 6.2 -> 4.2, 1.1
+// 11.9 -> 13.6; 16 qubits f32 load 20 1.5 -> 0.7, 3.5 1.9 -> 1.6, 1.2 3.0 -> 4.8;
+// 14 qubits f32 load 23 0.42 -> 0.53, f64 load 4.1 0.92 -> 0.93.
+static bool steps_pay(const std::vector<uint32_t> &lengths, uint32_t n_slots, uint32_t n_cu,
+                      size_t sv_bytes) {
+  if (sv_bytes < (size_t(512) << 10))
+    return false;
+  // The slots take the tasks in order, each when it is free.
+  std::priority_queue<uint64_t, std::vector<uint64_t>, std::greater<uint64_t>> busy;
+  uint64_t total = 0, longest = 0;
+  for (uint32_t g : lengths) {
+    uint64_t end = g;
+    if (busy.size() == n_slots) {
+      end += busy.top();
+      busy.pop();
+    }
+    busy.push(end);
+    longest = std::max(longest, end);
+    total += g;
+  }
+  const double load = total ? double(longest) * double(n_cu) / double(total) : 0.0;
+  return load >= (sv_bytes < (size_t(2) << 20) ? 3.0 : 2.0);
+}
+
 TrajectoryRun TrajectoryEngine::run(const std::vector<TrajectorySample> &samples,
                                     const TrajectoryTuning &tn, bool dump) {
   const double t_start = now_s();
@@ -692,6 +724,11 @@ TrajectoryRun TrajectoryEngine::run(const std::vector<TrajectorySample> &samples
   L.waves_per_simd = tn.waves_per_simd;
   L.flags = tn.mfma_f32 ? CAST_HIP_TRAJ_FLAG_MFMA_F32 : 0u;
 
+  std::vector<uint32_t> lengths;
+  lengths.reserve(order.size());
+  for (uint32_t t : order)
+    lengths.push_back(tasks[t].n_gates);
+
   void *e0 = cast_hip_event_create(err, kErr);
   if (!e0)
     throw Error(err);
@@ -703,7 +740,9 @@ TrajectoryRun TrajectoryEngine::run(const std::vector<TrajectorySample> &samples
   float ms = 0.f;
   int rc = cast_hip_event_record(e0, s, err, kErr);
   if (rc == 0)
-    rc = cast_hip_traj_run(&L, s, err, kErr);
+    rc = steps_pay(lengths, uint32_t(n_slots), std::max(1u, info.n_cu), svb)
+             ? cast_hip_traj_run_steps(&L, lengths.data(), s, err, kErr)
+             : cast_hip_traj_run(&L, s, err, kErr);
   if (rc == 0)
     rc = cast_hip_event_record(e1, s, err, kErr);
   if (rc == 0)

@@ -421,6 +421,14 @@ typedef struct cast_hip_traj_launch_t {
 int cast_hip_traj_run(const cast_hip_traj_launch_t *args, void *stream, char *err_buf,
                       size_t err_buf_len);
 
+/* The same work with one launch per gate step instead of one workgroup per
+ * task: rounds of n_slots tasks of the order, step g applying gate g of every
+ * task that has one, each statevector shared by many workgroups.  n_gates[t]
+ * (host, not increasing) is the length of the task order[t].  A task whose
+ * device length exceeds the first n_gates of its round sets the error flag. */
+int cast_hip_traj_run_steps(const cast_hip_traj_launch_t *args, const uint32_t *n_gates,
+                            void *stream, char *err_buf, size_t err_buf_len);
+
 /* Library version string (static storage). */
 const char *cast_hip_version(void);
 
