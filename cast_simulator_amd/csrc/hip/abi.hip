@@ -192,7 +192,7 @@ GatePlan *build_plan(const cast_hip_kernel_gen_spec_t *spec, const cast_complex6
   const size_t KK = K * K, sb = fp32 ? 4 : 8;
   const bool real3 = variant != CAST_HIP_VARIANT_MONOMIAL && n_qubits >= 4;
   const size_t mat3_at = 2 * KK * sb, op_at = mat3_at + (real3 ? 3 * KK * sb : 0);
-  const bool op = real3 && n_qubits <= 5;
+  const bool op = real3 && (n_qubits <= 5 || fp32);
   plan->block_bytes =
       op_at + (op ? group_operand_bytes(uint32_t(n_qubits), plan->precision) : 0);
   std::vector<unsigned char> host(plan->block_bytes);

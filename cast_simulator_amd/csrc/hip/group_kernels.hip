@@ -20,7 +20,7 @@
 //                 rows by scalar loads, each row used for 2^(R-k) combos;
 //   k = 4, f64 5  three real products on the matrix cores, 16 combos per
 //                 MFMA tile, operands laid out by lane when the plan is built;
-//   f32 k = 5     bf16 split products as in the single-gate kernel;
+//   f32 k = 5, 6  bf16 split products as in the single-gate kernel;
 //   monomial      diagonal gates (any k) multiply in place, permutations
 //                 (k <= 4) move amplitudes between LDS slots.
 //
@@ -351,6 +351,93 @@ __device__ __forceinline__ void split_gate5(unsigned char *lds, const GroupGate 
   }
 }
 
+// f32 k = 6 likewise.  Its 48 KiB of operands neither fit the registers nor,
+// beside two tiles, the LDS: they stream from the caches in 12 steps (row
+// block, split), each step's 4 KiB requested D steps before its products.
+// Bound by the products (41 us at 25 qubits at the chip's bf16 rate): it adds
+// about 55 us to a pass there, where its own pass takes 130-155.  25 qubits,
+// 37 gates of which 13 have k = 6: 2829 us with those alone, 2515 in groups.
+template <int R>
+__device__ __forceinline__ void split_gate6(unsigned char *lds, const GroupGate &g, uint32_t tid) {
+  constexpr int KL = 6, LB = R + 2 - KL, NT = 1 << LB, D = R == 5 ? 2 : 1, STEPS = 12;
+  const uint32_t lane = tid & 63u, col = lane & 15u, j = lane >> 4, wave = tid >> 6;
+  const bf16x8_t *op = static_cast<const bf16x8_t *>(g.mat) + lane;
+  bf16x8_t a[D + 1][2][2]; // ring of steps, [Re, Im][k step]
+  auto fetch = [&](int step) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        a[step % (D + 1)][m][ks] =
+            op[dev::SplitOperands<6>::at(m, 2 - step % 3, step / 3, ks)];
+  };
+#pragma unroll
+  for (int s = 0; s < D; ++s)
+    fetch(s);
+  const uint32_t base = select_offsets<4>(g, KL, col) ^ select_offsets<7 - R>(g, R + 6, wave);
+  const uint32_t in = base ^ select_offsets<2>(g, 3, j);
+  const uint32_t out = base ^ select_offsets<2>(g, 2, j);
+  __syncthreads();
+  bf16x8_t br[NT][3][2], bi[NT][3][2];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const dev::f2v x =
+            lds_get<float>(lds, in ^ select_offsets<LB>(g, KL + 4, uint32_t(t)) ^
+                                    select_offsets<3>(g, 0, uint32_t(e)) ^
+                                    select_offsets<1>(g, 5, uint32_t(ks)));
+        const Split3 sr = split3(x.x), si = split3(x.y);
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+          br[t][s][ks][e] = sr.p[s];
+          bi[t][s][ks][e] = si.p[s];
+        }
+      }
+  f32x4_t t1[NT], t2[NT], t3[NT];
+#pragma unroll
+  for (int step = 0; step < STEPS; ++step) {
+    const int sa = 2 - step % 3, rb = step / 3;
+    if (step + D < STEPS)
+      fetch(step + D);
+    __builtin_amdgcn_sched_barrier(0);
+    if (sa == 2)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        t1[t] = t2[t] = t3[t] = {0, 0, 0, 0};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const bf16x8_t ar = a[step % (D + 1)][0][ks], ai = a[step % (D + 1)][1][ks];
+#pragma unroll
+      for (int sb = 2 - sa; sb >= 0; --sb)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          t1[t] = dev::mfma_bf16(ar, br[t][sb][ks], t1[t]);
+          t3[t] = dev::mfma_bf16(ar, bi[t][sb][ks], t3[t]);
+          t2[t] = dev::mfma_bf16(ai, bi[t][sb][ks], t2[t]);
+          t3[t] = dev::mfma_bf16(ai, br[t][sb][ks], t3[t]);
+        }
+    }
+    if (sa == 0)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          dev::f2v o;
+          o.x = t1[t][i] - t2[t][i];
+          o.y = t3[t][i];
+          lds_put<float>(lds,
+                         out ^ select_offsets<LB>(g, KL + 4, uint32_t(t)) ^
+                             select_offsets<2>(g, 0, uint32_t(i)) ^
+                             select_offsets<2>(g, 4, uint32_t(rb)),
+                         o);
+        }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 // v times an entry (re, im).
 template <typename T>
 __device__ __forceinline__ typename NV<T>::type times(typename NV<T>::type v, T re, T im) {
@@ -513,11 +600,15 @@ __global__ void __launch_bounds__(1 << (12 + Shape<T>::P - R), R == 3 + Shape<T>
       case 4:
         mfma_gate<R, 4>(lds, g, tid, T(0));
         break;
-      default:
+      case 5:
         if constexpr (sizeof(T) == 8)
           mfma_gate<R, 5>(lds, g, tid, T(0));
         else
           split_gate5<R>(lds, g, tid);
+        break;
+      default: // f32 only
+        if constexpr (sizeof(T) == 4)
+          split_gate6<R>(lds, g, tid);
         break;
       }
     }
@@ -556,7 +647,7 @@ bool can_join(const GatePlan &p, uint32_t n) {
     return false;
   if (p.variant == 2)
     return is_diagonal(p) || p.k <= 4;
-  return p.k <= 5;
+  return p.k <= (p.precision == 0 ? 6u : 5u);
 }
 
 // LDS byte offset of local index bit `p` (see the file comment).
@@ -582,11 +673,13 @@ void launch_k_group(dim3 grid, dim3 block, size_t lds, hipStream_t stream, void 
 //        Re M;
 //   f32 k = 4: x = matrix, four entries of row l % 16 from column 4 (l / 16)
 //        on, matrices Re M, Im M, Re M + Im M;
-//   f32 k = 5: the bf16 fragments of dev::split_stage.
+//   f32 k = 5, 6: the bf16 fragments of dev::split_stage.
 size_t group_operand_bytes(uint32_t k, uint8_t precision) {
   const size_t K = size_t(1) << k;
   if (precision == 0)
-    return k == 4 ? 3 * K * K * sizeof(float) : dev::SplitOperands<5>::kFragments * 16;
+    return k == 4   ? 3 * K * K * sizeof(float)
+           : k == 5 ? dev::SplitOperands<5>::kFragments * 16
+                    : dev::SplitOperands<6>::kFragments * 16;
   return 3 * K * K * sizeof(double);
 }
 
@@ -634,18 +727,23 @@ void group_operands(const double *m, uint32_t k, uint8_t precision, void *out) {
         }
   } else {
     uint16_t *h = static_cast<uint16_t *>(out);
+    const uint32_t n_ks = K / 32;
     for (uint32_t x = 0; x < 2; ++x)
-      for (uint32_t rb = 0; rb < 2; ++rb)
-        for (uint32_t l = 0; l < 64; ++l)
-          for (uint32_t e = 0; e < 8; ++e) {
-            const uint32_t r = 16 * rb + (l & 15u), c = 8 * (l >> 4) + e;
-            float rest = float(x == 0 ? re(r, c) : im(r, c));
-            for (uint32_t s = 0; s < 3; ++s) {
-              const uint16_t b = to_bf16(rest);
-              h[(size_t(dev::SplitOperands<5>::at(int(x), int(s), int(rb), 0)) + l) * 8 + e] = b;
-              rest -= from_bf16(b);
+      for (uint32_t rb = 0; rb < RB; ++rb)
+        for (uint32_t ks = 0; ks < n_ks; ++ks)
+          for (uint32_t l = 0; l < 64; ++l)
+            for (uint32_t e = 0; e < 8; ++e) {
+              const uint32_t r = 16 * rb + (l & 15u), c = 32 * ks + 8 * (l >> 4) + e;
+              float rest = float(x == 0 ? re(r, c) : im(r, c));
+              for (uint32_t s = 0; s < 3; ++s) {
+                const uint16_t b = to_bf16(rest);
+                const size_t at = size_t(
+                    k == 5 ? dev::SplitOperands<5>::at(int(x), int(s), int(rb), int(ks))
+                           : dev::SplitOperands<6>::at(int(x), int(s), int(rb), int(ks)));
+                h[(at + l) * 8 + e] = b;
+                rest -= from_bf16(b);
+              }
             }
-          }
   }
 }
 
