@@ -127,6 +127,16 @@ class GroupInfo(C.Structure):
     ]
 
 
+class GroupItem(C.Structure):
+    _fields_ = [
+        ("plans", C.POINTER(C.c_void_p)),
+        ("n_plans", C.c_size_t),
+        ("sv", C.c_uint64),
+        ("round", C.c_uint32),
+        ("reserved", C.c_uint32),
+    ]
+
+
 _vp, _sz, _u8, _u32, _u64, _i = C.c_void_p, C.c_size_t, C.c_uint8, C.c_uint32, C.c_uint64, C.c_int
 _err = C.c_char_p
 _SIGS = {
@@ -177,6 +187,9 @@ _SIGS = {
         _i, [C.POINTER(_vp), C.POINTER(_u64), C.POINTER(_u32), _sz, _vp, _err, _sz]),
     "cast_hip_gate_group_info": (_i, [_vp, _u32, C.POINTER(GroupInfo), _err, _sz]),
     "cast_hip_gate_apply_group": (_i, [C.POINTER(_vp), _sz, _vp, _u64, _u32, _err, _sz]),
+    "cast_hip_group_batch_scratch_bytes": (_sz, [_sz, _sz]),
+    "cast_hip_gate_apply_group_batch": (
+        _i, [C.POINTER(GroupItem), _sz, _u32, _u64, _vp, _err, _sz]),
     "cast_hip_expect_zz": (
         _i, [_u64, _u32, _u8, C.POINTER(_u32), _sz, C.POINTER(C.c_double), _vp, _err, _sz]),
     "cast_hip_traj_run": (_i, [C.POINTER(TrajLaunch), _vp, _err, _sz]),
@@ -325,6 +338,19 @@ def gate_group_info(plan: int, n_qubits: int) -> GroupInfo:
 def gate_apply_group(plans, dptr: int, n_qubits: int, stream: int | None = None) -> None:
     n = len(plans)
     _call("cast_hip_gate_apply_group", (_vp * n)(*plans), n, stream, dptr, n_qubits)
+
+
+def group_batch_scratch_bytes(n_groups: int, n_plans: int) -> int:
+    return int(lib().cast_hip_group_batch_scratch_bytes(n_groups, n_plans))
+
+
+def gate_apply_group_batch(items, n_qubits: int, scratch: int, stream: int | None = None) -> None:
+    """items: (plans, statevector pointer, round) triples, rounds not decreasing."""
+    lists = [(_vp * max(1, len(p)))(*p) for p, _, _ in items]
+    arr = (GroupItem * max(1, len(items)))()
+    for a, lst, (p, sv, rnd) in zip(arr, lists, items):
+        a.plans, a.n_plans, a.sv, a.round = C.cast(lst, C.POINTER(_vp)), len(p), sv, rnd
+    _call("cast_hip_gate_apply_group_batch", arr, len(items), n_qubits, scratch, stream)
 
 
 def expect_zz(dptr: int, n_qubits: int, precision: int, pairs, stream: int | None = None):

@@ -718,6 +718,37 @@ int cast_hip_gate_apply_group(const void *const *plans, size_t n_plans, void *st
   });
 }
 
+size_t cast_hip_group_batch_scratch_bytes(size_t n_groups, size_t n_plans) {
+  return group_batch_bytes(n_groups, n_plans);
+}
+
+int cast_hip_gate_apply_group_batch(const cast_hip_group_item_t *items, size_t n_items,
+                                    uint32_t sv_n_qubits, uint64_t scratch, void *stream,
+                                    char *err, size_t len) {
+  return guard(err, len, [&] {
+    if (n_items == 0)
+      return;
+    if (!items || !scratch)
+      throw Error("null group list or scratch");
+    std::vector<GroupItem> list(n_items);
+    for (size_t i = 0; i < n_items; ++i) {
+      const std::string at = " at group " + std::to_string(i);
+      if (!items[i].plans || items[i].n_plans == 0)
+        throw Error("no plans" + at);
+      for (size_t g = 0; g < items[i].n_plans; ++g)
+        if (!items[i].plans[g])
+          throw Error("null plan" + at);
+      if (!items[i].sv)
+        throw Error("null statevector pointer" + at);
+      check_aligned(items[i].sv);
+      list[i] = {reinterpret_cast<const GatePlan *const *>(items[i].plans), items[i].n_plans,
+                 reinterpret_cast<void *>(items[i].sv), items[i].round};
+    }
+    launch_group_batch(list.data(), n_items, sv_n_qubits, reinterpret_cast<void *>(scratch),
+                       static_cast<hipStream_t>(stream));
+  });
+}
+
 int cast_hip_expect_zz(uint64_t sv_dptr, uint32_t sv_n_qubits, uint8_t precision,
                        const uint32_t *pairs, size_t n_pairs, double *out, void *stream,
                        char *err, size_t len) {

@@ -137,6 +137,18 @@ void group_operands(const double *m, uint32_t k, uint8_t precision, void *out);
 // Enqueues the gates, in order, as one pass over the statevector.
 void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stream, void *sv,
                   uint32_t n_qubits);
+// Groups on several n-qubit statevectors, one launch per round (rounds do not
+// decrease along the list); `table` is group_batch_bytes of device memory that
+// is free on `stream`.
+struct GroupItem {
+  const GatePlan *const *plans;
+  size_t n_plans; // 1 or more
+  void *sv;
+  uint32_t round;
+};
+size_t group_batch_bytes(size_t n_groups, size_t n_plans);
+void launch_group_batch(const GroupItem *items, size_t n_items, uint32_t n, void *table,
+                        hipStream_t stream);
 
 // Statevector utility kernels implemented in sv_kernels.hip.
 void launch_sv_zero(void *sv, size_t n_elements, uint8_t precision, hipStream_t stream);

@@ -42,6 +42,7 @@
 #include <algorithm>
 #include <cstring>
 #include <string>
+#include <vector>
 
 namespace cast_hip {
 namespace {
@@ -68,12 +69,19 @@ struct GroupGate {
   uint32_t kind;
 };
 
-struct GroupArgs {
+// A group on one statevector.
+struct GroupHead {
   uint32_t n_gates;
   uint32_t thread_bits;  // log2(threads per workgroup)
   uint32_t m;            // tile qubits
   uint32_t xcd_bits;     // 0, or log2(tiles): tiles in XCD order
   uint8_t s[16];         // tile qubits, ascending
+  void *sv;
+  uint64_t first;        // of its gates, in a table of several groups
+};
+
+struct GroupArgs {
+  GroupHead h;
   GroupGate g[kMaxGroupGates];
 };
 
@@ -89,8 +97,14 @@ template <> struct Shape<float> {
 typedef float Unit __attribute__((ext_vector_type(4))); // 16 bytes
 
 template <typename T> using Const = const __attribute__((address_space(4))) T *;
+template <typename T> using Global = const __attribute__((address_space(1))) T *;
+// A pointer read from a table, known to be one to global memory.
+template <typename T> __device__ __forceinline__ Global<T> global_ptr(const void *p) {
+  return (Global<T>)(reinterpret_cast<uintptr_t>(p));
+}
 
-__device__ __forceinline__ uint32_t offset_of(const GroupGate &g, int b) {
+// G: a GroupGate in the kernel's arguments or in constant memory.
+template <typename G> __device__ __forceinline__ uint32_t offset_of(G &g, int b) {
   return (g.off2[b >> 1] >> (16 * (b & 1))) & 0xffffu;
 }
 
@@ -104,8 +118,8 @@ __device__ __forceinline__ void lds_put(unsigned char *lds, uint32_t a, typename
 }
 
 // XOR of the offsets first .. first + N - 1 selected by the bits of v.
-template <int N>
-__device__ __forceinline__ uint32_t select_offsets(const GroupGate &g, int first, uint32_t v) {
+template <int N, typename G>
+__device__ __forceinline__ uint32_t select_offsets(G &g, int first, uint32_t v) {
   uint32_t a = 0;
 #pragma unroll
   for (int b = 0; b < N; ++b)
@@ -116,8 +130,8 @@ __device__ __forceinline__ uint32_t select_offsets(const GroupGate &g, int first
 // Dense gate on k <= 3 targets.  Offsets: k targets, R - k combos of the
 // thread, then the thread index bits.  Row r + 1 of the matrix is requested
 // (scalar loads) before row r is used.
-template <typename T, int R, int KL>
-__device__ __forceinline__ void small_gate(unsigned char *lds, const GroupGate &g, uint32_t tid) {
+template <typename T, int R, int KL, typename G>
+__device__ __forceinline__ void small_gate(unsigned char *lds, G &g, uint32_t tid) {
   constexpr int K = 1 << KL, U = 1 << (R - KL);
   using V = typename NV<T>::type;
   typedef T Row __attribute__((ext_vector_type(2 * K)));
@@ -172,8 +186,8 @@ __device__ __forceinline__ void small_gate(unsigned char *lds, const GroupGate &
 // instruction (an f64 MFMA keeps the vector unit busy too).  f32: t1 = Re M
 // vr, t2 = Im M vi, t3 = (Re M + Im M)(vr + vi), Re = t1 - t2, Im = t3 - t1 -
 // t2, the form of the single-gate kernels.
-template <int R, int KL>
-__device__ __forceinline__ void mfma_gate(unsigned char *lds, const GroupGate &g, uint32_t tid,
+template <int R, int KL, typename G>
+__device__ __forceinline__ void mfma_gate(unsigned char *lds, G &g, uint32_t tid,
                                           double) {
   constexpr int K = 1 << KL, RB = K / 16, KS = K / 4, LB = R + 2 - KL, NT = 1 << LB;
   using AV = dev::Acc4<double>::type;
@@ -182,7 +196,7 @@ __device__ __forceinline__ void mfma_gate(unsigned char *lds, const GroupGate &g
   const uint32_t base = select_offsets<4>(g, KL, col) ^ select_offsets<6 - R>(g, R + 6, wave);
   const uint32_t in = base ^ select_offsets<2>(g, KL - 2, j);
   const uint32_t out = base ^ select_offsets<2>(g, 0, j);
-  const Pair *op = static_cast<const Pair *>(g.mat) + lane;
+  const Global<Pair> op = global_ptr<Pair>(g.mat) + lane;
   Pair a[3][KS / 2];
   auto load_rows = [&](int rb) {
 #pragma unroll
@@ -243,8 +257,8 @@ __device__ __forceinline__ void mfma_gate(unsigned char *lds, const GroupGate &g
   }
 }
 
-template <int R, int KL>
-__device__ __forceinline__ void mfma_gate(unsigned char *lds, const GroupGate &g, uint32_t tid,
+template <int R, int KL, typename G>
+__device__ __forceinline__ void mfma_gate(unsigned char *lds, G &g, uint32_t tid,
                                           float) {
   static_assert(KL == 4, "f32 k = 5 has the split products");
   constexpr int LB = R + 2 - KL, NT = 1 << LB;
@@ -252,7 +266,7 @@ __device__ __forceinline__ void mfma_gate(unsigned char *lds, const GroupGate &g
   const uint32_t lane = tid & 63u, col = lane & 15u, j = lane >> 4, wave = tid >> 6;
   const uint32_t base = select_offsets<4>(g, KL, col) ^ select_offsets<7 - R>(g, R + 6, wave);
   const uint32_t in = base ^ select_offsets<2>(g, 2, j); // rows and columns alike
-  const Unit *op = static_cast<const Unit *>(g.mat) + lane;
+  const Global<Unit> op = global_ptr<Unit>(g.mat) + lane;
   const Unit ar = op[0], ai = op[64], as = op[128];
   __syncthreads();
   dev::f2v x[NT][4];
@@ -286,11 +300,11 @@ __device__ __forceinline__ void mfma_gate(unsigned char *lds, const GroupGate &g
 // f32 k = 5 as bf16 split products (the partial products and their order are
 // those of dev::split_tile); the operands are the splits of Re M and Im M.
 // Offsets as in mfma_gate.
-template <int R>
-__device__ __forceinline__ void split_gate5(unsigned char *lds, const GroupGate &g, uint32_t tid) {
+template <int R, typename G>
+__device__ __forceinline__ void split_gate5(unsigned char *lds, G &g, uint32_t tid) {
   constexpr int KL = 5, LB = R + 2 - KL, NT = 1 << LB;
   const uint32_t lane = tid & 63u, col = lane & 15u, j = lane >> 4, wave = tid >> 6;
-  const bf16x8_t *op = static_cast<const bf16x8_t *>(g.mat) + lane;
+  const Global<bf16x8_t> op = global_ptr<bf16x8_t>(g.mat) + lane;
   bf16x8_t a[2][3][2]; // [Re, Im][split][row block]
 #pragma unroll
   for (int m = 0; m < 2; ++m)
@@ -357,11 +371,11 @@ __device__ __forceinline__ void split_gate5(unsigned char *lds, const GroupGate 
 // Bound by the products (41 us at 25 qubits at the chip's bf16 rate): it adds
 // about 55 us to a pass there, where its own pass takes 130-155.  25 qubits,
 // 37 gates of which 13 have k = 6: 2829 us with those alone, 2515 in groups.
-template <int R>
-__device__ __forceinline__ void split_gate6(unsigned char *lds, const GroupGate &g, uint32_t tid) {
+template <int R, typename G>
+__device__ __forceinline__ void split_gate6(unsigned char *lds, G &g, uint32_t tid) {
   constexpr int KL = 6, LB = R + 2 - KL, NT = 1 << LB, D = R == 5 ? 2 : 1, STEPS = 12;
   const uint32_t lane = tid & 63u, col = lane & 15u, j = lane >> 4, wave = tid >> 6;
-  const bf16x8_t *op = static_cast<const bf16x8_t *>(g.mat) + lane;
+  const Global<bf16x8_t> op = global_ptr<bf16x8_t>(g.mat) + lane;
   bf16x8_t a[D + 1][2][2]; // ring of steps, [Re, Im][k step]
   auto fetch = [&](int step) {
 #pragma unroll
@@ -451,8 +465,8 @@ __device__ __forceinline__ typename NV<T>::type times(typename NV<T>::type v, T 
 // entry (r, col(r)) times amplitude col(r).  Rows equal to the identity's
 // touch nothing.  Offsets as in small_gate; the mask of the other rows is in
 // the upper half of off2[6].
-template <typename T, int R, int KL>
-__device__ __forceinline__ void monomial_gate(unsigned char *lds, const GroupGate &g,
+template <typename T, int R, int KL, typename G>
+__device__ __forceinline__ void monomial_gate(unsigned char *lds, G &g,
                                               uint32_t tid) {
   constexpr int K = 1 << KL, U = 1 << (R - KL);
   using V = typename NV<T>::type;
@@ -484,14 +498,14 @@ __device__ __forceinline__ void monomial_gate(unsigned char *lds, const GroupGat
 // Monomial gate on more than R targets: the targets from the R-th on are the
 // lowest thread index bits, so a wave holds whole combos and reads them
 // before it writes.
-template <typename T, int R>
-__device__ __forceinline__ void wide_monomial_gate(unsigned char *lds, const GroupGate &g,
+template <typename T, int R, typename G>
+__device__ __forceinline__ void wide_monomial_gate(unsigned char *lds, G &g,
                                                    uint32_t tid, uint32_t k, bool diagonal) {
   constexpr int N = 1 << R;
   using V = typename NV<T>::type;
   const uint32_t base = select_offsets<12 - R + Shape<T>::P>(g, R, tid);
   const uint32_t hi = tid & ((1u << (k - R)) - 1);
-  const V *mat = static_cast<const V *>(g.mat);
+  const Global<V> mat = global_ptr<V>(g.mat);
   __syncthreads();
   V x[N], e[N];
 #pragma unroll
@@ -518,7 +532,8 @@ template <typename T, int RU> struct TileUnits {
   uint64_t reg[RU]; // global unit offsets of the bits of i
   uint32_t lds_t, thread_bits;
 
-  __device__ __forceinline__ TileUnits(T *sv, const GroupArgs &a, uint64_t tile, uint32_t tid) {
+  template <typename H>
+  __device__ __forceinline__ TileUnits(T *sv, H &a, uint64_t tile, uint32_t tid) {
     for (uint32_t b = 0; b < a.m; ++b)
       tile = insert_zero(tile, a.s[b]);
 #pragma unroll
@@ -547,10 +562,8 @@ template <typename T, int RU> struct TileUnits {
 // R amplitude bits per thread.  The gate functions begin with the barrier that
 // orders them after the previous gate; what they need from global memory is
 // requested before it.
-template <typename T, int R>
-__global__ void __launch_bounds__(1 << (12 + Shape<T>::P - R), R == 3 + Shape<T>::P ? 4 : 2)
-    k_group(T *__restrict__ sv, GroupArgs a) {
-  extern __shared__ __align__(16) unsigned char lds[];
+template <typename T, int R, typename H, typename G>
+__device__ __forceinline__ void run_group(T *sv, H &a, G *gates, unsigned char *lds) {
   using Units = TileUnits<T, R - Shape<T>::P>;
   const uint32_t tid = threadIdx.x;
   uint64_t tile = blockIdx.x;
@@ -567,7 +580,7 @@ __global__ void __launch_bounds__(1 << (12 + Shape<T>::P - R), R == 3 + Shape<T>
       *reinterpret_cast<Unit *>(lds + t.local(i)) = x[i];
   }
   for (uint32_t gi = 0; gi < a.n_gates; ++gi) {
-    const GroupGate &g = a.g[gi];
+    G &g = gates[gi];
     if (g.kind != kDense) {
       switch (g.k) {
       case 1:
@@ -624,6 +637,29 @@ __global__ void __launch_bounds__(1 << (12 + Shape<T>::P - R), R == 3 + Shape<T>
     __builtin_nontemporal_store(*reinterpret_cast<const Unit *>(lds + t.local(i)), t.global(i));
 }
 
+template <typename T, int R>
+__global__ void __launch_bounds__(1 << (12 + Shape<T>::P - R), R == 3 + Shape<T>::P ? 4 : 2)
+    k_group(T *__restrict__ sv, GroupArgs a) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const GroupHead &h = a.h;
+  run_group<T, R>(sv, h, static_cast<const GroupGate *>(a.g), lds);
+}
+
+// Groups on several statevectors, one per grid row, from a table.  A small
+// statevector has few tiles (16 qubits f64: 16), and its pass is a chain of
+// gates of about 1 us each on that many CUs; here they run side by side.
+// 16 members of a noisy 16-qubit ensemble, 3 layers: 6447 us with a launch
+// per member and pass (950 launches), 1666 with these.
+template <typename T, int R>
+__global__ void __launch_bounds__(1 << (12 + Shape<T>::P - R), R == 3 + Shape<T>::P ? 4 : 2)
+    k_group_batch(Const<GroupHead> heads, Const<GroupGate> gates) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  auto &h = heads[blockIdx.y];
+  using GT = __attribute__((address_space(1))) T;
+  T *sv = (T *)((GT *)(reinterpret_cast<uintptr_t>(h.sv)));
+  run_group<T, R>(sv, h, gates + h.first, lds);
+}
+
 // ── Host side ───────────────────────────────────────────────────────────────
 
 bool is_diagonal(const GatePlan &p) {
@@ -662,6 +698,14 @@ template <typename T, int R>
 void launch_k_group(dim3 grid, dim3 block, size_t lds, hipStream_t stream, void *sv,
                     const GroupArgs &a) {
   hipLaunchKernelGGL((k_group<T, R>), grid, block, lds, stream, static_cast<T *>(sv), a);
+}
+
+template <typename T, int R>
+void launch_k_group_batch(dim3 grid, dim3 block, size_t lds, hipStream_t stream,
+                          const GroupHead *heads, const GroupGate *gates) {
+  hipLaunchKernelGGL((k_group_batch<T, R>), grid, block, lds, stream,
+                     (Const<GroupHead>)(reinterpret_cast<uintptr_t>(heads)),
+                     (Const<GroupGate>)(reinterpret_cast<uintptr_t>(gates)));
 }
 
 } // namespace
@@ -759,10 +803,18 @@ GroupLimits group_limits(const GatePlan &p, uint32_t n) {
   return l;
 }
 
-void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stream, void *sv,
-                  uint32_t n) {
-  if (n_plans == 0)
-    return;
+namespace {
+
+// Amplitudes per thread: twice as many, with half the threads, from 2^10
+// tiles on.  There the tiles are enough to fill the chip and a wave that
+// runs more MFMA tiles per operand load is the faster one (30 qubits f64,
+// 90 gates in 44 passes: 373 ms against 393); below it the latency of a
+// gate counts (12 qubits f64, 23 gates: 64 us against 74).
+bool many_tiles(uint32_t n, uint8_t prec) { return n >= max_tile(prec) + 10; }
+
+// Head and gates (identities left out) of a group; `gates` holds n_plans.
+void describe_group(const GatePlan *const *plans, size_t n_plans, uint32_t n, GroupHead &a,
+                    GroupGate *gates) {
   if (n_plans > size_t(kMaxGroupGates))
     throw Error("a gate group holds at most " + std::to_string(kMaxGroupGates) + " gates");
   if (n > 40)
@@ -781,13 +833,7 @@ void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stre
       set |= uint64_t(1) << p.q[b];
   }
   const uint32_t m = std::min(n, max_tile(prec));
-  // Amplitudes per thread: twice as many, with half the threads, from 2^10
-  // tiles on.  There the tiles are enough to fill the chip and a wave that
-  // runs more MFMA tiles per operand load is the faster one (30 qubits f64,
-  // 90 gates in 44 passes: 373 ms against 393); below it the latency of a
-  // gate counts (12 qubits f64, 23 gates: 64 us against 74).
-  const bool large = n - m >= 10;
-  const uint32_t R = regs_log2(prec) + large;
+  const uint32_t R = regs_log2(prec) + many_tiles(n, prec);
   const uint32_t low = low_qubits(prec);
   set |= (uint64_t(1) << low) - 1;
   if (uint32_t(__builtin_popcountll(set)) > m)
@@ -797,7 +843,7 @@ void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stre
   for (uint32_t q = 0; uint32_t(__builtin_popcountll(set)) < m; ++q)
     set |= uint64_t(1) << q;
 
-  GroupArgs a{};
+  a = {};
   a.m = m;
   a.thread_bits = m - R;
   uint8_t local[64] = {};
@@ -814,7 +860,8 @@ void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stre
     const bool mono = p.variant == 2;
     if (mono && p.n_active == 0)
       continue; // identity
-    GroupGate &g = a.g[a.n_gates++];
+    GroupGate &g = gates[a.n_gates++];
+    g = {};
     const bool diag = mono && is_diagonal(p);
     const bool mfma = !mono && p.k >= 4;
     g.mat = mfma ? p.d_op : p.d_mat;
@@ -865,19 +912,83 @@ void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stre
     for (uint32_t b = 0; b < kMaxOffsets; ++b)
       g.off2[b >> 1] |= off[b] << (16 * (b & 1));
   }
-  if (a.n_gates == 0)
-    return;
   const uint32_t tile_bits = n - m;
   a.xcd_bits = tile_bits >= 6 ? tile_bits : 0;
-  const size_t lds = size_t(16) << (m - (f32 ? 1 : 0));
-  const dim3 grid(1u << tile_bits), block(1u << a.thread_bits);
-  if (f32)
-    large ? launch_k_group<float, 5>(grid, block, lds, stream, sv, a)
-          : launch_k_group<float, 4>(grid, block, lds, stream, sv, a);
+}
+
+size_t tile_bytes(uint32_t m, uint8_t prec) { return size_t(prec == 0 ? 8 : 16) << m; }
+
+} // namespace
+
+void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stream, void *sv,
+                  uint32_t n) {
+  if (n_plans == 0)
+    return;
+  const uint8_t prec = plans[0]->precision;
+  GroupArgs a;
+  describe_group(plans, n_plans, n, a.h, a.g);
+  if (a.h.n_gates == 0)
+    return;
+  const size_t lds = tile_bytes(a.h.m, prec);
+  const dim3 grid(1u << (n - a.h.m)), block(1u << a.h.thread_bits);
+  if (prec == 0)
+    many_tiles(n, prec) ? launch_k_group<float, 5>(grid, block, lds, stream, sv, a)
+                        : launch_k_group<float, 4>(grid, block, lds, stream, sv, a);
   else
-    large ? launch_k_group<double, 4>(grid, block, lds, stream, sv, a)
-          : launch_k_group<double, 3>(grid, block, lds, stream, sv, a);
+    many_tiles(n, prec) ? launch_k_group<double, 4>(grid, block, lds, stream, sv, a)
+                        : launch_k_group<double, 3>(grid, block, lds, stream, sv, a);
   check(hipGetLastError(), "hipLaunchKernelGGL(k_group)");
+}
+
+size_t group_batch_bytes(size_t n_groups, size_t n_plans) {
+  return n_groups * sizeof(GroupHead) + n_plans * sizeof(GroupGate);
+}
+
+void launch_group_batch(const GroupItem *items, size_t n_items, uint32_t n, void *table,
+                        hipStream_t stream) {
+  if (n_items == 0)
+    return;
+  const uint8_t prec = items[0].plans[0]->precision;
+  if (many_tiles(n, prec))
+    throw Error("grouped gates on a " + std::to_string(n) +
+                "-qubit statevector fill the chip by themselves");
+  size_t n_plans = 0;
+  for (size_t i = 0; i < n_items; ++i)
+    n_plans += items[i].n_plans;
+  std::vector<unsigned char> host(group_batch_bytes(n_items, n_plans));
+  GroupHead *heads = reinterpret_cast<GroupHead *>(host.data());
+  GroupGate *gates = reinterpret_cast<GroupGate *>(heads + n_items);
+  uint64_t at = 0;
+  for (size_t i = 0; i < n_items; ++i) {
+    const GroupItem &it = items[i];
+    if (it.plans[0]->precision != prec)
+      throw Error("grouped plans must share the precision");
+    if (i && it.round < items[i - 1].round)
+      throw Error("rounds of grouped gates must not decrease");
+    describe_group(it.plans, it.n_plans, n, heads[i], gates + at);
+    heads[i].sv = it.sv;
+    heads[i].first = at;
+    at += it.n_plans;
+  }
+  check(hipMemcpyAsync(table, host.data(), host.size(), hipMemcpyHostToDevice, stream),
+        "hipMemcpyAsync(group table)");
+  const auto *d_heads = static_cast<const GroupHead *>(table);
+  const auto *d_gates = reinterpret_cast<const GroupGate *>(d_heads + n_items);
+  const size_t lds = tile_bytes(heads[0].m, prec);
+  const dim3 block(1u << heads[0].thread_bits);
+  for (size_t i = 0; i < n_items;) {
+    size_t end = i + 1;
+    while (end < n_items && items[end].round == items[i].round && end - i < 32768)
+      ++end;
+    const dim3 grid(1u << (n - heads[0].m), unsigned(end - i));
+    if (prec == 0)
+      launch_k_group_batch<float, 4>(grid, block, lds, stream, d_heads + i, d_gates);
+    else
+      launch_k_group_batch<double, 3>(grid, block, lds, stream, d_heads + i, d_gates);
+    check(hipGetLastError(), "hipLaunchKernelGGL(k_group_batch)");
+    i = end;
+  }
+  // Pageable memory: the copy has read it when hipMemcpyAsync returns.
 }
 
 } // namespace cast_hip

@@ -155,6 +155,29 @@ TrajectoryResult Simulator::sample_trajectory(const CircuitGraph &graph,
   // Ensemble (trajectory.rs:186-265).
   const size_t max_ensemble = std::max<size_t>(1, opts.max_ensemble);
   std::vector<Member> ens;
+  std::vector<HipStatevector> spare; // of members that were dropped
+  // No gate stays queued for a member that is gone, also when this throws.
+  struct Unqueue {
+    HipKernelManager &mgr;
+    std::vector<Member> &ens;
+    ~Unqueue() {
+      for (const Member &m : ens)
+        mgr.discard(m.sv.dptr());
+    }
+  } unqueue{mgr_, ens};
+  // The state without its queued gates, copied on the manager's stream.
+  auto copy_of = [&](const HipStatevector &sv) {
+    HipStatevector to = spare.empty() ? HipStatevector(n_physical, spec_.precision)
+                                      : std::move(spare.back());
+    if (!spare.empty())
+      spare.pop_back();
+    char err[1024];
+    throw_if(cast_hip_memcpy_dtod_async(to.dptr(), sv.dptr(),
+                                        sv.n_elements() * spec_.scalar_bytes(), mgr_.stream(),
+                                        err, sizeof(err)),
+             err);
+    return to;
+  };
   {
     HipStatevector sv(n_physical, spec_.precision);
     sv.zero();
@@ -183,24 +206,39 @@ TrajectoryResult Simulator::sample_trajectory(const CircuitGraph &graph,
       mgr_.apply(kids[cand[0].branch], ens[0].sv);
       continue;
     }
-    mgr_.sync(false); // every queued gate lands before a member is copied
+    // Only a member that is copied needs its queued gates first; the copy
+    // follows them on the manager's stream.
     std::vector<size_t> refs(ens.size(), 0);
     for (const auto &c : cand)
       ++refs[c.member];
+    std::vector<uint64_t> copied;
+    for (size_t m = 0; m < ens.size(); ++m)
+      if (refs[m] > 1)
+        copied.push_back(ens[m].sv.dptr());
+    mgr_.launch(copied);
+    for (size_t m = 0; m < ens.size(); ++m)
+      if (refs[m] == 0) {
+        mgr_.discard(ens[m].sv.dptr());
+        spare.push_back(std::move(ens[m].sv));
+      }
     std::vector<Member> next;
     next.reserve(kept);
+    std::vector<size_t> moved(ens.size(), kept); // a moved member's place in next
     for (const auto &c : cand) {
       Member &parent = ens[c.member];
-      const bool last_ref = --refs[c.member] == 0;
-      if (last_ref) {
-        next.push_back(Member{std::move(parent.sv), c.weight, std::move(parent.path)});
+      // The member's own buffer goes to its first candidate; every other one
+      // copies the state as it is before this gate.
+      if (moved[c.member] == kept) {
+        moved[c.member] = next.size();
+        next.push_back(Member{std::move(parent.sv), c.weight, parent.path});
       } else {
-        next.push_back(Member{parent.sv.clone_device(), c.weight, parent.path});
+        next.push_back(Member{copy_of(next[moved[c.member]].sv), c.weight, parent.path});
       }
       next.back().path.push_back(c.branch);
-      mgr_.apply(kids[c.branch], next.back().sv);
     }
     ens = std::move(next);
+    for (size_t x = 0; x < kept; ++x)
+      mgr_.apply(kids[cand[x].branch], ens[x].sv);
   }
   mgr_.sync(false);
 

@@ -131,6 +131,8 @@ HipKernelManager::~HipKernelManager() {
     char err[kErr];
     (void)cast_hip_stream_sync(stream_, err, kErr);
   }
+  if (group_scratch_)
+    cast_hip_free(group_scratch_);
   for (void *e : events_)
     cast_hip_event_destroy(e);
   if (stream_)
@@ -381,6 +383,8 @@ void HipKernelManager::launch_passes_locked(const std::vector<Pending> &work,
       lists.emplace_back();
     lists[it->second].push_back(i);
   }
+  if (lists.size() > 1 && spec_.variant == CAST_HIP_VARIANT_AUTO)
+    lists = launch_shared_locked(work, std::move(lists));
   std::vector<const void *> plans;
   for (const auto &list : lists) {
     const uint64_t dptr = work[list[0]].dptr;
@@ -407,6 +411,122 @@ void HipKernelManager::launch_passes_locked(const std::vector<Pending> &work,
       plans.push_back(work[i].base);
     apply_in_passes(plans, stream_, dptr, n, single);
   }
+}
+
+// A pass over a small statevector is bound by the chain of its gates on a few
+// CUs, so the passes of several such statevectors go side by side: launch r
+// takes pass r of each.
+std::vector<std::vector<size_t>>
+HipKernelManager::launch_shared_locked(const std::vector<Pending> &work,
+                                       std::vector<std::vector<size_t>> lists) {
+  char err[kErr];
+  std::vector<std::vector<size_t>> rest;
+  std::map<uint32_t, std::vector<std::vector<size_t>>> by_size;
+  for (auto &list : lists) {
+    const Pending &w = work[list[0]];
+    cast_hip_group_info_t info{};
+    throw_if(cast_hip_gate_group_info(w.base, w.n_qubits, &info, err, kErr), err);
+    bool tuning = false;
+    for (size_t i : list)
+      tuning = tuning || work[i].cand >= 0;
+    if (info.targets && w.n_qubits < info.max_qubits + 10 && !tuning)
+      by_size[w.n_qubits].push_back(std::move(list));
+    else
+      rest.push_back(std::move(list));
+  }
+  for (auto &[n, some] : by_size) {
+    if (some.size() == 1) {
+      rest.push_back(std::move(some[0]));
+      continue;
+    }
+    struct Passes {
+      std::vector<const void *> plans; // pass after pass
+      std::vector<size_t> end;
+      uint64_t sv;
+    };
+    std::vector<Passes> all;
+    size_t most = 0, n_plans = 0, n_groups = 0;
+    for (auto &list : some) {
+      std::vector<const void *> plans;
+      for (size_t i : list)
+        plans.push_back(work[i].base);
+      bool join = true;
+      const auto passes = plan_passes(plans, n, &join);
+      if (!join) {
+        rest.push_back(std::move(list));
+        continue;
+      }
+      Passes p;
+      p.sv = work[list[0]].dptr;
+      for (const auto &pass : passes) {
+        for (uint32_t i : pass)
+          p.plans.push_back(plans[i]);
+        p.end.push_back(p.plans.size());
+      }
+      most = std::max(most, p.end.size());
+      n_plans += p.plans.size();
+      n_groups += p.end.size();
+      all.push_back(std::move(p));
+    }
+    if (all.empty())
+      continue;
+    std::vector<cast_hip_group_item_t> items;
+    items.reserve(n_groups);
+    for (size_t r = 0; r < most; ++r)
+      for (const Passes &p : all)
+        if (r < p.end.size()) {
+          const size_t first = r ? p.end[r - 1] : 0;
+          items.push_back({p.plans.data() + first, p.end[r] - first, p.sv, uint32_t(r), 0});
+        }
+    const size_t need = cast_hip_group_batch_scratch_bytes(n_groups, n_plans);
+    if (need > group_scratch_bytes_) {
+      if (group_scratch_) {
+        throw_if(cast_hip_stream_sync(stream_, err, kErr), err);
+        cast_hip_free(group_scratch_);
+        group_scratch_ = 0;
+        group_scratch_bytes_ = 0;
+      }
+      const size_t bytes = std::max(need, size_t(1) << 20);
+      group_scratch_ = cast_hip_malloc(bytes, err, kErr);
+      if (!group_scratch_)
+        throw Error(err);
+      group_scratch_bytes_ = bytes;
+    }
+    throw_if(cast_hip_gate_apply_group_batch(items.data(), items.size(), n, group_scratch_,
+                                             stream_, err, kErr),
+             err);
+  }
+  return rest;
+}
+
+void HipKernelManager::launch(const std::vector<uint64_t> &svs) {
+  {
+    std::lock_guard<std::mutex> lock(mu_);
+    std::vector<Pending> work, keep;
+    bool tuning = false;
+    for (const Pending &p : pending_) {
+      const bool mine = std::find(svs.begin(), svs.end(), p.dptr) != svs.end();
+      (mine ? work : keep).push_back(p);
+      tuning = tuning || (mine && p.cand >= 0);
+    }
+    if (work.empty())
+      return;
+    if (!tuning) {
+      ensure_stream_locked();
+      pending_.swap(keep);
+      std::vector<size_t> sampled;
+      launch_passes_locked(work, sampled);
+      return;
+    }
+  }
+  sync(false); // tuning samples are read after a wait
+}
+
+void HipKernelManager::discard(uint64_t sv) {
+  std::lock_guard<std::mutex> lock(mu_);
+  pending_.erase(std::remove_if(pending_.begin(), pending_.end(),
+                                [&](const Pending &p) { return p.dptr == sv; }),
+                 pending_.end());
 }
 
 SyncStats HipKernelManager::sync(bool timed) {

@@ -146,6 +146,11 @@ public:
   KernelId generate(const QuantumGate &gate);
   void apply(KernelId id, HipStatevector &sv);
   SyncStats sync(bool timed = true);
+  // Launches the gates queued for `svs` (device pointers) on the manager's
+  // stream without waiting; gates for other statevectors stay queued.
+  void launch(const std::vector<uint64_t> &svs);
+  // Drops the gates queued for a statevector that is no longer wanted.
+  void discard(uint64_t sv);
   TimingStats time_adaptive(KernelId id, HipStatevector &sv, double budget_s);
   PlanInfo plan_info(KernelId id) const;
   // Kernel family (CAST_HIP_VARIANT_*) launched for `id` on n_qubits; with
@@ -180,6 +185,11 @@ private:
     std::vector<char> dropped;
     int chosen = -1;
   };
+  // Every list (queue positions of one statevector) whose gates can all run in
+  // groups, on statevectors too small to fill the chip, in launches shared by
+  // such lists; returns the other lists.
+  std::vector<std::vector<size_t>>
+  launch_shared_locked(const std::vector<Pending> &work, std::vector<std::vector<size_t>> lists);
   // Untimed work in few passes; the queue positions of tuning samples (each
   // between two events) go to `sampled`.
   void launch_passes_locked(const std::vector<Pending> &work, std::vector<size_t> &sampled);
@@ -199,6 +209,8 @@ private:
   bool autotune_ = true;
   uint32_t tune_min_qubits_ = 22;
   uint32_t tune_samples_ = 2;
+  uint64_t group_scratch_ = 0; // tables of shared launches, on stream_
+  size_t group_scratch_bytes_ = 0;
   std::map<std::pair<KernelId, uint32_t>, TuneState> tune_;
 };
 

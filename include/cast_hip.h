@@ -280,6 +280,25 @@ int cast_hip_gate_apply_group(const void *const *plans, size_t n_plans, void *st
                               uint64_t sv_dptr, uint32_t sv_n_qubits, char *err_buf,
                               size_t err_buf_len);
 
+/* Groups on several statevectors of sv_n_qubits qubits with one launch per
+ * round (rounds must not decrease along the list; the groups of one round act
+ * on different statevectors).  Statevectors that fill the chip by themselves
+ * (group tiles of 2^max_qubits amplitudes: 2^10 of them or more) are an error.
+ * `scratch` is cast_hip_group_batch_scratch_bytes of device memory, free for
+ * the work queued on `stream`; `items` and the plan lists may be released
+ * when the call returns.  Copies from pageable memory: not for capture. */
+typedef struct cast_hip_group_item_t {
+  const void *const *plans;
+  size_t n_plans;
+  uint64_t sv;
+  uint32_t round;
+  uint32_t reserved;
+} cast_hip_group_item_t;
+size_t cast_hip_group_batch_scratch_bytes(size_t n_groups, size_t n_plans);
+int cast_hip_gate_apply_group_batch(const cast_hip_group_item_t *items, size_t n_items,
+                                    uint32_t sv_n_qubits, uint64_t scratch, void *stream,
+                                    char *err_buf, size_t err_buf_len);
+
 /* ⟨Z_a Z_b⟩ for n_pairs qubit pairs (pairs = [a0,b0,a1,b1,...]), accumulated
  * in f64 over |amp|^2; no normalisation is applied.  Synchronous on `stream`.
  * No reference counterpart (the reference downloads the whole statevector,
