@@ -75,7 +75,7 @@ struct GroupHead {
   uint32_t thread_bits;  // log2(threads per workgroup)
   uint32_t m;            // tile qubits
   uint32_t xcd_bits;     // 0, or log2(tiles): tiles in XCD order
-  uint8_t s[16];         // tile qubits, ascending
+  uint32_t s[16];        // tile qubits, ascending (words: a byte is no scalar load)
   void *sv;
   uint64_t first;        // of its gates, in a table of several groups
 };
@@ -852,7 +852,7 @@ void describe_group(const GatePlan *const *plans, size_t n_plans, uint32_t n, Gr
     for (uint32_t q = 0; q < n; ++q)
       if (set >> q & 1u) {
         local[q] = uint8_t(i);
-        a.s[i++] = uint8_t(q);
+        a.s[i++] = q;
       }
   }
   for (size_t i = 0; i < n_plans; ++i) {

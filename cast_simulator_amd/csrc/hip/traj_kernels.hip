@@ -390,13 +390,17 @@ __device__ __forceinline__ void wg_gate_k(const T *src, T *dst, const T *__restr
 // Squared norm and the pair sums of the workgroup's final state, written to
 // out_row[0 .. 1 + n_pairs).  Amplitude i = tid + B r (B = blockDim.x = 2^bB).
 // The sign of pair (a, b) at i factors into a per-thread part (positions
-// below bB), applied once at the end, and a part that depends only on the row
-// r: the parity of r & m for the pair's row mask m, computed with scalar
-// instructions since r is uniform across the workgroup.  The inner loop then
-// does one f64 FMA per pair with a uniform +-1; 16 rows are loaded at a time.
+// below bB), applied once at the end, and the parity of r & m for the pair's
+// row mask m.  16 rows are taken at a time: the 16-point Walsh-Hadamard
+// transform of their probabilities (64 additions) holds the sums under every
+// mask of the low 4 row bits, and the parity of the others is the same for the
+// whole workgroup, so a pair costs one f64 FMA for 16 amplitudes instead of
+// one each: the sums of 188 states of 20 qubits (f32, 19 pairs, one workgroup
+// each) 1.67 -> 1.1 ms.  Rows [first_row, first_row + n_rows) are summed.
 template <typename T>
 __device__ __forceinline__ void wg_observe(const T *sv, uint32_t n, uint32_t n_pairs, uint32_t bB,
-                           const uint32_t *s_pairs, double *out_row, double *red) {
+                           const uint32_t *s_pairs, uint32_t first_row, uint32_t n_rows,
+                           double *out_row, double *red) {
   using VT = typename V2<T>::type;
   constexpr int R = 16;
   const VT *amp = reinterpret_cast<const VT *>(sv);
@@ -419,8 +423,9 @@ __device__ __forceinline__ void wg_observe(const T *sv, uint32_t n, uint32_t n_p
   for (int j = 0; j < 1 + kMaxPairs; ++j)
     acc[j] = 0.0;
   const uint64_t len = uint64_t(1) << n;
-  const uint32_t rows = n > bB ? (1u << (n - bB)) : 1u;
-  for (uint32_t r0 = 0; r0 < rows; r0 += R) {
+  const uint32_t rows = first_row + n_rows;
+  typedef double Rows __attribute__((ext_vector_type(R)));
+  for (uint32_t r0 = first_row; r0 < rows; r0 += R) {
     double p[R];
 #pragma unroll
     for (int u = 0; u < R; ++u) {
@@ -432,18 +437,26 @@ __device__ __forceinline__ void wg_observe(const T *sv, uint32_t n, uint32_t n_p
         p[u] = re * re + im * im;
       }
     }
+    Rows w;
 #pragma unroll
-    for (int u = 0; u < R; ++u) {
-      const uint32_t r = r0 + u;
-      acc[0] += p[u];
-      // All 32 slots are accumulated (unused ones have mask 0 and are never
-      // read): no per-pair guard for the compiler to turn into selects.
+    for (int u = 0; u < R; ++u)
+      w[u] = p[u];
 #pragma unroll
-      for (int j = 0; j < kMaxPairs; ++j) {
-        const double sg = (__builtin_popcount(r & rmask[j]) & 1) ? -1.0 : 1.0;
-        acc[1 + j] = __builtin_fma(sg, p[u], acc[1 + j]);
+    for (int b = 1; b < R; b <<= 1)
+#pragma unroll
+      for (int u = 0; u < R; ++u)
+        if (!(u & b)) {
+          const double lo = w[u], hi = w[u | b];
+          w[u] = lo + hi;
+          w[u | b] = lo - hi;
+        }
+    acc[0] += w[0];
+#pragma unroll
+    for (int j = 0; j < kMaxPairs; ++j)
+      if (uint32_t(j) < n_pairs) { // uniform
+        const bool neg = __builtin_popcount(r0 & rmask[j]) & 1;
+        acc[1 + j] = __builtin_fma(neg ? -1.0 : 1.0, w[rmask[j] & (R - 1)], acc[1 + j]);
       }
-    }
   }
 #pragma unroll
   for (int j = 0; j < kMaxPairs; ++j)
@@ -555,7 +568,12 @@ __device__ __forceinline__ bool fetch_task(const cast_hip_traj_task_t *tasks,
   return ok;
 }
 
-// The workgroup's copy of a final state.
+// Rows of wg_observe in a whole statevector.
+__host__ __device__ __forceinline__ uint32_t observe_rows(uint32_t n, uint32_t log2_block) {
+  return n > log2_block ? 1u << (n - log2_block) : 1u;
+}
+
+// The workgroup's copy of (a part of) a final state.
 template <typename T> __device__ __forceinline__ void wg_dump(const T *cur, T *to, uint64_t len) {
   using VT = typename V2<T>::type;
   const VT *src = reinterpret_cast<const VT *>(cur);
@@ -622,8 +640,8 @@ __global__ void __launch_bounds__(kMaxBlock, OCC)
       cur = slot;
       __syncthreads();
     }
-    wg_observe<T>(cur, n, a.n_pairs, a.log2_block, s_pairs, out + uint64_t(ti) * (1 + a.n_pairs),
-                  red);
+    wg_observe<T>(cur, n, a.n_pairs, a.log2_block, s_pairs, 0, observe_rows(n, a.log2_block),
+                  out + uint64_t(ti) * (1 + a.n_pairs), red);
     if (dump) {
       wg_dump<T>(cur, dump + 2 * len * ti, len);
       __syncthreads();
@@ -636,8 +654,8 @@ __global__ void __launch_bounds__(kMaxBlock, OCC)
 // owns a statevector (k_traj) is held to what one CU can do, and the launch to
 // its longest task: 188 tasks of 20 qubits and up to 40 gates at f32 took
 // 29.4 ms with 0.73 ms per gate on each of 188 CUs.  With a launch per step all
-// CUs share the tasks that are left: 17.0 ms (4.6 us per gate of 16.8 MB moved,
-// 3.7 TB/s, k = 5 and 6 bound by the split products), 32 tasks 23.6 -> 4.4 ms.
+// CUs share the tasks that are left: 15.7 ms (4.2 us per gate of 16.8 MB moved,
+// 4.0 TB/s, k = 5 and 6 bound by the split products), 32 tasks 23.6 -> 3.9 ms.
 // Each amplitude goes through the same operations as in k_traj.
 template <typename T, int OCC>
 __global__ void __launch_bounds__(kMaxBlock, OCC)
@@ -662,32 +680,56 @@ __global__ void __launch_bounds__(kMaxBlock, OCC)
     atomicOr(&work[1], 1u);
 }
 
-// Sums and dump of the tasks order[first ...), one workgroup each, after
-// their last step.  A task with more gates than `n_steps` is an error.
+// Sums and dump of the tasks order[first ...) after their last step, `parts`
+// workgroups each.  With several, a part leaves its sums at the start of the range of the
+// slot that it alone has read (or that holds nothing, for a task without
+// gates); k_traj_sum adds them up.  A task with more gates than `n_steps` is an
+// error.  188 states of 20 qubits, f32: 1.1 ms in one part, 0.56 in eight.
 template <typename T>
 __global__ void __launch_bounds__(kMaxBlock, 2)
     k_traj_finish(const cast_hip_traj_task_t *__restrict__ tasks,
-                  const uint32_t *__restrict__ order, const T *__restrict__ checkpoints,
-                  const T *__restrict__ slots, double *__restrict__ out, T *__restrict__ dump,
-                  uint32_t *__restrict__ work, TrajScalars a, uint32_t first, uint32_t n_steps) {
+                  const uint32_t *__restrict__ order, const T *__restrict__ checkpoints, T *slots,
+                  double *__restrict__ out, T *__restrict__ dump, uint32_t *__restrict__ work,
+                  TrajScalars a, uint32_t first, uint32_t n_steps, uint32_t parts) {
   __shared__ uint32_t s_pairs[2 * kMaxPairs];
   __shared__ double red[kMaxWaves * (1 + kMaxPairs)];
   if (threadIdx.x < 2 * a.n_pairs)
     s_pairs[threadIdx.x] = a.pairs[threadIdx.x];
   __syncthreads();
+  const uint32_t slot_i = blockIdx.x / parts, part = blockIdx.x % parts;
   uint32_t ti;
   cast_hip_traj_task_t task{};
-  if (!fetch_task(tasks, order, first + blockIdx.x, work, a, ti, task))
+  if (!fetch_task(tasks, order, first + slot_i, work, a, ti, task))
     return;
   if (task.n_gates > n_steps)
     atomicOr(&work[1], 1u);
-  const uint64_t len = uint64_t(1) << a.n_qubits;
-  const T *cur = task.n_gates == 0 ? checkpoints + 2 * len * task.checkpoint
-                                   : slots + 2 * len * blockIdx.x;
-  wg_observe<T>(cur, a.n_qubits, a.n_pairs, a.log2_block, s_pairs,
-                out + uint64_t(ti) * (1 + a.n_pairs), red);
-  if (dump)
-    wg_dump<T>(cur, dump + 2 * len * ti, len);
+  const uint64_t len = uint64_t(1) << a.n_qubits, mine = len / parts;
+  T *slot = slots + 2 * len * slot_i;
+  const T *cur = task.n_gates == 0 ? checkpoints + 2 * len * task.checkpoint : slot;
+  if (dump) {
+    wg_dump<T>(cur + 2 * mine * part, dump + 2 * (len * ti + mine * part), mine);
+    __syncthreads();
+  }
+  const uint32_t n_rows = observe_rows(a.n_qubits, a.log2_block) / parts;
+  // Every read of the range is over at the barrier before the sums go out.
+  double *sums = parts == 1 ? out + uint64_t(ti) * (1 + a.n_pairs)
+                            : reinterpret_cast<double *>(slot + 2 * mine * part);
+  wg_observe<T>(cur, a.n_qubits, a.n_pairs, a.log2_block, s_pairs, n_rows * part, n_rows, sums,
+                red);
+}
+
+template <typename T>
+__global__ void k_traj_sum(const uint32_t *__restrict__ order, const T *__restrict__ slots,
+                           double *__restrict__ out, TrajScalars a, uint32_t first,
+                           uint32_t parts) {
+  const uint32_t ti = order[first + blockIdx.x], slots_n = 1 + a.n_pairs;
+  if (ti >= a.n_tasks || threadIdx.x >= slots_n)
+    return;
+  const uint64_t len = uint64_t(1) << a.n_qubits, mine = len / parts;
+  double s = 0.0;
+  for (uint32_t p = 0; p < parts; ++p)
+    s += reinterpret_cast<const double *>(slots + 2 * (len * blockIdx.x + mine * p))[threadIdx.x];
+  out[uint64_t(ti) * slots_n + threadIdx.x] = s;
 }
 
 template <typename T, int OCC>
@@ -717,6 +759,14 @@ void launch_steps_t(const cast_hip_traj_launch_t &L, const TrajScalars &a, const
   // At most as many parts as leave every wave a k = 6 tile of 2^10 amplitudes.
   const uint32_t most =
       L.n_qubits > 10 ? std::max(1u, (1u << std::min(L.n_qubits - 10, 20u)) / waves) : 1u;
+  // Parts of the closing sums: four or more groups of 16 rows (4096 amplitudes) each.
+  auto parts_of = [&](uint32_t tasks_here) {
+    const uint32_t rows = observe_rows(L.n_qubits, a.log2_block);
+    uint32_t parts = 1;
+    while (parts * tasks_here < kStepGroups && rows / (2 * parts) >= 64)
+      parts *= 2;
+    return parts;
+  };
   for (uint32_t first = 0; first < L.n_tasks; first += L.n_slots) {
     const uint32_t here = std::min(L.n_slots, L.n_tasks - first);
     uint32_t active = here;
@@ -729,10 +779,16 @@ void launch_steps_t(const cast_hip_traj_launch_t &L, const TrajScalars &a, const
                          order, gates, mats, ckpt, slots, work, a, first, g, parts);
       check(hipGetLastError(), "hipLaunchKernelGGL(k_traj_step)");
     }
-    hipLaunchKernelGGL((k_traj_finish<T>), dim3(here), dim3(L.block), 0, s, tasks, order, ckpt,
-                       slots, reinterpret_cast<double *>(L.out), reinterpret_cast<T *>(L.dump),
-                       work, a, first, n_steps);
+    const uint32_t parts = parts_of(here);
+    hipLaunchKernelGGL((k_traj_finish<T>), dim3(here * parts), dim3(L.block), 0, s, tasks, order,
+                       ckpt, slots, reinterpret_cast<double *>(L.out),
+                       reinterpret_cast<T *>(L.dump), work, a, first, n_steps, parts);
     check(hipGetLastError(), "hipLaunchKernelGGL(k_traj_finish)");
+    if (parts == 1)
+      continue;
+    hipLaunchKernelGGL((k_traj_sum<T>), dim3(here), dim3(64), 0, s, order, slots,
+                       reinterpret_cast<double *>(L.out), a, first, parts);
+    check(hipGetLastError(), "hipLaunchKernelGGL(k_traj_sum)");
   }
 }
 
