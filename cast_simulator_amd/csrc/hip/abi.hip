@@ -187,14 +187,15 @@ GatePlan *build_plan(const cast_hip_kernel_gen_spec_t *spec, const cast_complex6
   ensure_device();
   check(hipGetDevice(&plan->device), "hipGetDevice");
   // The complex matrix, for dense k >= 4 the real matrices Re M, Im M, Re M +
-  // Im M of the three-product form, and the operands for groups of gates:
-  // one allocation, one copy.
+  // Im M of the three-product form, and the operands (of a monomial gate, the
+  // entries) for groups of gates: one allocation, one copy.
   const size_t KK = K * K, sb = fp32 ? 4 : 8;
   const bool real3 = variant != CAST_HIP_VARIANT_MONOMIAL && n_qubits >= 4;
   const size_t mat3_at = 2 * KK * sb, op_at = mat3_at + (real3 ? 3 * KK * sb : 0);
-  const bool op = real3 && (n_qubits <= 5 || fp32);
-  plan->block_bytes =
-      op_at + (op ? group_operand_bytes(uint32_t(n_qubits), plan->precision) : 0);
+  const bool op = real3 && (n_qubits <= 5 || fp32), entries = variant == CAST_HIP_VARIANT_MONOMIAL;
+  plan->block_bytes = op_at + (op        ? group_operand_bytes(uint32_t(n_qubits), plan->precision)
+                               : entries ? 2 * K * sb
+                                         : 0);
   std::vector<unsigned char> host(plan->block_bytes);
   auto put = [&](size_t at, const double *v, size_t n) {
     if (fp32) {
@@ -217,11 +218,21 @@ GatePlan *build_plan(const cast_hip_kernel_gen_spec_t *spec, const cast_complex6
   }
   if (op)
     group_operands(m.data(), uint32_t(n_qubits), plan->precision, host.data() + op_at);
+  if (entries) { // one per row
+    std::vector<double> e(2 * K, 0.0);
+    for (size_t r = 0; r < K; ++r)
+      e[2 * r] = 1.0;
+    for (uint32_t x = 0; x < plan->n_active; ++x) {
+      e[2 * plan->act_row[x]] = plan->act_re[x];
+      e[2 * plan->act_row[x] + 1] = plan->act_im[x];
+    }
+    put(op_at, e.data(), e.size());
+  }
   plan->d_block = cache_alloc(plan->block_bytes);
   unsigned char *d = static_cast<unsigned char *>(plan->d_block);
   plan->d_mat = d;
   plan->d_mat3 = real3 ? d + mat3_at : nullptr;
-  plan->d_op = op ? d + op_at : nullptr;
+  plan->d_op = op || entries ? d + op_at : nullptr;
   const hipError_t copied =
       hipMemcpy(plan->d_block, host.data(), plan->block_bytes, hipMemcpyHostToDevice);
   if (copied != hipSuccess)

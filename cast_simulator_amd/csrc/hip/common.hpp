@@ -91,8 +91,8 @@ struct GatePlan {
   size_t block_bytes = 0;
   void *d_mat = nullptr;       // K*K complex, interleaved, device precision
   void *d_mat3 = nullptr;      // [Re M | Im M | Re M + Im M], 3*K*K real (dense k >= 4)
-  void *d_op = nullptr;        // matrix-core operands in the order of the lanes (dense k = 4,
-                               // 5; group_operands)
+  void *d_op = nullptr;        // for groups: matrix-core operands in the order of the lanes
+                               // (dense k >= 4; group_operands), a monomial gate's K entries
   double *h_mat = nullptr;     // snapped matrix in f64 (host copy, 2*K*K)
   uint64_t scalar_nnz = 0;
   // Monomial form: rows that differ from identity, each with one source col.

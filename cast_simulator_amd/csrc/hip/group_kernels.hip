@@ -21,8 +21,8 @@
 //   k = 4, f64 5  three real products on the matrix cores, 16 combos per
 //                 MFMA tile, operands laid out by lane when the plan is built;
 //   f32 k = 5, 6  bf16 split products as in the single-gate kernel;
-//   monomial      diagonal gates (any k) multiply in place, permutations
-//                 (k <= 4) move amplitudes between LDS slots.
+//   monomial      phases and diagonal gates (any k) multiply in place,
+//                 permutations (k <= 4) move amplitudes between LDS slots.
 //
 // What bounds it (30 qubits, f64): loading and storing the tiles alone takes
 // 6.0-7.5 ms a pass, depending on where the tile's qubits fall on the memory
@@ -59,10 +59,11 @@ constexpr uint32_t kMaxOffsets = 13; // one per tile bit
 constexpr int kMaxGroupGates = 64;
 constexpr uint32_t kMaxGroupQubits = 34; // 2^22 workgroups at most
 
-enum Kind : uint32_t { kDense = 0, kDiagonal = 1, kPermutation = 2 };
+enum Kind : uint32_t { kDense = 0, kDiagonal = 1, kPermutation = 2, kPhase = 3 };
 
 struct GroupGate {
-  const void *mat;       // dense k >= 4: matrix-core operands (plan.d_op); else the matrix
+  const void *mat;       // dense k <= 3: the matrix; else matrix-core operands or, of a
+                         // monomial gate, the entry of each row (plan.d_op)
   uint64_t cols;         // monomial k <= 4: source column of row r in nibble r
   uint32_t off2[7];      // LDS byte offsets of the index bits, two per word, in use order
   uint32_t k;
@@ -471,7 +472,8 @@ __device__ __forceinline__ void monomial_gate(unsigned char *lds, G &g,
   constexpr int K = 1 << KL, U = 1 << (R - KL);
   using V = typename NV<T>::type;
   const uint32_t base = select_offsets<12 - R + Shape<T>::P>(g, R, tid), active = g.off2[6] >> 16;
-  Const<T> mat = (Const<T>)(reinterpret_cast<uintptr_t>(g.mat));
+  typedef T Entries __attribute__((ext_vector_type(2 * K)));
+  const Entries e = *(Const<Entries>)(reinterpret_cast<uintptr_t>(g.mat));
   __syncthreads();
   V x[U][K];
 #pragma unroll
@@ -486,8 +488,7 @@ __device__ __forceinline__ void monomial_gate(unsigned char *lds, G &g,
 #pragma unroll
   for (int r = 0; r < K; ++r)
     if (active >> r & 1u) {
-      const uint32_t c = uint32_t(g.cols >> (4 * r)) & 15u;
-      const T re = mat[2 * (r * K + c)], im = mat[2 * (r * K + c) + 1];
+      const T re = e[2 * r], im = e[2 * r + 1];
 #pragma unroll
       for (int u = 0; u < U; ++u)
         lds_put<T>(lds, base ^ select_offsets<R>(g, 0, uint32_t(u << KL | r)),
@@ -512,7 +513,7 @@ __device__ __forceinline__ void wide_monomial_gate(unsigned char *lds, G &g,
   for (int c = 0; c < N; ++c) {
     const uint32_t r = hi << R | uint32_t(c);
     const uint32_t col = diagonal ? r : uint32_t(g.cols >> (4 * r)) & 15u;
-    e[c] = mat[r << k | col];
+    e[c] = mat[r];
     x[c] = lds_get<T>(lds, base ^ select_offsets<R>(g, 0, col) ^
                                select_offsets<6 - R>(g, R, (col >> R) ^ hi));
   }
@@ -523,6 +524,54 @@ __device__ __forceinline__ void wide_monomial_gate(unsigned char *lds, G &g,
     const V o = times<T>(x[c], e[c].x, e[c].y);
     lds_put<T>(lds, base ^ select_offsets<R>(g, 0, uint32_t(c)), keep ? x[c] : o);
   }
+}
+
+// Diagonal gate with one entry other than 1 (a phase, controlled or not; any
+// k): multiplies the amplitudes of that row, 2^(R-k) per thread or one in each
+// of the first threads.  The targets' positions are the nibbles of `cols`,
+// off2[0] is the offset of the row; free index bit j of the tile is bit j of
+// (combo, thread), and off2[1 + b] the offset of the b-th one above the
+// thread's (b < 4).  The entry itself is in `mat` and off2[5, 6]: a load of it
+// would be a cache miss per gate.  Bound by its
+// instructions: as a diagonal gate on two targets, with a test per row and
+// offsets by table, it took 0.85 us on a CU, now 0.5; the 20-qubit Fourier
+// transform (180 such gates) 292 -> 235 us.
+template <typename T, int R, int KL>
+__device__ __forceinline__ void phase_gate(unsigned char *lds, const GroupGate &g, uint32_t tid,
+                                           uint32_t k) {
+  constexpr int P = Shape<T>::P, LU = KL < R ? R - KL : 0, U = 1 << LU;
+  uint32_t i = tid;
+  for (uint32_t b = 0; b < (KL < 4 ? uint32_t(KL) : k); ++b)
+    i = uint32_t(insert_zero(i, uint32_t(g.cols >> (4 * b)) & 15u));
+  const uint32_t u = i >> P;
+  uint32_t at = 16 * (u ^ ((u >> 4) & 15u) ^ ((u >> 8) & 15u)) ^ g.off2[0];
+  if (P)
+    at ^= (i & 1u) << 3;
+  const uint64_t re = reinterpret_cast<uintptr_t>(g.mat), im = uint64_t(g.off2[6]) << 32 | g.off2[5];
+  typename NV<T>::type e;
+  if constexpr (sizeof(T) == 8) {
+    e.x = __builtin_bit_cast(double, re);
+    e.y = __builtin_bit_cast(double, im);
+  } else {
+    e.x = __builtin_bit_cast(float, uint32_t(re));
+    e.y = __builtin_bit_cast(float, uint32_t(im));
+  }
+  __syncthreads();
+  if (KL >= 4 && k > uint32_t(R) && tid >= blockDim.x >> (k - R))
+    return;
+  typename NV<T>::type x[U];
+  uint32_t a[U];
+#pragma unroll
+  for (int c = 0; c < U; ++c) {
+    a[c] = at;
+#pragma unroll
+    for (int b = 0; b < LU; ++b)
+      a[c] ^= c >> b & 1 ? g.off2[1 + b] : 0u;
+    x[c] = lds_get<T>(lds, a[c]);
+  }
+#pragma unroll
+  for (int c = 0; c < U; ++c)
+    lds_put<T>(lds, a[c], times<T>(x[c], e.x, e.y));
 }
 
 // The 16-byte units of a thread: unit i * threads + tid of a tile, i < 2^RU.
@@ -559,6 +608,18 @@ template <typename T, int RU> struct TileUnits {
   }
 };
 
+template <typename G> __device__ __forceinline__ GroupGate fetch(G &from) {
+  GroupGate g;
+  g.mat = from.mat;
+  g.cols = from.cols;
+#pragma unroll
+  for (int i = 0; i < 7; ++i)
+    g.off2[i] = from.off2[i];
+  g.k = from.k;
+  g.kind = from.kind;
+  return g;
+}
+
 // R amplitude bits per thread.  The gate functions begin with the barrier that
 // orders them after the previous gate; what they need from global memory is
 // requested before it.
@@ -579,9 +640,31 @@ __device__ __forceinline__ void run_group(T *sv, H &a, G *gates, unsigned char *
     for (int i = 0; i < Units::N; ++i)
       *reinterpret_cast<Unit *>(lds + t.local(i)) = x[i];
   }
+  // The next descriptor is requested a gate ahead.
+  GroupGate ahead = fetch(gates[0]);
+  asm volatile("" ::"s"(ahead.kind)); // arrived: the loop's first wait is not for the next one
   for (uint32_t gi = 0; gi < a.n_gates; ++gi) {
-    G &g = gates[gi];
-    if (g.kind != kDense) {
+    const GroupGate g = ahead;
+    ahead = fetch(gates[gi + 1 < a.n_gates ? gi + 1 : gi]);
+    if (g.kind == kPhase) {
+      switch (g.k) {
+      case 1:
+        phase_gate<T, R, 1>(lds, g, tid, 1);
+        break;
+      case 2:
+        phase_gate<T, R, 2>(lds, g, tid, 2);
+        break;
+      case 3:
+        phase_gate<T, R, 3>(lds, g, tid, 3);
+        break;
+      case 4:
+        phase_gate<T, R, 4>(lds, g, tid, 4);
+        break;
+      default:
+        phase_gate<T, R, 6>(lds, g, tid, g.k);
+        break;
+      }
+    } else if (g.kind != kDense) {
       switch (g.k) {
       case 1:
         monomial_gate<T, R, 1>(lds, g, tid);
@@ -864,12 +947,36 @@ void describe_group(const GatePlan *const *plans, size_t n_plans, uint32_t n, Gr
     g = {};
     const bool diag = mono && is_diagonal(p);
     const bool mfma = !mono && p.k >= 4;
-    g.mat = mfma ? p.d_op : p.d_mat;
+    g.mat = mfma || mono ? p.d_op : p.d_mat;
     g.k = p.k;
     g.kind = mono ? (diag ? kDiagonal : kPermutation) : kDense;
     uint32_t used = 0;
     for (uint32_t b = 0; b < p.k; ++b)
       used |= 1u << local[p.q[b]];
+    if (diag && p.n_active == 1) {
+      // (identity entries take no part, so the row is not the identity's)
+      g.kind = kPhase;
+      uint64_t part[2] = {};
+      const float fl[2] = {float(p.act_re[0]), float(p.act_im[0])};
+      for (int x = 0; x < 2; ++x)
+        f32 ? std::memcpy(&part[x], &fl[x], 4)
+            : std::memcpy(&part[x], x ? &p.act_im[0] : &p.act_re[0], 8);
+      g.mat = reinterpret_cast<const void *>(uintptr_t(part[0]));
+      g.off2[5] = uint32_t(part[1]);
+      g.off2[6] = uint32_t(part[1] >> 32);
+      for (uint32_t b = 0; b < p.k; ++b) {
+        g.cols |= uint64_t(local[p.q[b]]) << (4 * b);
+        g.off2[0] ^= p.act_row[0] >> b & 1u ? bit_offset(local[p.q[b]], f32) : 0u;
+      }
+      uint32_t free_bit = 0;
+      for (uint32_t b = 0; b < m; ++b)
+        if (!(used >> b & 1u)) {
+          if (free_bit >= a.thread_bits && free_bit - a.thread_bits < 4)
+            g.off2[1 + free_bit - a.thread_bits] = bit_offset(b, f32);
+          ++free_bit;
+        }
+      continue;
+    }
     if (mono && p.k <= 4) {
       for (uint32_t r = 0; r < (1u << p.k); ++r)
         g.cols |= uint64_t(r) << (4 * r);
