@@ -39,10 +39,16 @@ constexpr int kMaxPairs = 32;
 constexpr int kMaxBlock = 512;
 constexpr int kMaxWaves = kMaxBlock / 64;
 constexpr uint32_t kMaxTrajGateQubits = 6; // 4 at f64
-// Workgroups a step is cut into, eight rounds of the CUs: 188 tasks of 20
-// qubits at f32 (3708 gates) take 20.2 ms in 512, 17.8 in 1024, 17.0 in 2048
-// and in 4096 workgroups of 512 threads (256 threads: 0.5 to 2 ms more).
-constexpr uint32_t kStepGroups = 2048;
+// A step is cut into this many workgroups of at most 256 threads: two share a
+// CU, so that one stages its operands while the other multiplies.  Several
+// rounds of the CUs even out gates of different size; f32 stages operands per
+// workgroup, so fewer.  188 tasks of 20 qubits, ms in 2048, 4096, 8192 groups:
+// f32 15.4, 14.9, 15.0 (512 threads 15.8, 15.9, 16.5), f64 38.8, 37.5, 36.0
+// (512: 38.1, 36.6, 36.1); 128 threads 16.4-18.6 and 38.1-42.0.
+template <typename T> constexpr uint32_t kStepGroups = sizeof(T) == 4 ? 4096 : 8192;
+constexpr uint32_t kStepBlock = 256;
+// ... and the closing sums into this many.
+constexpr uint32_t kSumGroups = 2048;
 
 // Layouts the host bindings rely on (no padding surprises across compilers).
 static_assert(sizeof(cast_hip_traj_gate_t) == 12, "cast_hip_traj_gate_t layout");
@@ -654,8 +660,8 @@ __global__ void __launch_bounds__(kMaxBlock, OCC)
 // owns a statevector (k_traj) is held to what one CU can do, and the launch to
 // its longest task: 188 tasks of 20 qubits and up to 40 gates at f32 took
 // 29.4 ms with 0.73 ms per gate on each of 188 CUs.  With a launch per step all
-// CUs share the tasks that are left: 15.7 ms (4.2 us per gate of 16.8 MB moved,
-// 4.0 TB/s, k = 5 and 6 bound by the split products), 32 tasks 23.6 -> 3.9 ms.
+// CUs share the tasks that are left: 14.9 ms (3.9 us per gate of 16.8 MB moved,
+// 4.3 TB/s, k = 5 and 6 bound by the split products), 32 tasks 23.6 -> 2.7 ms.
 // Each amplitude goes through the same operations as in k_traj.
 template <typename T, int OCC>
 __global__ void __launch_bounds__(kMaxBlock, OCC)
@@ -755,7 +761,7 @@ void launch_steps_t(const cast_hip_traj_launch_t &L, const TrajScalars &a, const
   const T *ckpt = reinterpret_cast<const T *>(L.checkpoints);
   T *slots = reinterpret_cast<T *>(L.slots);
   uint32_t *work = reinterpret_cast<uint32_t *>(L.work);
-  const uint32_t waves = L.block / 64;
+  const uint32_t block = std::min(L.block, kStepBlock), waves = block / 64;
   // At most as many parts as leave every wave a k = 6 tile of 2^10 amplitudes.
   const uint32_t most =
       L.n_qubits > 10 ? std::max(1u, (1u << std::min(L.n_qubits - 10, 20u)) / waves) : 1u;
@@ -763,7 +769,7 @@ void launch_steps_t(const cast_hip_traj_launch_t &L, const TrajScalars &a, const
   auto parts_of = [&](uint32_t tasks_here) {
     const uint32_t rows = observe_rows(L.n_qubits, a.log2_block);
     uint32_t parts = 1;
-    while (parts * tasks_here < kStepGroups && rows / (2 * parts) >= 64)
+    while (parts * tasks_here < kSumGroups && rows / (2 * parts) >= 64)
       parts *= 2;
     return parts;
   };
@@ -774,8 +780,8 @@ void launch_steps_t(const cast_hip_traj_launch_t &L, const TrajScalars &a, const
     for (uint32_t g = 0; g < n_steps; ++g) {
       while (n_gates[first + active - 1] <= g)
         --active;
-      const uint32_t parts = std::min(most, std::max(1u, kStepGroups / active));
-      hipLaunchKernelGGL((k_traj_step<T, OCC>), dim3(active * parts), dim3(L.block), 0, s, tasks,
+      const uint32_t parts = std::min(most, std::max(1u, kStepGroups<T> / active));
+      hipLaunchKernelGGL((k_traj_step<T, OCC>), dim3(active * parts), dim3(block), 0, s, tasks,
                          order, gates, mats, ckpt, slots, work, a, first, g, parts);
       check(hipGetLastError(), "hipLaunchKernelGGL(k_traj_step)");
     }

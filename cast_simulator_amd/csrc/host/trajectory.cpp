@@ -587,10 +587,11 @@ TrajectoryPlan TrajectoryEngine::plan(const std::vector<TrajectorySample> &sampl
 // as long as its busiest slot; `load` below is that against gates shared evenly
 // by the CUs.  Steps read and write every state from memory, where a slot of
 // the persistent launch may stay in the caches, and cost a launch each.
-// Measured, persistent -> steps: 20 qubits f32 load 18 23.6 -> 4.4 ms, 2.8
-// 29.7 -> 17.1, 1.2 51.5 -> 53.8; 18 qubits f32 load 3.0 6.2 -> 4.2, 1.1
-// 11.9 -> 13.6; 16 qubits f32 load 20 1.5 -> 0.7, 3.5 1.9 -> 1.6, 1.2 3.0 -> 4.8;
-// 14 qubits f32 load 23 0.42 -> 0.53, f64 load 4.1 0.92 -> 0.93.
+// Measured with steps of 512 threads, persistent -> steps: 20 qubits f32 load
+// 18 23.6 -> 4.4 ms, 2.8 29.7 -> 17.1, 1.2 51.5 -> 53.8; 18 qubits f32 load
+// 3.0 6.2 -> 4.2, 1.1 11.9 -> 13.6; 16 qubits f32 load 20 1.5 -> 0.7, 3.5
+// 1.9 -> 1.6, 1.2 3.0 -> 4.8; 14 qubits f32 load 23 0.42 -> 0.53, f64 load 4.1
+// 0.92 -> 0.93.
 static bool steps_pay(const std::vector<uint32_t> &lengths, uint32_t n_slots, uint32_t n_cu,
                       size_t sv_bytes) {
   if (sv_bytes < (size_t(512) << 10))
