@@ -451,7 +451,7 @@ HipKernelManager::launch_shared_locked(const std::vector<Pending> &work,
       for (size_t i : list)
         plans.push_back(work[i].base);
       bool join = true;
-      const auto passes = plan_passes(plans, n, &join);
+      const auto passes = plan_passes(plans, n, join);
       if (!join) {
         rest.push_back(std::move(list));
         continue;

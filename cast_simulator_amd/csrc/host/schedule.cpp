@@ -87,18 +87,18 @@ bool PassPlanner::next(std::vector<uint32_t> &pass) {
   return true;
 }
 
-std::vector<std::vector<uint32_t>> plan_passes(const std::vector<const void *> &plans,
-                                               uint32_t n_qubits, bool *all_join) {
+namespace {
+PassPlanner planner_of(const std::vector<const void *> &plans, uint32_t n_qubits, bool &all_join) {
   char err[kErr];
   std::vector<PlannedGate> gates(plans.size());
   PassLimits lim;
-  bool join = true;
+  all_join = true;
   for (size_t i = 0; i < plans.size(); ++i) {
     cast_hip_group_info_t info{};
     throw_if(cast_hip_gate_group_info(plans[i], n_qubits, &info, err, kErr), err);
     gates[i].qubits = info.targets;
     gates[i].may_join = info.targets != 0;
-    join = join && gates[i].may_join;
+    all_join = all_join && gates[i].may_join;
     if (gates[i].may_join) {
       lim = {n_qubits, info.max_qubits, info.low_qubits, info.max_gates};
       continue;
@@ -108,10 +108,14 @@ std::vector<std::vector<uint32_t>> plan_passes(const std::vector<const void *> &
     for (uint32_t b = 0; b < p.n_qubits; ++b)
       gates[i].qubits |= uint64_t(1) << p.qubits[b];
   }
-  if (all_join)
-    *all_join = join;
   lim.n_qubits = n_qubits;
-  PassPlanner planner(std::move(gates), lim);
+  return PassPlanner(std::move(gates), lim);
+}
+} // namespace
+
+std::vector<std::vector<uint32_t>> plan_passes(const std::vector<const void *> &plans,
+                                               uint32_t n_qubits, bool &all_join) {
+  PassPlanner planner = planner_of(plans, n_qubits, all_join);
   std::vector<std::vector<uint32_t>> passes;
   std::vector<uint32_t> pass;
   while (planner.next(pass))
@@ -122,8 +126,11 @@ std::vector<std::vector<uint32_t>> plan_passes(const std::vector<const void *> &
 void apply_in_passes(const std::vector<const void *> &plans, void *stream, uint64_t sv_dptr,
                      uint32_t n_qubits, const std::function<void(uint32_t)> &single) {
   char err[kErr];
+  bool all_join;
+  PassPlanner planner = planner_of(plans, n_qubits, all_join);
+  std::vector<uint32_t> pass;
   std::vector<const void *> group;
-  for (const auto &pass : plan_passes(plans, n_qubits, nullptr)) {
+  while (planner.next(pass)) { // the device works on a pass while the next is planned
     if (pass.size() == 1) {
       single(pass[0]);
       continue;

@@ -44,10 +44,10 @@ private:
   std::vector<uint32_t> left_; // not yet in a pass, in order
 };
 
-// The passes of `plans` on one statevector, as indices; `all_join` (may be
-// null): whether every gate can run in a group.
+// The passes of `plans` on one statevector, as indices; `all_join`:
+// whether every gate can run in a group.
 std::vector<std::vector<uint32_t>> plan_passes(const std::vector<const void *> &plans,
-                                               uint32_t n_qubits, bool *all_join);
+                                               uint32_t n_qubits, bool &all_join);
 
 // Enqueues `plans` in order on `stream`, the groups that the planner finds as
 // one pass each and every other gate i by `single(i)`.
