@@ -106,14 +106,15 @@ def run_gpu(cs, n: int, precision: str, steps: int, warmup: int, max_size: int):
     ctype = "double" if precision == "f64" else "float"
 
     def symbol(kid):
-        """Kernel symbol as the profiler names it."""
+        """Kernel symbol as the profiler names it, without the load mode (the
+        last argument of k_dense and k_mfma; the traffic record has none)."""
         k, f = info[kid].k, fam[kid]
         if f in (3, 5, 6, 7, 8, 9, 13, 14):
             low = sum(1 for q in info[kid].qubits if q < 6)
             return (f"k_tile3<{ctype}, {k}, {low}>" if f in (6, 7, 9, 14)
                     else f"k_tile<{ctype}, {k}, {low}>")
         if f == 1:  # dense: the store mode is a template argument
-            nts = precision == "f64" and min(info[kid].qubits) >= 3
+            nts = precision == "f64" and n > 24 and min(info[kid].qubits) >= 3
             return f"k_dense<{ctype}, {k}, {'true' if nts else 'false'}>"
         return mfma_symbol(f, ctype, k)
 

@@ -585,16 +585,28 @@ TrajectoryPlan TrajectoryEngine::plan(const std::vector<TrajectorySample> &sampl
 // Whether a launch per gate step (every CU on the tasks that are left) beats
 // the persistent launch (a workgroup per slot, whole tasks).  The latter takes
 // as long as its busiest slot; `load` below is that against gates shared evenly
-// by the CUs.  Steps read and write every state from memory, where a slot of
-// the persistent launch may stay in the caches, and cost a launch each.
-// Measured with steps of 512 threads, persistent -> steps: 20 qubits f32 load
-// 18 23.6 -> 4.4 ms, 2.8 29.7 -> 17.1, 1.2 51.5 -> 53.8; 18 qubits f32 load
-// 3.0 6.2 -> 4.2, 1.1 11.9 -> 13.6; 16 qubits f32 load 20 1.5 -> 0.7, 3.5
-// 1.9 -> 1.6, 1.2 3.0 -> 4.8; 14 qubits f32 load 23 0.42 -> 0.53, f64 load 4.1
-// 0.92 -> 0.93.
+// by the CUs.  Steps read and write every state from memory, where a small
+// slot of the persistent launch stays in the caches, and cost a launch each.
+// Measured, persistent -> steps in ms, by statevector (number of tasks):
+//   128 MiB f32 (294) 632 -> 547; 8 MiB f32 (188) 29.4 -> 14.9, (270) 34.2 ->
+//   27.5, (496) 50.9 -> 49.1, (1426) 133.8 -> 133.4; 16 MiB f64 (496) 128 -> 124;
+//   2 MiB f32 (174) 6.0 -> 3.7, (271) 7.4 -> 6.6, (491) 11.6 -> 12.4;
+//   512 KiB f32 (157) 1.84 -> 1.50, (482) 2.9 -> 4.3; 1 MiB f64 (157) 3.4 -> 2.2;
+//   256 KiB (28) f32 0.72 -> 0.49, f64 0.96 -> 0.71, (144) f32 0.75 -> 0.90;
+//   128 KiB f32 (28) 0.42 -> 0.47.
 static bool steps_pay(const std::vector<uint32_t> &lengths, uint32_t n_slots, uint32_t n_cu,
                       size_t sv_bytes) {
-  if (sv_bytes < (size_t(512) << 10))
+  constexpr struct {
+    size_t kib;
+    double load;
+  } kLines[] = {{8192, 1.05}, {2048, 1.6}, {512, 3.0}, {256, 8.0}};
+  double need = 0.0;
+  for (const auto &l : kLines)
+    if (sv_bytes >= l.kib << 10) {
+      need = l.load;
+      break;
+    }
+  if (need == 0.0)
     return false;
   // The slots take the tasks in order, each when it is free.
   std::priority_queue<uint64_t, std::vector<uint64_t>, std::greater<uint64_t>> busy;
@@ -610,11 +622,16 @@ static bool steps_pay(const std::vector<uint32_t> &lengths, uint32_t n_slots, ui
     total += g;
   }
   const double load = total ? double(longest) * double(n_cu) / double(total) : 0.0;
-  return load >= (sv_bytes < (size_t(2) << 20) ? 3.0 : 2.0);
+  return load >= need;
 }
 
 TrajectoryRun TrajectoryEngine::run(const std::vector<TrajectorySample> &samples,
                                     const TrajectoryTuning &tn, bool dump) {
+  return run_tasks(samples, tn, dump, true);
+}
+
+TrajectoryRun TrajectoryEngine::run_tasks(const std::vector<TrajectorySample> &samples,
+                                          const TrajectoryTuning &tn, bool dump, bool may_step) {
   const double t_start = now_s();
   const uint32_t B = tn.chunk_layers;
   TrajectoryPlan P = plan(samples, tn);
@@ -741,7 +758,7 @@ TrajectoryRun TrajectoryEngine::run(const std::vector<TrajectorySample> &samples
   float ms = 0.f;
   int rc = cast_hip_event_record(e0, s, err, kErr);
   if (rc == 0)
-    rc = steps_pay(lengths, uint32_t(n_slots), std::max(1u, info.n_cu), svb)
+    rc = may_step && steps_pay(lengths, uint32_t(n_slots), std::max(1u, info.n_cu), svb)
              ? cast_hip_traj_run_steps(&L, lengths.data(), s, err, kErr)
              : cast_hip_traj_run(&L, s, err, kErr);
   if (rc == 0)
@@ -813,7 +830,7 @@ TrajectoryTuning TrajectoryEngine::autotune(const std::vector<TrajectorySample> 
   auto trial = [&](const TrajectoryTuning &t) {
     // Checkpoints are part of the cost of a chunk size: time them too.
     ckpt_chunk_ = 0;
-    const TrajectoryRun r = run(sample, t);
+    const TrajectoryRun r = run_tasks(sample, t, false, false);
     const double s = r.total_s / double(sample.size());
     if (log)
       log->push_back({t, s});

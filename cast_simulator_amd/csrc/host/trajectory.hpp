@@ -168,12 +168,18 @@ public:
   // Project-written autotuner: coordinate search over the launch shape
   // (block, slots per CU) and then the planning knobs (chunk layers, fusion
   // size), each candidate timed end to end (plan + checkpoints + launch) on
-  // `sample`.  Returns the best tuning; `log` receives every trial.
+  // `sample`, in the persistent launch: a sample has fewer tasks than the batch
+  // it stands for, and the steps that few tasks take do not show what a shape
+  // costs there.  Returns the best tuning; `log` receives every trial.
   TrajectoryTuning autotune(const std::vector<TrajectorySample> &sample,
                             const TrajectoryTuning &start,
                             std::vector<TrajectoryTuneRecord> *log = nullptr);
 
 private:
+  // `may_step`: whether few tasks may take the launch per gate step.
+  TrajectoryRun run_tasks(const std::vector<TrajectorySample> &samples, const TrajectoryTuning &t,
+                          bool dump, bool may_step);
+
   struct FusedGate {
     std::vector<uint32_t> qubits;
     ComplexSquareMatrix m;

@@ -25,7 +25,7 @@ import argparse
 import csv
 from collections import OrderedDict, defaultdict
 
-GATE_KERNELS = ("k_tile", "k_mfma", "k_dense", "k_monomial")
+GATE_KERNELS = ("k_tile", "k_mfma", "k_dense", "k_monomial", "k_diagonal")
 
 
 def _short(name: str) -> str:
