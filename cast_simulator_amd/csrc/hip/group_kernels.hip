@@ -811,19 +811,26 @@ size_t group_operand_bytes(uint32_t k, uint8_t precision) {
 }
 
 namespace {
-// Round to nearest even, as the device's conversion does (finite values).
-uint16_t to_bf16(float x) {
-  uint32_t b;
-  std::memcpy(&b, &x, 4);
-  if ((b & 0x7fffffffu) > 0x7f800000u)
-    return uint16_t(b >> 16 | 0x40u); // NaN
-  return uint16_t((b + 0x7fffu + (b >> 16 & 1u)) >> 16);
-}
-float from_bf16(uint16_t h) {
-  const uint32_t b = uint32_t(h) << 16;
-  float x;
-  std::memcpy(&x, &b, 4);
-  return x;
+// The bf16 parts of 8 values, each rounded to nearest even as the device's
+// conversion does (without branches, for the vectoriser).
+void split8(const float *x, uint16_t out[3][8]) {
+  float rest[8];
+  std::memcpy(rest, x, sizeof(rest));
+  for (int s = 0; s < 3; ++s) {
+    uint32_t b[8], h[8];
+    float part[8];
+    std::memcpy(b, rest, sizeof(b));
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t nan = b[e] | 0x400000u, round = b[e] + 0x7fffu + (b[e] >> 16 & 1u);
+      // magnitudes are positive as signed numbers
+      h[e] = (int32_t(b[e] & 0x7fffffffu) > 0x7f800000 ? nan : round) & 0xffff0000u;
+    }
+    std::memcpy(part, h, sizeof(part));
+    for (int e = 0; e < 8; ++e)
+      rest[e] -= part[e];
+    for (int e = 0; e < 8; ++e)
+      out[s][e] = uint16_t(h[e] >> 16);
+  }
 }
 } // namespace
 
@@ -853,24 +860,25 @@ void group_operands(const double *m, uint32_t k, uint8_t precision, void *out) {
               float(x == 0 ? re(r, c) : x == 1 ? im(r, c) : re(r, c) + im(r, c));
         }
   } else {
-    uint16_t *h = static_cast<uint16_t *>(out);
+    unsigned char *h = static_cast<unsigned char *>(out);
     const uint32_t n_ks = K / 32;
-    for (uint32_t x = 0; x < 2; ++x)
+    std::vector<float> part(K * K);
+    for (uint32_t x = 0; x < 2; ++x) {
+      for (uint32_t i = 0; i < K * K; ++i)
+        part[i] = float(m[2 * i + x]);
       for (uint32_t rb = 0; rb < RB; ++rb)
         for (uint32_t ks = 0; ks < n_ks; ++ks)
-          for (uint32_t l = 0; l < 64; ++l)
-            for (uint32_t e = 0; e < 8; ++e) {
-              const uint32_t r = 16 * rb + (l & 15u), c = 32 * ks + 8 * (l >> 4) + e;
-              float rest = float(x == 0 ? re(r, c) : im(r, c));
-              for (uint32_t s = 0; s < 3; ++s) {
-                const uint16_t b = to_bf16(rest);
-                const size_t at = size_t(
-                    k == 5 ? dev::SplitOperands<5>::at(int(x), int(s), int(rb), int(ks))
-                           : dev::SplitOperands<6>::at(int(x), int(s), int(rb), int(ks)));
-                h[(at + l) * 8 + e] = b;
-                rest -= from_bf16(b);
-              }
+          for (uint32_t l = 0; l < 64; ++l) {
+            uint16_t b[3][8];
+            split8(&part[(16 * rb + (l & 15u)) * K + 32 * ks + 8 * (l >> 4)], b);
+            for (uint32_t s = 0; s < 3; ++s) {
+              const int at = k == 5
+                                 ? dev::SplitOperands<5>::at(int(x), int(s), int(rb), int(ks))
+                                 : dev::SplitOperands<6>::at(int(x), int(s), int(rb), int(ks));
+              std::memcpy(h + (size_t(at) + l) * 16, b[s], 16);
             }
+          }
+    }
   }
 }
 
