@@ -31,9 +31,10 @@
 // ms (matrix cores alone 1.3 and 2.6 for k = 4, 5), where its own pass would
 // take 5.9-6.5.  Measured and not kept: tiles of 2^11 (379 ms against 350 for
 // 90 gates), workgroups that stay and fetch their next tile during the gates
-// (409 against 372 then), operands in LDS instead of in registers (the same
-// time), one workgroup per CU (474-540), wave priorities and staggered starts
-// (no change).
+// (409 against 372 then; one of 512 threads per CU with all operands in LDS,
+// so that no gate waits for the tile fetch, 379 against 339), operands in LDS
+// instead of in registers (the same time), one workgroup per CU (474-540), wave
+// priorities and staggered starts (no change).
 
 #include "cast_hip.h"
 #include "common.hpp"
