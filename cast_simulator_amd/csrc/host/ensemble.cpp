@@ -154,17 +154,20 @@ TrajectoryResult Simulator::sample_trajectory(const CircuitGraph &graph,
 
   // Ensemble (trajectory.rs:186-265).
   const size_t max_ensemble = std::max<size_t>(1, opts.max_ensemble);
-  std::vector<Member> ens;
+  std::vector<Member> ens, next;     // next: the members after the gate at hand
   std::vector<HipStatevector> spare; // of members that were dropped
-  // No gate stays queued for a member that is gone, also when this throws.
+  // No gate stays queued for a member that is gone, also when this throws:
+  // then members may be in either list.
   struct Unqueue {
     HipKernelManager &mgr;
-    std::vector<Member> &ens;
+    const std::vector<Member> &ens, &next;
     ~Unqueue() {
-      for (const Member &m : ens)
-        mgr.discard(m.sv.dptr());
+      for (const auto *list : {&ens, &next})
+        for (const Member &m : *list)
+          if (m.sv.dptr()) // not moved on
+            mgr.discard(m.sv.dptr());
     }
-  } unqueue{mgr_, ens};
+  } unqueue{mgr_, ens, next};
   // The state without its queued gates, copied on the manager's stream.
   auto copy_of = [&](const HipStatevector &sv) {
     HipStatevector to = spare.empty() ? HipStatevector(n_physical, spec_.precision)
@@ -221,20 +224,22 @@ TrajectoryResult Simulator::sample_trajectory(const CircuitGraph &graph,
         mgr_.discard(ens[m].sv.dptr());
         spare.push_back(std::move(ens[m].sv));
       }
-    std::vector<Member> next;
+    next.clear();
     next.reserve(kept);
     std::vector<size_t> moved(ens.size(), kept); // a moved member's place in next
     for (const auto &c : cand) {
       Member &parent = ens[c.member];
+      std::vector<size_t> path = parent.path;
+      path.push_back(c.branch);
       // The member's own buffer goes to its first candidate; every other one
       // copies the state as it is before this gate.
       if (moved[c.member] == kept) {
         moved[c.member] = next.size();
-        next.push_back(Member{std::move(parent.sv), c.weight, parent.path});
+        next.push_back(Member{std::move(parent.sv), c.weight, std::move(path)});
       } else {
-        next.push_back(Member{copy_of(next[moved[c.member]].sv), c.weight, parent.path});
+        next.push_back(
+            Member{copy_of(next[moved[c.member]].sv), c.weight, std::move(path)});
       }
-      next.back().path.push_back(c.branch);
     }
     ens = std::move(next);
     for (size_t x = 0; x < kept; ++x)
