@@ -49,6 +49,8 @@ template <typename T> constexpr uint32_t kStepGroups = sizeof(T) == 4 ? 4096 : 8
 constexpr uint32_t kStepBlock = 256;
 // ... and the closing sums into this many.
 constexpr uint32_t kSumGroups = 2048;
+// Host lengths of tasks that k_traj_lengths takes, in its arguments (4 KiB at most).
+constexpr uint32_t kMaxLengths = 960;
 
 // Layouts the host bindings rely on (no padding surprises across compilers).
 static_assert(sizeof(cast_hip_traj_gate_t) == 12, "cast_hip_traj_gate_t layout");
@@ -687,16 +689,16 @@ __global__ void __launch_bounds__(kMaxBlock, OCC)
 }
 
 // Sums and dump of the tasks order[first ...) after their last step, `parts`
-// workgroups each.  With several, a part leaves its sums at the start of the range of the
-// slot that it alone has read (or that holds nothing, for a task without
-// gates); k_traj_sum adds them up.  A task with more gates than `n_steps` is an
-// error.  188 states of 20 qubits, f32: 1.1 ms in one part, 0.56 in eight.
+// workgroups each.  With several, a part leaves its sums at the start of the
+// range of the slot that it alone has read (or that holds nothing, for a task
+// without gates); k_traj_sum adds them up.  188 states of 20 qubits, f32: 1.1
+// ms in one part, 0.56 in eight.
 template <typename T>
 __global__ void __launch_bounds__(kMaxBlock, 2)
     k_traj_finish(const cast_hip_traj_task_t *__restrict__ tasks,
                   const uint32_t *__restrict__ order, const T *__restrict__ checkpoints, T *slots,
                   double *__restrict__ out, T *__restrict__ dump, uint32_t *__restrict__ work,
-                  TrajScalars a, uint32_t first, uint32_t n_steps, uint32_t parts) {
+                  TrajScalars a, uint32_t first, uint32_t parts) {
   __shared__ uint32_t s_pairs[2 * kMaxPairs];
   __shared__ double red[kMaxWaves * (1 + kMaxPairs)];
   if (threadIdx.x < 2 * a.n_pairs)
@@ -707,8 +709,6 @@ __global__ void __launch_bounds__(kMaxBlock, 2)
   cast_hip_traj_task_t task{};
   if (!fetch_task(tasks, order, first + slot_i, work, a, ti, task))
     return;
-  if (task.n_gates > n_steps)
-    atomicOr(&work[1], 1u);
   const uint64_t len = uint64_t(1) << a.n_qubits, mine = len / parts;
   T *slot = slots + 2 * len * slot_i;
   const T *cur = task.n_gates == 0 ? checkpoints + 2 * len * task.checkpoint : slot;
@@ -722,6 +722,24 @@ __global__ void __launch_bounds__(kMaxBlock, 2)
                             : reinterpret_cast<double *>(slot + 2 * mine * part);
   wg_observe<T>(cur, a.n_qubits, a.n_pairs, a.log2_block, s_pairs, n_rows * part, n_rows, sums,
                 red);
+}
+
+// Sets the error flag for tasks of order[first ...) with more gates than the
+// host says: these gates would be left out, since the steps follow the host's
+// lengths.  One launch a run (about 3 us) for every 960 tasks.
+struct TrajLengths {
+  uint32_t n;
+  uint32_t n_gates[kMaxLengths];
+};
+__global__ void __launch_bounds__(256)
+    k_traj_lengths(const cast_hip_traj_task_t *__restrict__ tasks,
+                   const uint32_t *__restrict__ order, uint32_t n_tasks, uint32_t first,
+                   uint32_t *__restrict__ work, TrajLengths a) {
+  for (uint32_t i = threadIdx.x; i < a.n; i += blockDim.x) {
+    const uint32_t ti = order[first + i];
+    if (ti < n_tasks && tasks[ti].n_gates > a.n_gates[i])
+      atomicOr(&work[1], 1u);
+  }
 }
 
 template <typename T>
@@ -773,6 +791,14 @@ void launch_steps_t(const cast_hip_traj_launch_t &L, const TrajScalars &a, const
       parts *= 2;
     return parts;
   };
+  for (uint32_t first = 0; first < L.n_tasks; first += kMaxLengths) {
+    TrajLengths lengths;
+    lengths.n = std::min(kMaxLengths, L.n_tasks - first);
+    std::copy_n(n_gates + first, lengths.n, lengths.n_gates);
+    hipLaunchKernelGGL(k_traj_lengths, dim3(1), dim3(256), 0, s, tasks, order, L.n_tasks, first,
+                       work, lengths);
+    check(hipGetLastError(), "hipLaunchKernelGGL(k_traj_lengths)");
+  }
   for (uint32_t first = 0; first < L.n_tasks; first += L.n_slots) {
     const uint32_t here = std::min(L.n_slots, L.n_tasks - first);
     uint32_t active = here;
@@ -788,7 +814,7 @@ void launch_steps_t(const cast_hip_traj_launch_t &L, const TrajScalars &a, const
     const uint32_t parts = parts_of(here);
     hipLaunchKernelGGL((k_traj_finish<T>), dim3(here * parts), dim3(L.block), 0, s, tasks, order,
                        ckpt, slots, reinterpret_cast<double *>(L.out),
-                       reinterpret_cast<T *>(L.dump), work, a, first, n_steps, parts);
+                       reinterpret_cast<T *>(L.dump), work, a, first, parts);
     check(hipGetLastError(), "hipLaunchKernelGGL(k_traj_finish)");
     if (parts == 1)
       continue;

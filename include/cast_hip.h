@@ -444,7 +444,7 @@ int cast_hip_traj_run(const cast_hip_traj_launch_t *args, void *stream, char *er
  * task: rounds of n_slots tasks of the order, step g applying gate g of every
  * task that has one, each statevector shared by many workgroups.  n_gates[t]
  * (host, not increasing) is the length of the task order[t].  A task whose
- * device length exceeds the first n_gates of its round sets the error flag.
+ * device length exceeds it sets the error flag (its results are then void).
  * The slots hold no states afterwards (take those from `dump`). */
 int cast_hip_traj_run_steps(const cast_hip_traj_launch_t *args, const uint32_t *n_gates,
                             void *stream, char *err_buf, size_t err_buf_len);
