@@ -280,26 +280,29 @@ void HipKernelManager::apply(KernelId id, HipStatevector &sv) {
     throw Error("statevector precision does not match kernel precision");
   if (info.qubits[info.n_qubits - 1] >= sv.n_qubits())
     throw Error("gate acts on a qubit outside the statevector");
-  const void *plan = it->second, *base = it->second;
-  int cand = -1;
   // Tuning applies to dense plans of the automatic family on large states.
-  if (autotune_ && spec_.variant == CAST_HIP_VARIANT_AUTO && sv.n_qubits() >= tune_min_qubits_ &&
-      info.variant != CAST_HIP_VARIANT_MONOMIAL) {
-    TuneState &st = tune_state_locked(id, sv.n_qubits());
-    if (st.chosen >= 0) {
-      plan = st.plans[size_t(st.chosen)];
-    } else {
-      // the surviving candidate with the fewest timings
-      size_t best = st.samples.size();
-      for (size_t c = 0; c < st.samples.size(); ++c)
-        if (!st.dropped[c] &&
-            (best == st.samples.size() || st.samples[c].size() < st.samples[best].size()))
-          best = c;
-      cand = int(best);
-      plan = st.plans[best];
-    }
-  }
-  pending_.push_back({id, sv.dptr(), sv.n_qubits(), plan, base, cand});
+  const bool tune = autotune_ && spec_.variant == CAST_HIP_VARIANT_AUTO &&
+                    sv.n_qubits() >= tune_min_qubits_ &&
+                    info.variant != CAST_HIP_VARIANT_MONOMIAL;
+  pending_.push_back({id, sv.dptr(), sv.n_qubits(), it->second, tune, -1});
+}
+
+// Candidates are built and sampled only for gates that are launched by
+// themselves: a pass with other gates takes the gate's own plan.
+const void *HipKernelManager::single_plan_locked(Pending &w) {
+  if (!w.tune)
+    return w.plan;
+  TuneState &st = tune_state_locked(w.id, w.n_qubits);
+  if (st.chosen >= 0)
+    return st.plans[size_t(st.chosen)];
+  // the surviving candidate with the fewest timings
+  size_t best = st.samples.size();
+  for (size_t c = 0; c < st.samples.size(); ++c)
+    if (!st.dropped[c] &&
+        (best == st.samples.size() || st.samples[c].size() < st.samples[best].size()))
+      best = c;
+  w.cand = int(best);
+  return st.plans[best];
 }
 
 uint32_t HipKernelManager::tune(const std::vector<KernelId> &ids, HipStatevector &sv,
@@ -372,7 +375,7 @@ void *HipKernelManager::stream() {
 // Gates on different statevectors are independent, so each statevector's
 // gates are taken together, in their order, and cut into passes.  A forced
 // kernel variant keeps one launch per gate.
-void HipKernelManager::launch_passes_locked(const std::vector<Pending> &work,
+void HipKernelManager::launch_passes_locked(std::vector<Pending> &work,
                                             std::vector<size_t> &sampled) {
   char err[kErr];
   std::vector<std::vector<size_t>> lists;
@@ -390,12 +393,13 @@ void HipKernelManager::launch_passes_locked(const std::vector<Pending> &work,
     const uint64_t dptr = work[list[0]].dptr;
     const uint32_t n = work[list[0]].n_qubits;
     auto single = [&](uint32_t j) {
-      const Pending &w = work[list[j]];
+      Pending &w = work[list[j]];
+      const void *plan = single_plan_locked(w);
       if (w.cand >= 0) {
         ensure_events_locked(2 * sampled.size() + 2);
         throw_if(cast_hip_event_record(events_[2 * sampled.size()], stream_, err, kErr), err);
       }
-      throw_if(cast_hip_gate_apply(w.plan, stream_, dptr, n, err, kErr), err);
+      throw_if(cast_hip_gate_apply(plan, stream_, dptr, n, err, kErr), err);
       if (w.cand >= 0) {
         throw_if(cast_hip_event_record(events_[2 * sampled.size() + 1], stream_, err, kErr), err);
         sampled.push_back(list[j]);
@@ -408,7 +412,7 @@ void HipKernelManager::launch_passes_locked(const std::vector<Pending> &work,
     }
     plans.clear();
     for (size_t i : list)
-      plans.push_back(work[i].base);
+      plans.push_back(work[i].plan);
     apply_in_passes(plans, stream_, dptr, n, single);
   }
 }
@@ -425,11 +429,8 @@ HipKernelManager::launch_shared_locked(const std::vector<Pending> &work,
   for (auto &list : lists) {
     const Pending &w = work[list[0]];
     cast_hip_group_info_t info{};
-    throw_if(cast_hip_gate_group_info(w.base, w.n_qubits, &info, err, kErr), err);
-    bool tuning = false;
-    for (size_t i : list)
-      tuning = tuning || work[i].cand >= 0;
-    if (info.targets && w.n_qubits < info.max_qubits + 10 && !tuning)
+    throw_if(cast_hip_gate_group_info(w.plan, w.n_qubits, &info, err, kErr), err);
+    if (info.targets && w.n_qubits < info.max_qubits + 10)
       by_size[w.n_qubits].push_back(std::move(list));
     else
       rest.push_back(std::move(list));
@@ -449,7 +450,7 @@ HipKernelManager::launch_shared_locked(const std::vector<Pending> &work,
     for (auto &list : some) {
       std::vector<const void *> plans;
       for (size_t i : list)
-        plans.push_back(work[i].base);
+        plans.push_back(work[i].plan);
       bool join = true;
       const auto passes = plan_passes(plans, n, join);
       if (!join) {
@@ -500,26 +501,23 @@ HipKernelManager::launch_shared_locked(const std::vector<Pending> &work,
 }
 
 void HipKernelManager::launch(const std::vector<uint64_t> &svs) {
+  std::vector<Pending> work, keep;
+  std::vector<size_t> sampled;
+  std::vector<void *> ev;
   {
     std::lock_guard<std::mutex> lock(mu_);
-    std::vector<Pending> work, keep;
-    bool tuning = false;
-    for (const Pending &p : pending_) {
-      const bool mine = std::find(svs.begin(), svs.end(), p.dptr) != svs.end();
-      (mine ? work : keep).push_back(p);
-      tuning = tuning || (mine && p.cand >= 0);
-    }
+    for (const Pending &p : pending_)
+      (std::find(svs.begin(), svs.end(), p.dptr) != svs.end() ? work : keep).push_back(p);
     if (work.empty())
       return;
-    if (!tuning) {
-      ensure_stream_locked();
-      pending_.swap(keep);
-      std::vector<size_t> sampled;
-      launch_passes_locked(work, sampled);
+    ensure_stream_locked();
+    pending_.swap(keep);
+    launch_passes_locked(work, sampled);
+    if (sampled.empty())
       return;
-    }
+    ev.assign(events_.begin(), events_.begin() + long(2 * sampled.size()));
   }
-  sync(false); // tuning samples are read after a wait
+  take_samples(work, sampled, ev); // waits for them
 }
 
 void HipKernelManager::discard(uint64_t sv) {
@@ -527,6 +525,57 @@ void HipKernelManager::discard(uint64_t sv) {
   pending_.erase(std::remove_if(pending_.begin(), pending_.end(),
                                 [&](const Pending &p) { return p.dptr == sv; }),
                  pending_.end());
+}
+
+namespace {
+double elapsed_s(void *from, void *to) {
+  char err[kErr];
+  float ms = 0.f;
+  throw_if(cast_hip_event_elapsed_ms(from, to, &ms, err, kErr), err);
+  return double(ms) * 1e-3;
+}
+} // namespace
+
+void HipKernelManager::take_samples(const std::vector<Pending> &work,
+                                    const std::vector<size_t> &sampled,
+                                    const std::vector<void *> &ev) {
+  char err[kErr];
+  throw_if(cast_hip_event_synchronize(ev[2 * sampled.size() - 1], err, kErr), err);
+  for (size_t s = 0; s < sampled.size(); ++s)
+    add_sample(work[sampled[s]], elapsed_s(ev[2 * s], ev[2 * s + 1]));
+}
+
+void HipKernelManager::add_sample(const Pending &w, double seconds) {
+  std::lock_guard<std::mutex> lock(mu_);
+  auto it = tune_.find(std::make_pair(w.id, w.n_qubits));
+  if (it == tune_.end() || it->second.chosen >= 0)
+    return;
+  TuneState &ts = it->second;
+  ts.samples[size_t(w.cand)].push_back(seconds);
+  // best minimum so far; drop candidates beyond the margin
+  double best = 1e300;
+  size_t arg = 0;
+  for (size_t c = 0; c < ts.samples.size(); ++c)
+    if (!ts.dropped[c] && !ts.samples[c].empty()) {
+      const double m = *std::min_element(ts.samples[c].begin(), ts.samples[c].end());
+      if (m < best) {
+        best = m;
+        arg = c;
+      }
+    }
+  bool done = true;
+  for (size_t c = 0; c < ts.samples.size(); ++c) {
+    if (ts.dropped[c])
+      continue;
+    if (!ts.samples[c].empty() && c != arg &&
+        *std::min_element(ts.samples[c].begin(), ts.samples[c].end()) > kTuneMargin * best) {
+      ts.dropped[c] = 1;
+      continue;
+    }
+    done = done && ts.samples[c].size() >= tune_samples_;
+  }
+  if (done)
+    ts.chosen = int(arg);
 }
 
 SyncStats HipKernelManager::sync(bool timed) {
@@ -542,6 +591,12 @@ SyncStats HipKernelManager::sync(bool timed) {
       return empty;
     ensure_stream_locked();
     stream = stream_;
+    // Plans before the first event (building one between two events would be
+    // timed) and before the queue is taken (this may throw).
+    std::vector<const void *> plans;
+    if (timed)
+      for (Pending &w : pending_)
+        plans.push_back(single_plan_locked(w));
     work.swap(pending_);
     char err[kErr];
     if (timed) {
@@ -550,8 +605,7 @@ SyncStats HipKernelManager::sync(bool timed) {
       if (!work.empty())
         throw_if(cast_hip_event_record(ev[0], stream, err, kErr), err);
       for (size_t i = 0; i < work.size(); ++i) {
-        throw_if(cast_hip_gate_apply(work[i].plan, stream, work[i].dptr, work[i].n_qubits, err,
-                                     kErr),
+        throw_if(cast_hip_gate_apply(plans[i], stream, work[i].dptr, work[i].n_qubits, err, kErr),
                  err);
         throw_if(cast_hip_event_record(ev[i + 1], stream, err, kErr), err);
       }
@@ -563,55 +617,15 @@ SyncStats HipKernelManager::sync(bool timed) {
   char err[kErr];
   throw_if(cast_hip_stream_sync(stream, err, kErr), err);
   SyncStats st;
-  std::vector<std::pair<size_t, double>> samples; // (queue position, seconds)
-  auto elapsed = [&](size_t a) {
-    float ms = 0.f;
-    throw_if(cast_hip_event_elapsed_ms(ev[a], ev[a + 1], &ms, err, kErr), err);
-    return double(ms) * 1e-3;
-  };
   if (timed) {
     for (size_t i = 0; i < work.size(); ++i) {
-      st.kernels.push_back({work[i].id, elapsed(i)});
+      st.kernels.push_back({work[i].id, elapsed_s(ev[i], ev[i + 1])});
       if (work[i].cand >= 0)
-        samples.emplace_back(i, st.kernels.back().gpu_s);
+        add_sample(work[i], st.kernels.back().gpu_s);
     }
   }
-  for (size_t s = 0; s < sampled.size(); ++s)
-    samples.emplace_back(sampled[s], elapsed(2 * s));
-  if (!samples.empty()) {
-    std::lock_guard<std::mutex> lock(mu_);
-    for (const auto &[i, seconds] : samples) {
-      auto it = tune_.find(std::make_pair(work[i].id, work[i].n_qubits));
-      if (it == tune_.end() || it->second.chosen >= 0)
-        continue;
-      TuneState &ts = it->second;
-      ts.samples[size_t(work[i].cand)].push_back(seconds);
-      // best minimum so far; drop candidates beyond the margin
-      double best = 1e300;
-      size_t arg = 0;
-      for (size_t c = 0; c < ts.samples.size(); ++c)
-        if (!ts.dropped[c] && !ts.samples[c].empty()) {
-          const double m = *std::min_element(ts.samples[c].begin(), ts.samples[c].end());
-          if (m < best) {
-            best = m;
-            arg = c;
-          }
-        }
-      bool done = true;
-      for (size_t c = 0; c < ts.samples.size(); ++c) {
-        if (ts.dropped[c])
-          continue;
-        if (!ts.samples[c].empty() && c != arg &&
-            *std::min_element(ts.samples[c].begin(), ts.samples[c].end()) > kTuneMargin * best) {
-          ts.dropped[c] = 1;
-          continue;
-        }
-        done = done && ts.samples[c].size() >= tune_samples_;
-      }
-      if (done)
-        ts.chosen = int(arg);
-    }
-  }
+  if (!sampled.empty())
+    take_samples(work, sampled, ev);
   st.wall_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - w0).count();
   return st;
 }

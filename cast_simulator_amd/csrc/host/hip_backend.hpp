@@ -97,8 +97,9 @@ struct PlanInfo {
 // Per-gate kernel autotuning: for a dense gate on a statevector of at least
 // `min_qubits` qubits, every applicable kernel (wave tile in four orders and
 // two product forms, matrix core in four orders and, at f32 k >= 5, two
-// product forms, direct) is timed on the real gate, and the
-// fastest (by minimum) is used from then on.  Keyed by (kernel id, n).
+// product forms, direct) is timed on the real gate where it is launched by
+// itself (timed work, or a pass of one gate), and the fastest (by minimum) is
+// used there from then on.  Keyed by (kernel id, n).
 // Successive halving: every candidate is timed once; candidates slower than
 // kTuneMargin x the best so far are dropped; the rest are timed until each
 // has `samples` timings.
@@ -147,7 +148,8 @@ public:
   void apply(KernelId id, HipStatevector &sv);
   SyncStats sync(bool timed = true);
   // Launches the gates queued for `svs` (device pointers) on the manager's
-  // stream without waiting; gates for other statevectors stay queued.
+  // stream, waiting only where a tuning sample is taken; gates for other
+  // statevectors stay queued.
   void launch(const std::vector<uint64_t> &svs);
   // Drops the gates queued for a statevector that is no longer wanted.
   void discard(uint64_t sv);
@@ -174,9 +176,9 @@ private:
     KernelId id;
     uint64_t dptr;
     uint32_t n_qubits;
-    const void *plan; // launched where the gate runs by itself
-    const void *base; // the gate's own plan, for a pass with other gates
-    int cand;         // tuning candidate index, -1 when not a tuning sample
+    const void *plan; // the gate's own
+    bool tune;        // where it is launched by itself, by the tuned plan
+    int cand;         // tuning candidate launched, -1 when not a tuning sample
   };
   struct TuneState {
     std::vector<uint32_t> fams;
@@ -192,7 +194,14 @@ private:
   launch_shared_locked(const std::vector<Pending> &work, std::vector<std::vector<size_t>> lists);
   // Untimed work in few passes; the queue positions of tuning samples (each
   // between two events) go to `sampled`.
-  void launch_passes_locked(const std::vector<Pending> &work, std::vector<size_t> &sampled);
+  void launch_passes_locked(std::vector<Pending> &work, std::vector<size_t> &sampled);
+  // The plan to launch for a gate that runs by itself; sets `cand` when the
+  // launch is a tuning sample.
+  const void *single_plan_locked(Pending &w);
+  // Waits for tuning samples and takes their times.
+  void take_samples(const std::vector<Pending> &work, const std::vector<size_t> &sampled,
+                    const std::vector<void *> &ev);
+  void add_sample(const Pending &w, double seconds);
   void ensure_stream_locked();
   void ensure_events_locked(size_t n);
   TuneState &tune_state_locked(KernelId id, uint32_t n);

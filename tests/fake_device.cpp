@@ -53,6 +53,7 @@ void cast_hip_stream_destroy(void *) {}
 int cast_hip_stream_sync(void *, char *, size_t) { return ++cast_fake.syncs, 0; }
 void *cast_hip_event_create(char *, size_t) { return &live; }
 int cast_hip_event_record(void *, void *, char *, size_t) { return 0; }
+int cast_hip_event_synchronize(void *, char *, size_t) { return ++cast_fake.syncs, 0; }
 void cast_hip_event_destroy(void *) {}
 int cast_hip_event_elapsed_ms(void *, void *, float *ms, char *, size_t) { return *ms = 1.f, 0; }
 

@@ -69,3 +69,64 @@ print(json.dumps([failed, snapshot()]))
 """)
     assert "out of memory" in out[0]
     assert out[1]["on_freed"] == 0
+
+
+def test_untimed_groups_build_no_tuning_candidates(fake_lib):
+    """With the autotuner on (the default), gates that run in a pass with others
+    take their own plan; candidates are for gates launched by themselves."""
+    out = run(fake_lib, """
+n = 24
+mgr = cs.HipKernelManager(cs.HipKernelGenSpec.f64())
+sv = cs.HipStatevector(n, cs.Precision.F64)
+ids = [mgr.generate(cs.QuantumGate.random_unitary([q, q + 1], q)) for q in range(8)]
+for i in ids:
+    mgr.apply(i, sv)
+mgr.sync(False)
+grouped = snapshot()
+tuned = len(mgr.tuning_report())
+for i in ids:
+    mgr.apply(i, sv)
+mgr.sync(True)
+print(json.dumps([grouped, tuned, len(mgr.tuning_report()), snapshot()]))
+""")
+    grouped, tuned, tuned_timed, timed = out
+    assert grouped["plans"] == 8 and grouped["grouped"] == 8 and grouped["singles"] == 0
+    assert tuned == 0
+    assert tuned_timed == 8 and timed["singles"] == 8  # timed work is gate by gate
+
+
+def test_untimed_single_gates_are_tuned(fake_lib):
+    """A gate that no group takes (f64, six qubits) is sampled in untimed work
+    until its kernel is chosen."""
+    out = run(fake_lib, """
+n = 24
+mgr = cs.HipKernelManager(cs.HipKernelGenSpec.f64())
+sv = cs.HipStatevector(n, cs.Precision.F64)
+big = mgr.generate(cs.QuantumGate.random_unitary(list(range(6)), 1))
+small = mgr.generate(cs.QuantumGate.random_unitary([0], 2))
+chosen = []
+for _ in range(12):
+    for i in (small, small, big):
+        mgr.apply(i, sv)
+    mgr.sync(False)
+    chosen.append([e["chosen"] for e in mgr.tuning_report()])
+print(json.dumps([big, chosen, snapshot()]))
+""")
+    big, chosen, counts = out
+    assert all(len(c) == 1 for c in chosen)
+    assert chosen[0] == [-1] and chosen[-1][0] > 0
+    assert counts["grouped"] == 24 and counts["singles"] == 12
+
+
+def test_ensemble_of_large_members_does_not_wait_at_noisy_gates(fake_lib):
+    out = run(fake_lib, """
+n = 22
+gates = [cs.QuantumGate.random_unitary([q], q) for q in range(n)]
+for q in range(3):
+    gates.append(cs.QuantumGate.depolarizing(q, 0.3))
+    gates += [cs.QuantumGate.random_unitary([t], 50 * q + t) for t in range(n)]
+sim = cs.Simulator.f64()
+sim.sample_trajectory(graph(n, gates), cs.TrajectoryOpts([0], 8, 1, 4))
+print(json.dumps(snapshot()))
+""")
+    assert out["syncs"] == 1 and out["on_freed"] == 0
