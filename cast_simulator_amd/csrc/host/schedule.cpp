@@ -3,6 +3,8 @@
 
 #include "hip_backend.hpp"
 
+#include <algorithm>
+
 namespace cast::hip {
 
 namespace {
@@ -18,9 +20,11 @@ PassPlanner::PassPlanner(std::vector<PlannedGate> gates, PassLimits limits)
 uint32_t PassPlanner::collect(uint64_t set, std::vector<uint32_t> *taken,
                               std::vector<uint64_t> *ready) const {
   const uint64_t all = (uint64_t(1) << lim_.n_qubits) - 1;
+  const size_t end = std::min(left_.size(), head_ + kWindow);
   uint64_t blocked = 0;
   uint32_t count = 0;
-  for (uint32_t i : left_) {
+  for (size_t at = head_; at < end; ++at) {
+    const uint32_t i = left_[at];
     const PlannedGate &g = gates_[i];
     if (!(g.qubits & blocked) && g.may_join) {
       if (!(g.qubits & ~set)) {
@@ -44,12 +48,11 @@ uint32_t PassPlanner::collect(uint64_t set, std::vector<uint32_t> *taken,
 // fits, the one that brings the most gates per added qubit.
 bool PassPlanner::next(std::vector<uint32_t> &pass) {
   pass.clear();
-  if (left_.empty())
+  if (head_ == left_.size())
     return false;
-  const PlannedGate &first = gates_[left_.front()];
+  const PlannedGate &first = gates_[left_[head_]];
   if (!first.may_join) {
-    pass.push_back(left_.front());
-    left_.erase(left_.begin());
+    pass.push_back(left_[head_++]);
     return true;
   }
   uint64_t set = first.qubits | ((uint64_t(1) << lim_.low_qubits) - 1);
@@ -76,14 +79,18 @@ bool PassPlanner::next(std::vector<uint32_t> &pass) {
     set = best;
   }
   collect(set, &pass, nullptr);
-  size_t keep = 0, t = 0;
-  for (uint32_t i : left_) {
-    if (t < pass.size() && pass[t] == i)
-      ++t;
+  // The gates that stay behind move up to the last one taken.
+  size_t at = head_;
+  for (size_t t = 0; t < pass.size(); ++at)
+    t += left_[at] == pass[t];
+  size_t to = at;
+  for (size_t t = pass.size(); at-- > head_;) {
+    if (t > 0 && left_[at] == pass[t - 1])
+      --t;
     else
-      left_[keep++] = i;
+      left_[--to] = left_[at];
   }
-  left_.resize(keep);
+  head_ = to;
   return true;
 }
 

@@ -39,9 +39,16 @@ private:
   // that could run now.
   uint32_t collect(uint64_t set, std::vector<uint32_t> *taken, std::vector<uint64_t> *ready) const;
 
+  // A pass takes gates among the next kWindow only.  A list that leaves a qubit
+  // idle never blocks every qubit, and each pass would look through all of it:
+  // 16000 gates on 19 of 20 qubits took 222 ms to plan, now 20 (all 20
+  // qubits: 10), with as many passes.
+  static constexpr size_t kWindow = 512;
+
   std::vector<PlannedGate> gates_;
   PassLimits lim_;
-  std::vector<uint32_t> left_; // not yet in a pass, in order
+  std::vector<uint32_t> left_; // from head_ on: not yet in a pass, in order
+  size_t head_ = 0;
 };
 
 // The passes of `plans` on one statevector, as indices; `all_join`:
