@@ -684,8 +684,15 @@ __global__ void __launch_bounds__(kMaxBlock, OCC)
   const T *src = g == 0 ? checkpoints + 2 * len * task.checkpoint : slot;
   const uint32_t waves = blockDim.x >> 6;
   const Share sh{part * waves + (threadIdx.x >> 6), parts * waves};
-  if (!wg_gate<T>(gates[task.first_gate + g], src, slot, matrices, a, n, sh, gate_lds))
-    atomicOr(&work[1], 1u);
+  if (wg_gate<T>(gates[task.first_gate + g], src, slot, matrices, a, n, sh, gate_lds))
+    return;
+  atomicOr(&work[1], 1u);
+  if (g == 0) { // left out: the next gate reads the slot
+    using VT = typename V2<T>::type;
+    for (uint64_t i = uint64_t(part) * blockDim.x + threadIdx.x; i < len;
+         i += uint64_t(parts) * blockDim.x)
+      reinterpret_cast<VT *>(slot)[i] = reinterpret_cast<const VT *>(src)[i];
+  }
 }
 
 // Sums and dump of the tasks order[first ...) after their last step, `parts`
@@ -743,12 +750,15 @@ __global__ void __launch_bounds__(256)
 }
 
 template <typename T>
-__global__ void k_traj_sum(const uint32_t *__restrict__ order, const T *__restrict__ slots,
-                           double *__restrict__ out, TrajScalars a, uint32_t first,
-                           uint32_t parts) {
-  const uint32_t ti = order[first + blockIdx.x], slots_n = 1 + a.n_pairs;
-  if (ti >= a.n_tasks || threadIdx.x >= slots_n)
-    return;
+__global__ void k_traj_sum(const cast_hip_traj_task_t *__restrict__ tasks,
+                           const uint32_t *__restrict__ order, const T *__restrict__ slots,
+                           double *__restrict__ out, uint32_t *__restrict__ work, TrajScalars a,
+                           uint32_t first, uint32_t parts) {
+  uint32_t ti;
+  cast_hip_traj_task_t task{};
+  const uint32_t slots_n = 1 + a.n_pairs;
+  if (!fetch_task(tasks, order, first + blockIdx.x, work, a, ti, task) || threadIdx.x >= slots_n)
+    return; // k_traj_finish left no sums for a task out of range
   const uint64_t len = uint64_t(1) << a.n_qubits, mine = len / parts;
   double s = 0.0;
   for (uint32_t p = 0; p < parts; ++p)
@@ -818,8 +828,8 @@ void launch_steps_t(const cast_hip_traj_launch_t &L, const TrajScalars &a, const
     check(hipGetLastError(), "hipLaunchKernelGGL(k_traj_finish)");
     if (parts == 1)
       continue;
-    hipLaunchKernelGGL((k_traj_sum<T>), dim3(here), dim3(64), 0, s, order, slots,
-                       reinterpret_cast<double *>(L.out), a, first, parts);
+    hipLaunchKernelGGL((k_traj_sum<T>), dim3(here), dim3(64), 0, s, tasks, order, slots,
+                       reinterpret_cast<double *>(L.out), work, a, first, parts);
     check(hipGetLastError(), "hipLaunchKernelGGL(k_traj_sum)");
   }
 }
