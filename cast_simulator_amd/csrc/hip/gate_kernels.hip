@@ -1077,9 +1077,11 @@ void launch_mfma_batch(const BatchArgs &a, unsigned n, uint8_t precision, uint32
 } // namespace
 
 // f32 k = 4 stays with the direct kernel: its product form is the more exact
-// one, and it holds its 16 amplitudes in registers.
+// one, and it holds its 16 amplitudes in registers.  So do plans that ask for a
+// variant or for f32 products: the batch has no other kernel for them.
 bool batch_on_matrix_cores(const GatePlan &p, uint32_t n) {
-  return p.d_mat3 && n >= p.k + 4 && (p.precision == 1 || p.k >= 5);
+  return p.d_mat3 && n >= p.k + 4 && (p.precision == 1 || p.k >= 5) && !p.forced &&
+         !(p.flags & CAST_HIP_FLAG_MFMA_F32);
 }
 
 uint32_t plan_family(const GatePlan &plan, uint32_t n_qubits) {

@@ -248,10 +248,12 @@ int cast_hip_gate_apply(const void *plan, void *stream, uint64_t sv_dptr, uint32
 /* Enqueue n_items independent (plan, statevector) pairs as ONE launch (64
  * items per launch, more in several launches): item i applies plans[i] to
  * svs[i] (2^sv_n_qubits[i] amplitudes, sv_n_qubits[i] <= 40) with the direct
- * kernel or, for dense gates of k = 4 (f64), 5 and 6 on k + 4 qubits or more,
- * on the matrix cores (then at most two launches per 64 items).  All plans must share precision and k.  For callers that hold many
- * small statevectors (one launch instead of one per statevector).  No
- * reference counterpart (the reference launches one kernel per apply). */
+ * kernel or, for dense gates of k = 4 (f64), 5 and 6 on k + 4 qubits or more
+ * whose plan asks for no variant and not for CAST_HIP_FLAG_MFMA_F32, on the
+ * matrix cores (then at most two launches per 64 items).  All plans must share
+ * precision and k.  For callers that hold many small statevectors (one launch
+ * instead of one per statevector).  No reference counterpart (the reference
+ * launches one kernel per apply). */
 int cast_hip_gate_apply_batch(const void *const *plans, const uint64_t *svs,
                               const uint32_t *sv_n_qubits, size_t n_items, void *stream,
                               char *err_buf, size_t err_buf_len);
