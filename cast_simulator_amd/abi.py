@@ -185,6 +185,7 @@ _SIGS = {
     "cast_hip_gate_apply": (_i, [_vp, _vp, _u64, _u32, _err, _sz]),
     "cast_hip_gate_apply_batch": (
         _i, [C.POINTER(_vp), C.POINTER(_u64), C.POINTER(_u32), _sz, _vp, _err, _sz]),
+    "cast_hip_gate_batch_launches": (_sz, [C.POINTER(_vp), C.POINTER(_u32), _sz]),
     "cast_hip_gate_group_info": (_i, [_vp, _u32, C.POINTER(GroupInfo), _err, _sz]),
     "cast_hip_gate_apply_group": (_i, [C.POINTER(_vp), _sz, _vp, _u64, _u32, _err, _sz]),
     "cast_hip_group_batch_scratch_bytes": (_sz, [_sz, _sz]),
@@ -327,6 +328,11 @@ def gate_apply_batch(plans, svs, n_qubits, stream: int | None = None) -> None:
     n = len(plans)
     _call("cast_hip_gate_apply_batch", (_vp * n)(*plans), (_u64 * n)(*svs),
           (_u32 * n)(*n_qubits), n, stream)
+
+
+def gate_batch_launches(plans, n_qubits) -> int:
+    n = len(plans)
+    return int(lib().cast_hip_gate_batch_launches((_vp * n)(*plans), (_u32 * n)(*n_qubits), n))
 
 
 def gate_group_info(plan: int, n_qubits: int) -> GroupInfo:

@@ -696,6 +696,16 @@ int cast_hip_gate_apply_batch(const void *const *plans, const uint64_t *svs,
   });
 }
 
+size_t cast_hip_gate_batch_launches(const void *const *plans, const uint32_t *sv_n_qubits,
+                                    size_t n_items) {
+  if (!plans || !sv_n_qubits)
+    return 0;
+  size_t cores = 0;
+  for (size_t i = 0; i < n_items; ++i)
+    cores += plans[i] && batch_on_matrix_cores(*static_cast<const GatePlan *>(plans[i]), sv_n_qubits[i]);
+  return batch_launches(n_items - cores) + batch_launches(cores);
+}
+
 int cast_hip_gate_group_info(const void *plan, uint32_t sv_n_qubits, cast_hip_group_info_t *out,
                              char *err, size_t len) {
   return guard(err, len, [&] {

@@ -118,6 +118,7 @@ struct BatchItem {
 // Whether an item of a batch runs on the matrix cores (its matrix then is
 // plan.d_mat3); the others run the direct kernel on plan.d_mat.
 bool batch_on_matrix_cores(const GatePlan &plan, uint32_t n_qubits);
+size_t batch_launches(size_t n); // launches of launch_gate_batch for n items
 void launch_gate_batch(const BatchItem *items, size_t n, uint8_t precision, uint32_t k,
                        bool matrix_cores, hipStream_t stream);
 

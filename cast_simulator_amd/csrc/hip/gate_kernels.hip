@@ -1111,6 +1111,8 @@ void launch_gate(const GatePlan &plan, hipStream_t stream, void *sv, uint32_t n_
     launch_by_k<double>(plan, stream, sv, g);
 }
 
+size_t batch_launches(size_t n) { return (n + kMaxBatch - 1) / kMaxBatch; }
+
 void launch_gate_batch(const BatchItem *items, size_t n, uint8_t precision, uint32_t k,
                        bool matrix_cores, hipStream_t stream) {
   for (size_t off = 0; off < n; off += kMaxBatch) {

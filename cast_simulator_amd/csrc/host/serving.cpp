@@ -490,7 +490,8 @@ std::vector<ServeResult> Server::run(const std::vector<ServeRequest> &reqs, Serv
           throw_if(cast_hip_gate_apply_batch(g.plans.data(), g.svs.data(), g.ns.data(),
                                              g.plans.size(), s.stream, err, kErr),
                    err);
-          n_batch_launches += (g.plans.size() + 63) / 64;
+          n_batch_launches +=
+              cast_hip_gate_batch_launches(g.plans.data(), g.ns.data(), g.plans.size());
         }
       }
     }

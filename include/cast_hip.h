@@ -257,6 +257,9 @@ int cast_hip_gate_apply(const void *plan, void *stream, uint64_t sv_dptr, uint32
 int cast_hip_gate_apply_batch(const void *const *plans, const uint64_t *svs,
                               const uint32_t *sv_n_qubits, size_t n_items, void *stream,
                               char *err_buf, size_t err_buf_len);
+/* Launches that cast_hip_gate_apply_batch takes for these items. */
+size_t cast_hip_gate_batch_launches(const void *const *plans, const uint32_t *sv_n_qubits,
+                                    size_t n_items);
 
 /* Gate groups: consecutive gates whose targets together lie in few qubits run
  * as ONE pass over the statevector (one read and one write of every amplitude
