@@ -187,6 +187,7 @@ _SIGS = {
         _i, [C.POINTER(_vp), C.POINTER(_u64), C.POINTER(_u32), _sz, _vp, _err, _sz]),
     "cast_hip_gate_batch_launches": (_sz, [C.POINTER(_vp), C.POINTER(_u32), _sz]),
     "cast_hip_gate_group_info": (_i, [_vp, _u32, C.POINTER(GroupInfo), _err, _sz]),
+    "cast_hip_gate_group_pays": (_i, [C.POINTER(_vp), _sz, _u32]),
     "cast_hip_gate_apply_group": (_i, [C.POINTER(_vp), _sz, _vp, _u64, _u32, _err, _sz]),
     "cast_hip_group_batch_scratch_bytes": (_sz, [_sz, _sz]),
     "cast_hip_gate_apply_group_batch": (
@@ -339,6 +340,11 @@ def gate_group_info(plan: int, n_qubits: int) -> GroupInfo:
     info = GroupInfo()
     _call("cast_hip_gate_group_info", plan, n_qubits, C.byref(info))
     return info
+
+
+def gate_group_pays(plans, n_qubits: int) -> bool:
+    n = len(plans)
+    return bool(lib().cast_hip_gate_group_pays((_vp * n)(*plans), n, n_qubits))
 
 
 def gate_apply_group(plans, dptr: int, n_qubits: int, stream: int | None = None) -> None:

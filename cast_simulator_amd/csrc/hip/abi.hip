@@ -720,6 +720,15 @@ int cast_hip_gate_group_info(const void *plan, uint32_t sv_n_qubits, cast_hip_gr
   });
 }
 
+int cast_hip_gate_group_pays(const void *const *plans, size_t n_plans, uint32_t sv_n_qubits) {
+  if (!plans)
+    return 0;
+  for (size_t i = 0; i < n_plans; ++i)
+    if (!plans[i])
+      return 0;
+  return group_pays(reinterpret_cast<const GatePlan *const *>(plans), n_plans, sv_n_qubits);
+}
+
 int cast_hip_gate_apply_group(const void *const *plans, size_t n_plans, void *stream,
                               uint64_t sv_dptr, uint32_t sv_n_qubits, char *err, size_t len) {
   return guard(err, len, [&] {

@@ -135,6 +135,8 @@ GroupLimits group_limits(const GatePlan &plan, uint32_t n_qubits);
 // buffer itself from the snapped matrix m of 2 K K doubles).
 size_t group_operand_bytes(uint32_t k, uint8_t precision);
 void group_operands(const double *m, uint32_t k, uint8_t precision, void *out);
+// Whether one pass is expected to be faster than a launch for each gate.
+bool group_pays(const GatePlan *const *plans, size_t n_plans, uint32_t n_qubits);
 // Enqueues the gates, in order, as one pass over the statevector.
 void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stream, void *sv,
                   uint32_t n_qubits);

@@ -1039,6 +1039,58 @@ size_t tile_bytes(uint32_t m, uint8_t prec) { return size_t(prec == 0 ? 8 : 16) 
 
 } // namespace
 
+namespace {
+
+// Share of the statevector's 128-byte lines that a monomial gate launched by
+// itself reads or writes.
+double touched_lines(const GatePlan &p) {
+  const uint32_t line_bits = p.precision == 0 ? 4 : 3;
+  uint32_t low = 0;
+  while (low < p.k && p.q[low] < line_bits)
+    ++low;
+  uint64_t rows = 0;
+  for (uint32_t x = 0; x < p.n_active; ++x)
+    rows |= uint64_t(1) << (p.act_row[x] >> low) | uint64_t(1) << (p.act_col[x] >> low);
+  return double(__builtin_popcountll(rows)) / double(1u << (p.k - low));
+}
+
+} // namespace
+
+// A pass reads and writes every amplitude, a monomial gate by itself only the
+// lines with rows other than the identity's.  On states that fill the chip a
+// few such gates (controlled phases, Toffolis) are therefore faster one by
+// one, from below against the time T of a read and a write of the state at 6.55
+// TB/s: a pass 5 us + 1.12 T and a quarter of a microsecond per gate; a launch
+// 5 us + a T per line touched, a = 0.75 up to 512 MiB, 1.15 up to 2 GiB, 1.4
+// above, and with four targets and more at least the share `least` of T (its
+// rows are gathered).  us, one by one / in a pass: two phases with 1, 2, 4 controls
+// on high qubits, f64 24 qubits 36 / 90, 23 / 99, 53 / 99, 28 qubits 850 /
+// 1500, 393 / 1591, 270 / 1593, 30 qubits 3772 / 5882, 1788 / 6342, 872 / 6301;
+// five with one control 88 / 100, 2105 / 1579, 9579 / 6460.
+bool group_pays(const GatePlan *const *plans, size_t n_plans, uint32_t n) {
+  constexpr double least[2][3] = {{0.1, 0.25, 0.7}, {0.06, 0.12, 0.35}}; // k = 4, 5, 6
+  if (n_plans < 2)
+    return false;
+  const uint8_t prec = plans[0]->precision;
+  if (!many_tiles(n, prec))
+    return true;
+  const double bytes = double(prec == 0 ? 8 : 16) * double(uint64_t(1) << n);
+  const double mib = bytes / (1 << 20), t = 2.0 * bytes / 6.55e6;
+  const double a = mib <= 512 ? 0.75 : mib <= 2048 ? 1.15 : 1.4;
+  double alone = 0.0;
+  for (size_t i = 0; i < n_plans; ++i) {
+    const GatePlan &p = *plans[i];
+    if (p.variant != 2)
+      return true;
+    double share = a * touched_lines(p);
+    if (p.k >= 4 && p.k <= 6)
+      share = std::max(share, least[n >= 27][p.k - 4]);
+    if (p.n_active > 0)
+      alone += 5.0 + share * t;
+  }
+  return alone >= 5.0 + 1.12 * t + 0.25 * double(n_plans);
+}
+
 void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stream, void *sv,
                   uint32_t n) {
   if (n_plans == 0)

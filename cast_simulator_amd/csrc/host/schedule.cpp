@@ -138,13 +138,14 @@ void apply_in_passes(const std::vector<const void *> &plans, void *stream, uint6
   std::vector<uint32_t> pass;
   std::vector<const void *> group;
   while (planner.next(pass)) { // the device works on a pass while the next is planned
-    if (pass.size() == 1) {
-      single(pass[0]);
-      continue;
-    }
     group.clear();
     for (uint32_t i : pass)
       group.push_back(plans[i]);
+    if (pass.size() == 1 || !cast_hip_gate_group_pays(group.data(), group.size(), n_qubits)) {
+      for (uint32_t i : pass)
+        single(i);
+      continue;
+    }
     throw_if(cast_hip_gate_apply_group(group.data(), group.size(), stream, sv_dptr, n_qubits, err,
                                        kErr),
              err);

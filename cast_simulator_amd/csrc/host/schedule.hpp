@@ -57,7 +57,7 @@ std::vector<std::vector<uint32_t>> plan_passes(const std::vector<const void *> &
                                                uint32_t n_qubits, bool &all_join);
 
 // Enqueues `plans` in order on `stream`, the groups that the planner finds as
-// one pass each and every other gate i by `single(i)`.
+// one pass each, where that pays, and every other gate i by `single(i)`.
 void apply_in_passes(const std::vector<const void *> &plans, void *stream, uint64_t sv_dptr,
                      uint32_t n_qubits, const std::function<void(uint32_t)> &single);
 

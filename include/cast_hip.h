@@ -281,6 +281,9 @@ typedef struct cast_hip_group_info_t {
 } cast_hip_group_info_t;
 int cast_hip_gate_group_info(const void *plan, uint32_t sv_n_qubits, cast_hip_group_info_t *out,
                              char *err_buf, size_t err_buf_len);
+/* 1 if that group is expected to be faster than a cast_hip_gate_apply of each
+ * plan (a few gates that touch a small part of the amplitudes are not). */
+int cast_hip_gate_group_pays(const void *const *plans, size_t n_plans, uint32_t sv_n_qubits);
 int cast_hip_gate_apply_group(const void *const *plans, size_t n_plans, void *stream,
                               uint64_t sv_dptr, uint32_t sv_n_qubits, char *err_buf,
                               size_t err_buf_len);

@@ -18,8 +18,8 @@ uint64_t next_sv = 4096;
 
 extern "C" {
 struct cast_fake_counts {
-  long plans, syncs, singles, grouped, on_freed, allocs, fail_alloc; // fail_alloc: -1 or which
-} cast_fake = {0, 0, 0, 0, 0, 0, -1};
+  long plans, syncs, singles, grouped, on_freed, allocs, fail_alloc, pays; // fail_alloc: -1 or which
+} cast_fake = {0, 0, 0, 0, 0, 0, -1, 1};
 
 uint64_t cast_hip_sv_alloc(size_t, uint8_t, char *err, size_t len) {
   if (cast_fake.allocs++ == cast_fake.fail_alloc) {
@@ -99,6 +99,7 @@ int cast_hip_gate_group_info(const void *plan, uint32_t n, cast_hip_group_info_t
   out->max_gates = 64;
   return 0;
 }
+int cast_hip_gate_group_pays(const void *const *, size_t, uint32_t) { return int(cast_fake.pays); }
 int cast_hip_gate_apply(const void *, void *, uint64_t sv, uint32_t, char *, size_t) {
   cast_fake.on_freed += !live.count(sv);
   return ++cast_fake.singles, 0;

@@ -17,7 +17,8 @@ import ctypes, json, sys
 fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 class Counts(ctypes.Structure):
     _fields_ = [(f, ctypes.c_long) for f in
-                ("plans", "syncs", "singles", "grouped", "on_freed", "allocs", "fail_alloc")]
+                ("plans", "syncs", "singles", "grouped", "on_freed", "allocs", "fail_alloc",
+                 "pays")]
 counts = Counts.in_dll(fake, "cast_fake")
 import cast_simulator_amd as cs
 def graph(n, gates):
@@ -130,3 +131,17 @@ sim.sample_trajectory(graph(n, gates), cs.TrajectoryOpts([0], 8, 1, 4))
 print(json.dumps(snapshot()))
 """)
     assert out["syncs"] == 1 and out["on_freed"] == 0
+
+
+@pytest.mark.parametrize("pays", [0, 1])
+def test_groups_that_do_not_pay_go_gate_by_gate(fake_lib, pays):
+    out = run(fake_lib, f"""
+counts.pays = {pays}
+mgr = cs.HipKernelManager(cs.HipKernelGenSpec.f64())
+sv = cs.HipStatevector(24, cs.Precision.F64)
+for q in range(3):
+    mgr.apply(mgr.generate(cs.QuantumGate.cz(q, q + 9)), sv)
+mgr.sync(False)
+print(json.dumps(snapshot()))
+""")
+    assert (out["grouped"], out["singles"]) == ((3, 0) if pays else (0, 3))
