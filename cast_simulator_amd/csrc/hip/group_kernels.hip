@@ -1041,10 +1041,9 @@ size_t tile_bytes(uint32_t m, uint8_t prec) { return size_t(prec == 0 ? 8 : 16) 
 
 namespace {
 
-// Share of the statevector's 128-byte lines that a monomial gate launched by
-// itself reads or writes.
-double touched_lines(const GatePlan &p) {
-  const uint32_t line_bits = p.precision == 0 ? 4 : 3;
+// Share of the statevector's lines of 2^line_bits amplitudes that a monomial
+// gate launched by itself reads or writes.
+double touched_lines(const GatePlan &p, uint32_t line_bits) {
   uint32_t low = 0;
   while (low < p.k && p.q[low] < line_bits)
     ++low;
@@ -1059,36 +1058,41 @@ double touched_lines(const GatePlan &p) {
 // A pass reads and writes every amplitude, a monomial gate by itself only the
 // lines with rows other than the identity's.  On states that fill the chip a
 // few such gates (controlled phases, Toffolis) are therefore faster one by
-// one, from below against the time T of a read and a write of the state at 6.55
-// TB/s: a pass 5 us + 1.12 T and a quarter of a microsecond per gate; a launch
-// 5 us + a T per line touched, a = 0.75 up to 512 MiB, 1.15 up to 2 GiB, 1.4
-// above, and with four targets and more at least the share `least` of T (its
-// rows are gathered).  us, one by one / in a pass: two phases with 1, 2, 4 controls
-// on high qubits, f64 24 qubits 36 / 90, 23 / 99, 53 / 99, 28 qubits 850 /
-// 1500, 393 / 1591, 270 / 1593, 30 qubits 3772 / 5882, 1788 / 6342, 872 / 6301;
-// five with one control 88 / 100, 2105 / 1579, 9579 / 6460.
+// one.  With T the time of a read and a write of the state at 6.55 TB/s, a pass
+// takes about 5 us + T (1.12 T above 512 MiB) and a quarter of a microsecond
+// per gate, a launch 5 us + a T times the share of lines touched, and with four
+// targets and more at least the share `least` of T (its rows are gathered).
+// Up to 512 MiB the caches serve lines of 64 bytes: a = 1 behind another pass
+// (two gates of four targets, 6 rows of 16, 24 qubits f64: 108 us, 74 in a
+// pass), 0.75 where the state was read before; above, lines of 128 bytes, a =
+// 1.15 up to 2 GiB, then 1.4.  us, one by one / in a pass: two phases with 1,
+// 2, 4 controls on high qubits, f64 24 qubits 36 / 90, 23 / 99, 53 / 99, 28
+// qubits 850 / 1500, 393 / 1591, 270 / 1593, 30 qubits 3772 / 5882, 1788 /
+// 6342, 872 / 6301; five with one control 88 / 100, 2105 / 1579, 9579 / 6460.
 bool group_pays(const GatePlan *const *plans, size_t n_plans, uint32_t n) {
   constexpr double least[2][3] = {{0.1, 0.25, 0.7}, {0.06, 0.12, 0.35}}; // k = 4, 5, 6
-  if (n_plans < 2)
+  if (n_plans < 2 || n > kMaxGroupQubits)
     return false;
   const uint8_t prec = plans[0]->precision;
   if (!many_tiles(n, prec))
     return true;
   const double bytes = double(prec == 0 ? 8 : 16) * double(uint64_t(1) << n);
   const double mib = bytes / (1 << 20), t = 2.0 * bytes / 6.55e6;
-  const double a = mib <= 512 ? 0.75 : mib <= 2048 ? 1.15 : 1.4;
+  const bool cached = mib <= 512;
+  const double a = cached ? 1.0 : mib <= 2048 ? 1.15 : 1.4;
+  const uint32_t line_bits = (prec == 0 ? 4 : 3) - cached;
   double alone = 0.0;
   for (size_t i = 0; i < n_plans; ++i) {
     const GatePlan &p = *plans[i];
     if (p.variant != 2)
       return true;
-    double share = a * touched_lines(p);
+    double share = a * touched_lines(p, line_bits);
     if (p.k >= 4 && p.k <= 6)
       share = std::max(share, least[n >= 27][p.k - 4]);
     if (p.n_active > 0)
       alone += 5.0 + share * t;
   }
-  return alone >= 5.0 + 1.12 * t + 0.25 * double(n_plans);
+  return alone >= 5.0 + (cached ? 1.0 : 1.12) * t + 0.25 * double(n_plans);
 }
 
 void launch_group(const GatePlan *const *plans, size_t n_plans, hipStream_t stream, void *sv,
