@@ -131,8 +131,8 @@ struct GroupLimits {
   uint32_t max_gates;
 };
 GroupLimits group_limits(const GatePlan &plan, uint32_t n_qubits);
-// Matrix-core operands of a dense k = 4 or 5 gate for a group (bytes, and the
-// buffer itself from the snapped matrix m of 2 K K doubles).
+// Matrix-core operands of a dense k = 4, 5 or (f32) 6 gate for a group (bytes,
+// and the buffer itself from the snapped matrix m of 2 K K doubles).
 size_t group_operand_bytes(uint32_t k, uint8_t precision);
 void group_operands(const double *m, uint32_t k, uint8_t precision, void *out);
 // Whether one pass is expected to be faster than a launch for each gate.
