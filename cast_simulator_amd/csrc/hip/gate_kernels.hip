@@ -839,6 +839,11 @@ void launch_tile_k(const GatePlan &p, hipStream_t s, void *sv, const TileGeom &t
 }
 
 // Wave-tile geometry for a gate on an n-qubit statevector (n >= k + 6).
+// Whether the statevector takes about half of the XCDs' L2 (16 MiB).
+bool xcd_resident(const GatePlan &p, uint32_t n) {
+  return (uint64_t(2 * scalar_bytes(p.precision)) << n) == uint64_t(16) << 20;
+}
+
 TileGeom tile_geom(const GatePlan &p, uint32_t n, uint32_t *n_low) {
   TileGeom tg{};
   tg.n_tiles = uint64_t(1) << (n - 6 - p.k);
@@ -859,9 +864,16 @@ TileGeom tile_geom(const GatePlan &p, uint32_t n, uint32_t *n_low) {
   // the 30-qubit headline circuit's k = 3, 4 gates.  Below it costs: f64 k =
   // 1..4 launch order / XCD at 24 qubits 82-95 / 86-102 us, at 26 339-397 /
   // 349-404, at 28 1393-1517 / 1352-1542; the per-gate autotuner tries all.
-  const bool large = (uint64_t(2 * scalar_bytes(p.precision)) << n) >= uint64_t(4) << 30;
+  // From 512 MiB on it pays for neighbouring targets among the highest bits but
+  // the top one, where tiles in launch order fall on few channels (f64 targets n
+  // - 4, n - 3 at 25, 26 qubits 219 / 181, 439 / 360; n - 7 .. n - 4 at 26, 27
+  // qubits 485 / 386, 1091 / 759, f32 at 28 qubits 930 / 758).
+  const uint64_t mib = (uint64_t(2 * scalar_bytes(p.precision)) << n) >> 20;
+  bool order = mib >= 4096 || xcd_resident(p, n);
+  for (uint32_t b = 0; b + 1 < p.k && mib >= 512; ++b)
+    order = order || (p.q[b] + 7 >= n && p.q[b + 1] == p.q[b] + 1 && p.q[b + 1] + 2 <= n);
   const bool xcd = (p.flags & CAST_HIP_FLAG_TILE_XCD) ||
-                   (auto_choice(p) && large && !(p.flags & CAST_HIP_FLAG_TILE_SWIZZLE));
+                   (auto_choice(p) && order && !(p.flags & CAST_HIP_FLAG_TILE_SWIZZLE));
   if (xcd && tg.n_tiles >= 32)
     tg.xcd_bits = n - 6 - p.k - 2;
   *n_low = L;
@@ -908,28 +920,53 @@ uint32_t count_low(const GatePlan &p) {
 //   k <= 3       the direct kernel: f32 k = 3 at 22, 24, 25 qubits 9-12, 34-42,
 //                70-103 against 10-21, 42-68, 87-131 on wave tiles; f64 k = 3
 //                at 18, 22, 24 qubits 4, 19-26, 66-80 against 4-6.5, 22-25,
-//                88-93;
-//   f64 k = 4    matrix cores up to 16 MiB (4-10 against 7-14 on tiles) and
-//                from 128 MiB on (43, 82 against 45-59, 91-109); between, wave
-//                tiles for L <= 2 (11.3-12.5, 23-27 against 17.6, 28);
+//                88-93.  Except where targets crowd in the lowest bits, so that
+//                the direct kernel's lanes read pieces of lines: f64 targets 0
+//                and 1 (k = 2 at 20, 22, 24 qubits 28, 23 and 89, 84 on tiles,
+//                k = 3 [0, 1, 2] 34, 30 and 115, 96), f32 two targets of k = 2
+//                or all of k = 3 below 3 (22, 25 qubits 15, 11 and 93, 82;
+//                [0, 1, 2] 25, 21 and 170, 142).  And except at 16 MiB, where in
+//                XCD order every XCD finds its tiles in its own L2 (f64 20
+//                qubits k = 1, 2 5.1-8.8 direct, 4.1-4.9 on tiles; k = 3 L = 0
+//                5.3, 4.2, L > 0 crowded 6.5-10.5, 5.1-8.4, else 5.2-5.4, 5.2-8.4);
+//   f64 k = 4    matrix cores up to 16 MiB (4-10 against 7-14 on tiles; at 16
+//                tiles for L = 0, 7.9-8.9 against 9.8-10.4) and from 128 MiB on
+//                (43, 82 against 45-59, 91-109); between, wave tiles for L <= 2
+//                (11.3-12.5, 23-27 against 17.6, 28);
 //   f32 k = 4    matrix cores up to 4 MiB (4.7 against 5.6-11); above, tiles for
-//                L = 0 (6.3-45 against 7.4-45 direct), else the direct kernel
-//                (22, 24 qubits 14.5-18, 45-60 against tiles 16-24, 51-75), at
-//                128 MiB and more matrix cores for L >= 3 (53, 98 against 60, 115);
+//                L = 0 below 128 MiB (6.3-24 against 7.4-26 direct; at 24, 25
+//                qubits 48-53, 90-113 against 44-49, 85-92), matrix cores from
+//                32 MiB on with three targets below 3 (23 qubits 44, 37 against
+//                60, 48) and from 128 MiB on for L >= 3 (53, 98 against 60, 115),
+//                else the direct kernel (22, 24 qubits 14.5-18, 45-60 against
+//                tiles 16-24, 51-75);
 //   f64 k = 5    wave tiles at 32 and 64 MiB for L <= 1 (26, 31 against 29, 54
 //                on the matrix cores) and at 128 MiB (63 against 66);
 //   else         matrix cores.
 uint32_t automatic_cached(const GatePlan &p, uint32_t n, uint32_t n_low, bool tile_ok,
                           bool mfma_ok) {
   const uint64_t mib = (uint64_t(2 * scalar_bytes(p.precision)) << n) >> 20;
-  if (p.k <= 3)
-    return 1;
+  const bool f64 = p.precision == 1;
   uint32_t v = 4;
-  if (p.precision == 1 && p.k == 4)
-    v = mib > 16 && mib < 128 && n_low <= 2 ? 3 : 4;
+  if (p.k <= 3) {
+    const uint32_t last = p.q[p.k - 1];
+    bool tile = false;
+    if (xcd_resident(p, n))
+      tile = p.k < 3 || n_low == 0 || p.q[n_low - 1] < (n_low == 1 ? 2u : 3u);
+    else if (p.k == 2)
+      tile = last < (f64 ? 2u : 3u);
+    else if (p.k == 3)
+      tile = mib > 8 && (f64 ? p.q[1] < 2 : last < 3);
+    v = tile ? 3 : 1;
+  } else if (f64 && p.k == 4)
+    v = xcd_resident(p, n) ? (n_low == 0 ? 3 : 4) : mib > 16 && mib < 128 && n_low <= 2 ? 3 : 4;
   else if (p.k == 4)
-    v = mib <= 4 ? 4 : n_low == 0 ? 3 : mib >= 128 && n_low >= 3 ? 4 : 1;
-  else if (p.precision == 1)
+    v = mib <= 4                     ? 4
+        : n_low == 0 && mib < 128    ? 3
+        : mib >= 32 && p.q[2] < 3    ? 4
+        : mib >= 128 && n_low >= 3   ? 4
+                                     : 1;
+  else if (f64)
     v = mib > 16 && mib <= 128 && n_low <= 1 ? 3 : 4;
   if (v == 4 && !mfma_ok)
     v = 3;
