@@ -115,6 +115,9 @@ struct BatchItem {
   uint8_t k;
   uint8_t pad;
 };
+// Share of the statevector's lines of 2^line_bits amplitudes that a monomial
+// gate touches: those with rows other than the identity's, and their columns.
+double touched_lines(const GatePlan &plan, uint32_t line_bits);
 // Whether an item of a batch runs on the matrix cores (its matrix then is
 // plan.d_mat3); the others run the direct kernel on plan.d_mat.
 bool batch_on_matrix_cores(const GatePlan &plan, uint32_t n_qubits);

@@ -573,13 +573,36 @@ void launch_dense_t(const GatePlan &p, hipStream_t s, void *sv, const GateGeom &
   check(hipGetLastError(), "hipLaunchKernelGGL(k_dense)");
 }
 
-// Diagonal gates with three quarters of their entries or more other than 1;
-// with fewer, k_monomial skips what it need not touch.
-bool streamed_diagonal(const GatePlan &p) {
+// Whether a diagonal gate with three quarters of its entries or more other than
+// 1 goes as a stream over all amplitudes.  k_monomial skips the lines that such a
+// gate need not touch, but gathers its K rows: that costs with many rows, and
+// where two targets lie within a line (24 qubits f64, 12 of 16 entries, targets
+// 0..3 300 us, streamed 78).  Otherwise by the share of lines touched; us
+// gathered / streamed, high targets:
+//   up to 32 MiB   k <= 3 above 3/4 (21 qubits f64, shares 3/4 and 1 7 / 8, 8 / 8),
+//                  k = 4 always (10 / 8);
+//   up to 256 MiB  only the full share (24 qubits f64, 3/4, 7/8, 15/16, 1: k = 2,
+//                  3, 4 58 / 78, 70 / 78, 74 / 78, 79 / 78), at 64 MiB only f32 k =
+//                  4 (28 / 24; f64 21 / 23, f32 k = 2 22 / 23.5);
+//   above          f64 and f32 k = 2 above 3/4 (28 qubits f64 1279 / 1413, 1488 /
+//                  1415; 29 qubits f32 1341 / 1408, 1801 / 1412), f32 k = 3, 4 always
+//                  (1687 / 1410).
+bool streamed_diagonal(const GatePlan &p, const GateGeom &g, size_t scalar) {
   for (uint32_t j = 0; j < p.n_active; ++j)
     if (p.act_row[j] != p.act_col[j])
       return false;
-  return 4 * p.n_active >= 3u << p.k;
+  if (4 * p.n_active < 3u << p.k)
+    return false;
+  if (p.k >= 5 || (p.k >= 2 && p.q[1] < 3))
+    return true;
+  const uint64_t mib = ((g.combos << g.k) * 2 * scalar) >> 20;
+  const bool f64 = scalar == 8, cached = mib <= 256;
+  const double share = touched_lines(p, (f64 ? 3u : 4u) - cached);
+  if (mib <= 32)
+    return p.k == 4 || share > 0.8;
+  if (cached)
+    return share > 0.95 && (mib > 64 || (!f64 && p.k == 4));
+  return share > 0.8 || (!f64 && p.k >= 3);
 }
 
 template <typename T> void launch_diagonal(const GatePlan &p, hipStream_t s, void *sv, GateGeom g) {
@@ -1032,7 +1055,7 @@ void launch_by_k(const GatePlan &p, hipStream_t s, void *sv, const GateGeom &g) 
   // k = 1 in the caches: two rows a lane are no gather (f64 22 qubits 19 us
   // against 21, f32 24 qubits 36 against 38).
   if (mono && g.combos << g.k >= 64 && (p.k > 1 || !cached_state(g, sizeof(T))) &&
-      streamed_diagonal(p))
+      streamed_diagonal(p, g, sizeof(T)))
     return launch_diagonal<T>(p, s, sv, g);
   if (!mono) {
     const uint32_t n = p.k + uint32_t(63 - __builtin_clzll(g.combos));
@@ -1112,6 +1135,16 @@ void launch_mfma_batch(const BatchArgs &a, unsigned n, uint8_t precision, uint32
 }
 
 } // namespace
+
+double touched_lines(const GatePlan &p, uint32_t line_bits) {
+  uint32_t low = 0;
+  while (low < p.k && p.q[low] < line_bits)
+    ++low;
+  uint64_t rows = 0;
+  for (uint32_t x = 0; x < p.n_active; ++x)
+    rows |= uint64_t(1) << (p.act_row[x] >> low) | uint64_t(1) << (p.act_col[x] >> low);
+  return double(__builtin_popcountll(rows)) / double(1u << (p.k - low));
+}
 
 // f32 k = 4 stays with the direct kernel: its product form is the more exact
 // one, and it holds its 16 amplitudes in registers.  So do plans that ask for a

@@ -1039,22 +1039,6 @@ size_t tile_bytes(uint32_t m, uint8_t prec) { return size_t(prec == 0 ? 8 : 16) 
 
 } // namespace
 
-namespace {
-
-// Share of the statevector's lines of 2^line_bits amplitudes that a monomial
-// gate launched by itself reads or writes.
-double touched_lines(const GatePlan &p, uint32_t line_bits) {
-  uint32_t low = 0;
-  while (low < p.k && p.q[low] < line_bits)
-    ++low;
-  uint64_t rows = 0;
-  for (uint32_t x = 0; x < p.n_active; ++x)
-    rows |= uint64_t(1) << (p.act_row[x] >> low) | uint64_t(1) << (p.act_col[x] >> low);
-  return double(__builtin_popcountll(rows)) / double(1u << (p.k - low));
-}
-
-} // namespace
-
 // A pass reads and writes every amplitude, a monomial gate by itself only the
 // lines with rows other than the identity's.  On states that fill the chip a
 // few such gates (controlled phases, Toffolis) are therefore faster one by
