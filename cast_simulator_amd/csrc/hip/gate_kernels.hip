@@ -1148,10 +1148,20 @@ double touched_lines(const GatePlan &p, uint32_t line_bits) {
 
 // f32 k = 4 stays with the direct kernel: its product form is the more exact
 // one, and it holds its 16 amplitudes in registers.  So do plans that ask for a
-// variant or for f32 products: the batch has no other kernel for them.
+// variant or for f32 products: the batch has no other kernel for them.  f64 k =
+// 4, 5 go back to it above 18 qubits, where the launch no longer waits for a
+// chain of products, unless all but two targets are among the lowest three
+// (matrix cores /
+// direct, us: k = 5 on 18, 19, 22 qubits, 20 items 65 / 61, 125 / 89, 1008 / 577,
+// targets 0..4 78 / 103, 149 / 171, 1148 / 1528; k = 4 4 items of 21 qubits 56 /
+// 45, targets 0..3 75 / 162).  By the item alone, so that a result does not
+// depend on the batch.
 bool batch_on_matrix_cores(const GatePlan &p, uint32_t n) {
-  return p.d_mat3 && n >= p.k + 4 && (p.precision == 1 || p.k >= 5) && !p.forced &&
-         !(p.flags & CAST_HIP_FLAG_MFMA_F32);
+  if (!p.d_mat3 || n < p.k + 4 || p.forced || p.flags & CAST_HIP_FLAG_MFMA_F32)
+    return false;
+  if (p.precision == 0)
+    return p.k >= 5;
+  return p.k == 6 || n <= 18 || p.q[p.k - 3] < 3;
 }
 
 uint32_t plan_family(const GatePlan &plan, uint32_t n_qubits) {

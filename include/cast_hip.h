@@ -249,8 +249,9 @@ int cast_hip_gate_apply(const void *plan, void *stream, uint64_t sv_dptr, uint32
  * items per launch, more in several launches): item i applies plans[i] to
  * svs[i] (2^sv_n_qubits[i] amplitudes, sv_n_qubits[i] <= 40) with the direct
  * kernel or, for dense gates of k = 4 (f64), 5 and 6 on k + 4 qubits or more
- * whose plan asks for no variant and not for CAST_HIP_FLAG_MFMA_F32, on the
- * matrix cores (then at most two launches per 64 items).  All plans must share
+ * (f64 k = 4, 5 up to 18, or with all but two targets below 3) whose plan asks
+ * for no variant and not for CAST_HIP_FLAG_MFMA_F32, on the matrix cores (then
+ * at most two launches per 64 items).  All plans must share
  * precision and k.  For callers that hold many small statevectors (one launch
  * instead of one per statevector).  No reference counterpart (the reference
  * launches one kernel per apply). */
