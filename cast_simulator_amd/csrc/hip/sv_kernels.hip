@@ -296,9 +296,12 @@ __device__ __forceinline__ uint64_t deposit_rest(uint64_t r, uint64_t mask) {
   return r;
 }
 
-template <typename T> __device__ __forceinline__ double amp_prob(const T *sv, uint64_t j) {
+// NT: nontemporal, where a wave reads whole lines.
+template <bool NT, typename T>
+__device__ __forceinline__ double amp_prob(const T *sv, uint64_t j) {
   using VT = T __attribute__((ext_vector_type(2)));
-  const VT v = __builtin_nontemporal_load(reinterpret_cast<const VT *>(sv) + j);
+  const VT *p = reinterpret_cast<const VT *>(sv) + j;
+  const VT v = NT ? __builtin_nontemporal_load(p) : *p;
   const double re = double(v.x), im = double(v.y);
   return __builtin_fma(re, re, im * im);
 }
@@ -341,7 +344,7 @@ __global__ void __launch_bounds__(kRedBlock) k_marginal_rest(const T *__restrict
     double p[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      p[u] = amp_prob(sv, j);
+      p[u] = amp_prob<true>(sv, j);
       j = (((j | skip) + 1) & ~skip) | base | lane;
     }
 #pragma unroll
@@ -388,7 +391,7 @@ __global__ void __launch_bounds__(kRedBlock) k_marginal_bin(const T *__restrict_
     const uint64_t base = scatter_bin(b, a);
     double acc = 0.0;
     for (uint64_t r = 0; r < n_rest; ++r)
-      acc += amp_prob(sv, deposit_rest(r, a.mask) | base);
+      acc += amp_prob<false>(sv, deposit_rest(r, a.mask) | base);
     out[b] = acc;
   }
 }
