@@ -702,7 +702,10 @@ void launch_mfma_t(const GatePlan &p, hipStream_t s, void *sv, const GateGeom &g
   // +0.5-0.7 % on the 30-qubit headline circuit's k = 5 gates.
   const unsigned grid = mfma_order(p, unsigned(std::max<uint64_t>(1, std::min(need, cap))), tiles,
                                    g, sizeof(T) == 8);
-  if (sizeof(T) == 4 || cached_state(g, sizeof(T)))
+  // 19 to 21 qubits as the wave tiles of these sizes: plain stores leave lines in
+  // the L2 of an XCD that the next gate's tile is not on (automatic_cached).
+  const uint64_t mib = ((g.combos << g.k) * 2 * sizeof(T)) >> 20;
+  if (sizeof(T) == 4 || (cached_state(g, sizeof(T)) && (mib < 8 || mib > 32)))
     hipLaunchKernelGGL((k_mfma<T, KL, false>), dim3(grid), dim3(kBlock), 0, s,
                        static_cast<T *>(sv), static_cast<const T *>(p.d_mat3), g, tiles);
   else
@@ -862,11 +865,6 @@ void launch_tile_k(const GatePlan &p, hipStream_t s, void *sv, const TileGeom &t
 }
 
 // Wave-tile geometry for a gate on an n-qubit statevector (n >= k + 6).
-// Whether the statevector takes about half of the XCDs' L2 (16 MiB).
-bool xcd_resident(const GatePlan &p, uint32_t n) {
-  return (uint64_t(2 * scalar_bytes(p.precision)) << n) == uint64_t(16) << 20;
-}
-
 TileGeom tile_geom(const GatePlan &p, uint32_t n, uint32_t *n_low) {
   TileGeom tg{};
   tg.n_tiles = uint64_t(1) << (n - 6 - p.k);
@@ -892,7 +890,9 @@ TileGeom tile_geom(const GatePlan &p, uint32_t n, uint32_t *n_low) {
   // - 4, n - 3 at 25, 26 qubits 219 / 181, 439 / 360; n - 7 .. n - 4 at 26, 27
   // qubits 485 / 386, 1091 / 759, f32 at 28 qubits 930 / 758).
   const uint64_t mib = (uint64_t(2 * scalar_bytes(p.precision)) << n) >> 20;
-  bool order = mib >= 4096 || xcd_resident(p, n);
+  // So do states of 19 (f64) to 21 qubits, whose parts stay in the XCDs' L2
+  // (automatic_cached).
+  bool order = mib >= 4096 || (mib >= 8 && n <= 21);
   for (uint32_t b = 0; b + 1 < p.k && mib >= 512; ++b)
     order = order || (p.q[b] + 7 >= n && p.q[b + 1] == p.q[b] + 1 && p.q[b + 1] + 2 <= n);
   const bool xcd = (p.flags & CAST_HIP_FLAG_TILE_XCD) ||
@@ -940,7 +940,14 @@ uint32_t count_low(const GatePlan &p) {
 // Automatic choice for k <= 5 on a statevector of at most 256 MiB (f64 24
 // qubits, f32 25), where the gather kernels read from the caches.  us per
 // gate, averages over random targets, L = targets below bit 6:
-//   k <= 3       the direct kernel: f32 k = 3 at 22, 24, 25 qubits 9-12, 34-42,
+//   20, 21 qubits  k <= 4 with L <= 3 on wave tiles in XCD order, others on the
+//                matrix cores, and f64 k <= 3 at 19 on those tiles: each XCD then
+//                finds its tiles in its own L2 from gate to gate.  That shows in
+//                circuits, where direct kernels and plain matrix-core accesses
+//                between slow the tiles down too (f64 gates of k <= 4, 5 at 20 and
+//                21 qubits 591, 567, 673 and 890 us with them, 476, 476, 642, 678
+//                now; f32 at 21 qubits 622, now 482);
+//   k <= 3       else the direct kernel: f32 k = 3 at 22, 24, 25 qubits 9-12, 34-42,
 //                70-103 against 10-21, 42-68, 87-131 on wave tiles; f64 k = 3
 //                at 18, 22, 24 qubits 4, 19-26, 66-80 against 4-6.5, 22-25,
 //                88-93.  Except where targets crowd in the lowest bits, so that
@@ -948,14 +955,10 @@ uint32_t count_low(const GatePlan &p) {
 //                and 1 (k = 2 at 20, 22, 24 qubits 28, 23 and 89, 84 on tiles,
 //                k = 3 [0, 1, 2] 34, 30 and 115, 96), f32 two targets of k = 2
 //                or all of k = 3 below 3 (22, 25 qubits 15, 11 and 93, 82;
-//                [0, 1, 2] 25, 21 and 170, 142).  And except at 16 MiB, where in
-//                XCD order every XCD finds its tiles in its own L2 (f64 20
-//                qubits k = 1, 2 5.1-8.8 direct, 4.1-4.9 on tiles; k = 3 L = 0
-//                5.3, 4.2, L > 0 crowded 6.5-10.5, 5.1-8.4, else 5.2-5.4, 5.2-8.4);
-//   f64 k = 4    matrix cores up to 16 MiB (4-10 against 7-14 on tiles; at 16
-//                tiles for L = 0, 7.9-8.9 against 9.8-10.4) and from 128 MiB on
-//                (43, 82 against 45-59, 91-109); between, wave tiles for L <= 2
-//                (11.3-12.5, 23-27 against 17.6, 28);
+//                [0, 1, 2] 25, 21 and 170, 142);
+//   f64 k = 4    matrix cores up to 8 MiB (4-10 against 7-14 on tiles) and from
+//                128 MiB on (43, 82 against 45-59, 91-109); between, wave tiles for
+//                L <= 2 (11.3-12.5, 23-27 against 17.6, 28);
 //   f32 k = 4    matrix cores up to 4 MiB (4.7 against 5.6-11); above, tiles for
 //                L = 0 below 128 MiB (6.3-24 against 7.4-26 direct; at 24, 25
 //                qubits 48-53, 90-113 against 44-49, 85-92), matrix cores from
@@ -963,34 +966,32 @@ uint32_t count_low(const GatePlan &p) {
 //                60, 48) and from 128 MiB on for L >= 3 (53, 98 against 60, 115),
 //                else the direct kernel (22, 24 qubits 14.5-18, 45-60 against
 //                tiles 16-24, 51-75);
-//   f64 k = 5    wave tiles at 32 and 64 MiB for L <= 1 (26, 31 against 29, 54
-//                on the matrix cores) and at 128 MiB (63 against 66);
+//   f64 k = 5    wave tiles at 64 MiB for L <= 1 (50 against 60 on the matrix
+//                cores in a circuit; at 128 MiB 83 against 81);
 //   else         matrix cores.
 uint32_t automatic_cached(const GatePlan &p, uint32_t n, uint32_t n_low, bool tile_ok,
                           bool mfma_ok) {
   const uint64_t mib = (uint64_t(2 * scalar_bytes(p.precision)) << n) >> 20;
   const bool f64 = p.precision == 1;
   uint32_t v = 4;
-  if (p.k <= 3) {
+  if (n == 20 || n == 21)
+    v = p.k <= 4 && n_low <= 3 ? 3 : 4;
+  else if (p.k <= 3) {
     const uint32_t last = p.q[p.k - 1];
-    bool tile = false;
-    if (xcd_resident(p, n))
-      tile = p.k < 3 || n_low == 0 || p.q[n_low - 1] < (n_low == 1 ? 2u : 3u);
-    else if (p.k == 2)
-      tile = last < (f64 ? 2u : 3u);
-    else if (p.k == 3)
-      tile = mib > 8 && (f64 ? p.q[1] < 2 : last < 3);
-    v = tile ? 3 : 1;
+    const bool crowded = p.k == 2   ? last < (f64 ? 2u : 3u)
+                         : p.k == 3 ? mib > 16 && (f64 ? p.q[1] < 2 : last < 3)
+                                    : false;
+    v = (f64 && n == 19) || crowded ? 3 : 1;
   } else if (f64 && p.k == 4)
-    v = xcd_resident(p, n) ? (n_low == 0 ? 3 : 4) : mib > 16 && mib < 128 && n_low <= 2 ? 3 : 4;
+    v = mib > 16 && mib < 128 && n_low <= 2 ? 3 : 4;
   else if (p.k == 4)
-    v = mib <= 4                     ? 4
-        : n_low == 0 && mib < 128    ? 3
-        : mib >= 32 && p.q[2] < 3    ? 4
-        : mib >= 128 && n_low >= 3   ? 4
-                                     : 1;
+    v = mib <= 4                   ? 4
+        : n_low == 0 && mib < 128  ? 3
+        : mib >= 32 && p.q[2] < 3  ? 4
+        : mib >= 128 && n_low >= 3 ? 4
+                                   : 1;
   else if (f64)
-    v = mib > 16 && mib <= 128 && n_low <= 1 ? 3 : 4;
+    v = mib == 64 && n_low <= 1 ? 3 : 4;
   if (v == 4 && !mfma_ok)
     v = 3;
   return v == 3 && !tile_ok ? 1 : v;

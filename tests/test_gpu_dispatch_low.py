@@ -1,5 +1,5 @@
-"""Single gates where targets crowd in the lowest bits or the state takes half of
-the XCDs' L2, and diagonal gates on both sides of the share of lines at which
+"""Single gates where targets crowd in the lowest bits or the state fits the XCDs'
+L2, and diagonal gates on both sides of the share of lines at which
 they go as a stream: the kernel chosen, and the result against the oracle.
 
 Relative L2 <= 1e-13 at f64 (one gate of K <= 64 terms rounds below 1e-14) and
@@ -22,11 +22,13 @@ DIRECT, TILE, CORES = 1, 3, 4
 @pytest.mark.parametrize("precision,n,q,family", [
     (abi.F64, 22, [0, 1], TILE), (abi.F64, 22, [0, 2], DIRECT), (abi.F64, 22, [0, 1, 9], TILE),
     (abi.F64, 22, [1, 2, 9], DIRECT), (abi.F64, 20, [5], TILE), (abi.F64, 20, [18, 19], TILE),
-    (abi.F64, 20, [2, 3, 4], DIRECT), (abi.F64, 20, [0, 1, 2], TILE),
-    (abi.F64, 20, [6, 7, 8, 9], TILE), (abi.F64, 20, [0, 7, 8, 9], CORES),
+    (abi.F64, 20, [2, 3, 4], TILE), (abi.F64, 20, [0, 7, 8, 9], TILE),
+    (abi.F64, 20, [0, 1, 2, 3], CORES), (abi.F64, 19, [18], TILE), (abi.F64, 21, [9, 10], TILE),
     (abi.F64, 18, [0, 1], TILE), (abi.F64, 18, [0, 1, 2], DIRECT),
+    (abi.F64, 21, [7, 8, 9, 10, 11], CORES), (abi.F64, 22, [7, 8, 9, 10, 11], TILE),
     (abi.F32, 22, [0, 2], TILE), (abi.F32, 22, [0, 3], DIRECT), (abi.F32, 22, [0, 1, 2], TILE),
-    (abi.F32, 22, [0, 1, 3], DIRECT), (abi.F32, 21, [20], TILE), (abi.F32, 21, [0, 1, 9], TILE),
+    (abi.F32, 22, [0, 1, 3], DIRECT), (abi.F32, 21, [20], TILE), (abi.F32, 20, [4, 9, 11], TILE),
+    (abi.F32, 20, [4, 9, 11, 13], TILE), (abi.F32, 19, [4, 9, 11], DIRECT),
     (abi.F32, 23, [0, 1, 2, 9], CORES), (abi.F32, 23, [0, 1, 3, 9], DIRECT),
     (abi.F32, 24, [20, 21, 22, 23], DIRECT), (abi.F32, 23, [19, 20, 21, 22], TILE),
 ])
