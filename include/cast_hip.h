@@ -85,9 +85,10 @@ typedef struct cast_hip_kernel_gen_spec_t {
  * cover a contiguous eighth of every grid-stride step.  Faster for most
  * target sets and slower for some; the host autotuner tries it.  With
  * variant AUTO (no order flag) the library uses it for wave tiles of states
- * from 4 GiB on, for F64 matrix-core launches and for F32 split-product
- * launches from 32 qubits on; an explicitly requested variant without this
- * flag keeps launch order. */
+ * that fit the XCDs' L2 (19 to 21 qubits), of states from 4 GiB on and, from 512
+ * MiB on, of neighbouring high targets, for F64 matrix-core launches and for F32
+ * split-product launches from 32 qubits on; an explicitly requested variant
+ * without this flag keeps launch order. */
 #define CAST_HIP_FLAG_TILE_XCD 4u
 /* Dense k = 6 at F32 on the matrix cores: through bf16 split products
  * (every f32 operand split into three bf16 parts, six partial products per
