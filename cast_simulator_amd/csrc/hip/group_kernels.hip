@@ -522,8 +522,11 @@ __device__ __forceinline__ void wide_monomial_gate(unsigned char *lds, G &g,
   for (int c = 0; c < N; ++c) {
     // A row equal to the identity's leaves the amplitude as it is.  (With R >=
     // 4 only diagonal gates are this wide.)
-    const uint32_t r = hi << R | uint32_t(c);
-    const bool on_diagonal = R >= 4 || diagonal || (uint32_t(g.cols >> (4 * r)) & 15u) == r;
+    bool on_diagonal = diagonal;
+    if constexpr (R < 4) {
+      const uint32_t r = hi << R | uint32_t(c);
+      on_diagonal = diagonal || (uint32_t(g.cols >> (4 * r)) & 15u) == r;
+    }
     const bool keep = on_diagonal && e[c].x == T(1) && e[c].y == T(0);
     const V o = times<T>(x[c], e[c].x, e[c].y);
     lds_put<T>(lds, base ^ select_offsets<R>(g, 0, uint32_t(c)), keep ? x[c] : o);
