@@ -1,5 +1,5 @@
 """Single gates on both sides of the sizes from 128 MiB to 16 GiB where the
-automatic kernel, its accesses or its tile order change: up to 512 MiB against
+automatic kernel, its accesses or its tile order change: up to 256 MiB against
 the oracle, above against the direct kernel on the device.
 
 Relative L2 of a chain of at most 12 gates <= 1e-12 at f64 (a gate of K <= 64
@@ -27,8 +27,8 @@ def unitary(k, rng):
     return np.linalg.qr(z)[0]
 
 
-@pytest.mark.parametrize("precision,n", [(abi.F64, 23), (abi.F64, 24), (abi.F64, 25),
-                                         (abi.F32, 24), (abi.F32, 25), (abi.F32, 26)])
+@pytest.mark.parametrize("precision,n", [(abi.F64, 23), (abi.F64, 24), (abi.F32, 24),
+                                         (abi.F32, 25)])
 def test_gates_around_the_cache_size(precision, n):
     rng = np.random.default_rng(n + 40 * precision)
     gates = [(unitary(k, rng), low_and_high(k, low, n, rng))
@@ -54,8 +54,9 @@ def test_gates_around_the_cache_size(precision, n):
     assert rel_l2(x.astype(np.float64), got) <= TOL[precision]
 
 
-@pytest.mark.parametrize("precision,n", [(abi.F64, 27), (abi.F64, 28), (abi.F64, 30),
-                                         (abi.F32, 28), (abi.F32, 29)])
+@pytest.mark.parametrize("precision,n", [(abi.F64, 25), (abi.F64, 27), (abi.F64, 28),
+                                         (abi.F64, 30), (abi.F32, 26), (abi.F32, 28),
+                                         (abi.F32, 29)])
 def test_large_states_equal_the_direct_kernel(precision, n):
     rng = np.random.default_rng(n + 40 * precision)
     f32 = precision == abi.F32
@@ -64,6 +65,9 @@ def test_large_states_equal_the_direct_kernel(precision, n):
     gates = [(unitary(1, rng), [q], 0) for q in range(n)]  # a state without zeros, on both sides
     gates += [(unitary(k, rng), low_and_high(k, low, n, rng), 1)
               for k, low in ((2, 0), (3, 1), (3, 3), (4, 2), (4, 3), (5, 2))]
+    gates += [(unitary(4, rng), list(range(n - 7, n - 3)), 1)]  # neighbouring high targets
+    gates += [(np.diag(np.exp(2j * np.pi * rng.random(1 << k))), low_and_high(k, 1, n, rng), 1)
+              for k in (1, 3, 6)]
     one.zero()
     two.zero()
     for m, q, automatic in gates:
