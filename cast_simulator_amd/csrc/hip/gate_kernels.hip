@@ -944,9 +944,11 @@ uint32_t count_low(const GatePlan &p) {
 //                matrix cores, and f64 k <= 3 at 19 on those tiles: each XCD then
 //                finds its tiles in its own L2 from gate to gate.  That shows in
 //                circuits, where direct kernels and plain matrix-core accesses
-//                between slow the tiles down too (f64 gates of k <= 4, 5 at 20 and
-//                21 qubits 591, 567, 673 and 890 us with them, 476, 476, 642, 678
-//                now; f32 at 21 qubits 622, now 482);
+//                between slow the tiles down too (f64 gates of k <= 4, 5 at 20
+//                qubits 591, 567 us with them, 476 now; f32 at 21 qubits 622, now
+//                482).  At f64 21 qubits (32 MiB, as much as the L2s together) only
+//                k = 4: circuits of k <= 2, 3 direct 1230, 733 us, tiles 1383, 825;
+//                of k <= 4, 5 (gates of k <= 3 between) 674, 740 against 637, 665;
 //   k <= 3       else the direct kernel: f32 k = 3 at 22, 24, 25 qubits 9-12, 34-42,
 //                70-103 against 10-21, 42-68, 87-131 on wave tiles; f64 k = 3
 //                at 18, 22, 24 qubits 4, 19-26, 66-80 against 4-6.5, 22-25,
@@ -974,7 +976,7 @@ uint32_t automatic_cached(const GatePlan &p, uint32_t n, uint32_t n_low, bool ti
   const uint64_t mib = (uint64_t(2 * scalar_bytes(p.precision)) << n) >> 20;
   const bool f64 = p.precision == 1;
   uint32_t v = 4;
-  if (n == 20 || n == 21)
+  if (n == 20 || (n == 21 && !(f64 && p.k <= 3)))
     v = p.k <= 4 && n_low <= 3 ? 3 : 4;
   else if (p.k <= 3) {
     const uint32_t last = p.q[p.k - 1];

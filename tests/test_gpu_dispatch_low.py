@@ -23,7 +23,7 @@ DIRECT, TILE, CORES = 1, 3, 4
     (abi.F64, 22, [0, 1], TILE), (abi.F64, 22, [0, 2], DIRECT), (abi.F64, 22, [0, 1, 9], TILE),
     (abi.F64, 22, [1, 2, 9], DIRECT), (abi.F64, 20, [5], TILE), (abi.F64, 20, [18, 19], TILE),
     (abi.F64, 20, [2, 3, 4], TILE), (abi.F64, 20, [0, 7, 8, 9], TILE),
-    (abi.F64, 20, [0, 1, 2, 3], CORES), (abi.F64, 19, [18], TILE), (abi.F64, 21, [9, 10], TILE),
+    (abi.F64, 20, [0, 1, 2, 3], CORES), (abi.F64, 19, [18], TILE), (abi.F64, 21, [9, 10], DIRECT),
     (abi.F64, 18, [0, 1], TILE), (abi.F64, 18, [0, 1, 2], DIRECT),
     (abi.F64, 21, [7, 8, 9, 10, 11], CORES), (abi.F64, 22, [7, 8, 9, 10, 11], TILE),
     (abi.F32, 22, [0, 2], TILE), (abi.F32, 22, [0, 3], DIRECT), (abi.F32, 22, [0, 1, 2], TILE),
